@@ -212,9 +212,13 @@ double planner_coord_bound(const mptg_ctx* ctx);
 // kernels launched from other translation units
 // n_dev: tree size read on the device (tree_n then only plans the split);
 // skip: device flag that turns the launch into a no-op
-// Allocates the kNN partial-result buffers for nq queries over a tree of
-// tree_n nodes (what launch_knn would allocate).
-int knn_reserve(mptg_ctx* ctx, int64_t nq, int k, int64_t tree_n);
+// Allocates the kNN partial-result buffers for nq k = 1 queries over a tree
+// of tree_n nodes (what launch_knn would allocate).
+int knn_reserve(mptg_ctx* ctx, int64_t nq, int64_t tree_n);
+// k = 1..64 neighbours in L1/L2 spaces over nodes [0, n), every node visited:
+// wave lists (knn_wave.hip).
+int knn_wave_path(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radius, int32_t* d_idx, double* d_dist,
+                  int64_t n);
 // Grid kNN (knn_grid.hip): whether it serves a tree of n nodes in this
 // context, and the search itself; the m queries it leaves (*m, listed at
 // *over on the device) are the caller's to answer.

@@ -19,30 +19,19 @@
 //   * SE(3) queries reverse the roles: a query gets a workgroup, its lanes take
 //     consecutive nodes (knn_wave_se3).
 //
-// Prefilter soundness.  With u = 2^-24, S = max|q| + max|p| and
-// eps = 2.01 u S, each FP32 coordinate difference satisfies
-// |t_i - (q_i - p_i)| <= eps.  For L2 (squared distances d):
-//   |d32 - d| <= 2 eps sqrt(D d) + D eps^2 + g_D (d + 2 eps sqrt(D d) + D eps^2),
-//   g_D = D u / (1 - D u)
-// and for L1: |d32 - d| <= D eps + g_D (d + D eps).  A node can enter the
-// list only if d <= T (T = current k-th distance, squared for L2), hence only
-// if d32 <= T + eta(T).  The kernels use 2 * eta plus a relative 2^-40 for
-// the sqrt rounding of list entries.
 #include <algorithm>
 #include <cfloat>
 #include <climits>
 #include <cmath>
 #include <limits>
 
-#include "internal.hpp"
+#include "knn_bound.hpp"
 #include "wave_list.hpp"
 
 namespace mptg {
 namespace {
 
 constexpr int kBlock = 256;
-// Longest k-list of the SE(3) wave kernel (one entry per lane).
-constexpr int kWaveMaxK = 64;
 // Fewest tree nodes per split of the scan: small trees still spread over
 // many waves, while every split's partial list stays worth its merge.
 constexpr int64_t kMinSplitNodes = 64;
@@ -50,9 +39,6 @@ constexpr int64_t kMinSplitNodes = 64;
 // (n / kSeedNodes)-th node, spread over the tree rather than its first nodes
 // (a planner's first nodes crowd around its start).
 constexpr int64_t kSeedNodes = 256;
-
-// Register list length of a k-list scan: k rounded up to 1, 20, 32 or 64.
-inline int k_bucket(int k) { return k <= 1 ? 1 : (k <= 20 ? 20 : (k <= 32 ? 32 : 64)); }
 
 __device__ __forceinline__ bool better(double a, int ia, double b, int ib) {
     return a < b || (a == b && ia < ib);
@@ -89,70 +75,6 @@ struct TopK {
         }
     }
 };
-
-// FP64 metric value, left-to-right, no contraction (matches the oracle).
-template <int D, int METRIC>
-__device__ __forceinline__ double exact_dist(const double* __restrict__ a, const double* __restrict__ b) {
-    double s = 0.0;
-    if constexpr (METRIC == MPTG_METRIC_L1) {
-#pragma unroll
-        for (int i = 0; i < D; ++i) s = s + __builtin_fabs(a[i] - b[i]);
-        return s;
-    } else {
-#pragma unroll
-        for (int i = 0; i < D; ++i) {
-            double t = a[i] - b[i];
-            s = s + t * t;
-        }
-        return __builtin_sqrt(s);
-    }
-}
-
-// Prefilter threshold in the prefilter's units (squared distance for L2,
-// distance for L1) from the list's k-th distance `dk` (metric value).
-template <int D, int METRIC>
-__device__ __forceinline__ float prefilter_threshold(double dk, double S) {
-    if (!(dk < __builtin_inf())) return __builtin_inff();
-    const double u = 0x1.0p-24;
-    const double eps = 2.01 * u * S;
-    const double g = D * u / (1.0 - D * u);
-    double T, eta;
-    if constexpr (METRIC == MPTG_METRIC_L1) {
-        T = dk;
-        eta = D * eps + g * (T + D * eps);
-    } else {
-        T = dk * dk;
-        double r = 2.0 * eps * __builtin_sqrt(D * T) + D * eps * eps;
-        eta = r + g * (T + r);
-    }
-    double thr = T * (1.0 + 0x1.0p-40) + 2.0 * eta + 1e-300;
-    float f = (float)thr;
-    // round up (thr > 0) so that the FP32 comparison never undercuts the FP64 bound
-    return (double)f < thr ? float_of(bits_of(f) + 1u) : f;
-}
-
-// An upper bound, in metric units, on the exact distance of a node whose
-// prefilter value (FP32 sum, squared for L2) is `a`: the inverse of the
-// error bound behind prefilter_threshold.  L1: |a - d| <= D eps + g (d +
-// D eps) gives d <= (a + D eps (1 + g)) / (1 - g).  L2: |a - T| <= r + g (T +
-// r) with r = 2 eps sqrt(D T) + D eps^2 gives, for x = sqrt(T), (1 - g) x^2
-// - 2 (1 + g) eps sqrt(D) x - (a + (1 + g) D eps^2) <= 0, bounded by the
-// quadratic's larger root.  A relative 2^-40 covers the FP64 rounding.
-template <int D, int METRIC>
-__device__ __forceinline__ double prefilter_upper(float a, double S) {
-    const double u = 0x1.0p-24;
-    const double eps = 2.01 * u * S;
-    const double g = D * u / (1.0 - D * u);
-    double x;
-    if constexpr (METRIC == MPTG_METRIC_L1) {
-        x = ((double)a + D * eps * (1.0 + g)) / (1.0 - g);
-    } else {
-        const double bq = (1.0 + g) * eps * __builtin_sqrt((double)D);
-        const double c = (double)a + (1.0 + g) * D * eps * eps;
-        x = (bq + __builtin_sqrt(bq * bq + (1.0 - g) * c)) / (1.0 - g);
-    }
-    return x * (1.0 + 0x1.0p-40) + 1e-300;
-}
 
 // Splits actually used for a tree of n nodes when the launch was planned
 // for `planned` (a graph captured for a larger tree): at least kMinSplitNodes
@@ -231,7 +153,7 @@ __global__ __launch_bounds__(kBlock) void knn_seed(const double* __restrict__ x6
 // rest of its wave idles.
 constexpr int kScanTile = 64;
 
-template <int D, int METRIC, int K>
+template <int D, int METRIC>
 __global__ __launch_bounds__(kBlock) void knn_scan(const float* __restrict__ x32, const double* __restrict__ x64,
                                                    int64_t n, int64_t chunk, const double* __restrict__ q,
                                                    int64_t nq, double radius, double pbound,
@@ -240,7 +162,6 @@ __global__ __launch_bounds__(kBlock) void knn_scan(const float* __restrict__ x32
                                                    const double* __restrict__ seed, const uint32_t* nq_dev) {
     constexpr int DP = (D <= 2) ? 2 : (D <= 4 ? 4 : (D <= 8 ? 8 : ((D + 3) / 4) * 4));
     __shared__ __align__(16) float t32[kScanTile * DP];
-    __shared__ __align__(16) double t64[kScanTile * D];
     if (!knn_extent(n_dev, skip, &n, &chunk)) return;  // block-uniform
     // live queries: all nq, or the first *nq_dev (nq stays the output stride)
     const int64_t live = nq_dev ? (int64_t)*nq_dev : nq;
@@ -260,9 +181,9 @@ __global__ __launch_bounds__(kBlock) void knn_scan(const float* __restrict__ x32
         mq = __builtin_fmax(mq, __builtin_fabs(v));
     }
     const double S = mq + pbound;
-    TopK<K> top;
+    TopK<1> top;
     top.init();
-    // seed bound (k = 1): the nearest of a subset of the tree, measured by
+    // seed bound: the nearest of a subset of the tree, measured by
     // knn_seed.  The nearest node overall is no farther, so it still passes
     // the prefilter in its own chunk; other chunks skip the nodes beyond the
     // bound (their partial lists may then hold nothing) and the merge of the
@@ -271,7 +192,7 @@ __global__ __launch_bounds__(kBlock) void knn_scan(const float* __restrict__ x32
     float rthr = prefilter_threshold<D, METRIC>(radius, S);
     float thr = rthr;
     if (!active) thr = -1.0f;  // inactive lanes never take the slow path
-    // k = 1 candidates awaiting their exact distance.  A node whose prefilter
+    // candidates awaiting their exact distance.  A node whose prefilter
     // value exceeds a threshold derived from a listed candidate's upper bound
     // is farther than that candidate, so it cannot be the nearest; every
     // listed node gets its exact distance before the result is written.
@@ -292,9 +213,6 @@ __global__ __launch_bounds__(kBlock) void knn_scan(const float* __restrict__ x32
         const int cnt = (int)(p1 - t0 < kScanTile ? p1 - t0 : kScanTile);
         __syncthreads();  // every wave is done with the previous tile
         for (int i = threadIdx.x; i < cnt * DP; i += kBlock) t32[i] = x32[t0 * DP + i];
-        // k = 1 candidates read their FP64 rows at the flush, from global memory
-        if constexpr (K > 1)
-            for (int i = threadIdx.x; i < cnt * D; i += kBlock) t64[i] = x64[t0 * D + i];
         __syncthreads();
         // four tree nodes per step, one branch for all
         constexpr int U = 4;
@@ -316,32 +234,16 @@ __global__ __launch_bounds__(kBlock) void knn_scan(const float* __restrict__ x32
             uint32_t pass = 0;
 #pragma unroll
             for (int u = 0; u < U; ++u) pass |= (acc[u] <= thr ? 1u : 0u) << u;
-            if constexpr (K == 1) {
-                // k = 1: list the candidates and tighten the threshold from
-                // their prefilter values; their exact distances are taken
-                // together, when the list is full or at the chunk's end
-                while (pass) {
-                    const int u = __builtin_ctz(pass);
-                    pass &= pass - 1;
-                    if (ncand == kCand) flush();
-                    cand[ncand++] = (int32_t)(t0 + j + u);
-                    float t = prefilter_threshold<D, METRIC>(prefilter_upper<D, METRIC>(acc[u], S), S);
-                    thr = t < thr ? t : thr;
-                }
-            } else {
-                // candidates in node order; a candidate that a lower
-                // threshold would now reject is still safe to evaluate
-                // (insert keeps the exact order)
-                while (pass) {
-                    const int u = __builtin_ctz(pass);
-                    pass &= pass - 1;
-                    double dq = exact_dist<D, METRIC>(q + qc * D, t64 + (j + u) * D);
-                    if (dq <= radius) {
-                        top.insert(dq, (int32_t)(t0 + j + u));
-                        float t = prefilter_threshold<D, METRIC>(top.d[K - 1], S);
-                        thr = t < rthr ? t : rthr;
-                    }
-                }
+            // list the candidates and tighten the threshold from their
+            // prefilter values; their exact distances are taken together,
+            // when the list is full or at the chunk's end
+            while (pass) {
+                const int u = __builtin_ctz(pass);
+                pass &= pass - 1;
+                if (ncand == kCand) flush();
+                cand[ncand++] = (int32_t)(t0 + j + u);
+                float t = prefilter_threshold<D, METRIC>(prefilter_upper<D, METRIC>(acc[u], S), S);
+                thr = t < thr ? t : thr;
             }
         }
         for (; j < cnt; ++j) {
@@ -354,30 +256,18 @@ __global__ __launch_bounds__(kBlock) void knn_scan(const float* __restrict__ x32
                 else acc = __builtin_fmaf(t, t, acc);
             }
             if (acc <= thr) {
-                if constexpr (K == 1) {
-                    if (ncand == kCand) flush();
-                    cand[ncand++] = (int32_t)(t0 + j);
-                    float t = prefilter_threshold<D, METRIC>(prefilter_upper<D, METRIC>(acc, S), S);
-                    thr = t < thr ? t : thr;
-                } else {
-                    double dq = exact_dist<D, METRIC>(q + qc * D, t64 + j * D);
-                    if (dq <= radius) {
-                        top.insert(dq, (int32_t)(t0 + j));
-                        float t = prefilter_threshold<D, METRIC>(top.d[K - 1], S);
-                        thr = t < rthr ? t : rthr;
-                    }
-                }
+                if (ncand == kCand) flush();
+                cand[ncand++] = (int32_t)(t0 + j);
+                float t = prefilter_threshold<D, METRIC>(prefilter_upper<D, METRIC>(acc, S), S);
+                thr = t < thr ? t : thr;
             }
         }
     }
-    if constexpr (K == 1) flush();
+    flush();
     if (!active) return;
-    const int64_t base = ((int64_t)blockIdx.y * nq + qi) * K;
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        out_d[base + j] = top.d[j];
-        out_i[base + j] = top.i[j];
-    }
+    const int64_t base = (int64_t)blockIdx.y * nq + qi;
+    out_d[base] = top.d[0];
+    out_i[base] = top.i[0];
 }
 
 // ---- k = 1 under L1 with a byte prefilter ------------------------------------
@@ -658,68 +548,6 @@ __global__ __launch_bounds__(kBlock) void knn_scan_q8(const float* __restrict__ 
     out_i[base] = top.i[0];
 }
 
-// Merge of the chunks' partial k-lists: each lane keeps its query's k best
-// over the splits' lists.
-template <int K>
-__global__ __launch_bounds__(kBlock) void knn_merge(const double* __restrict__ pd, const int32_t* __restrict__ pi,
-                                                    int splits, int64_t nq, int k, double* __restrict__ out_d,
-                                                    int32_t* __restrict__ out_i, const int32_t* skip,
-                                                    const int64_t* n_dev) {
-    const int64_t qi = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (qi >= nq || (skip && *skip)) return;
-    if (n_dev) {
-        int64_t chunk;
-        splits = (int)knn_used_splits(*n_dev, splits, &chunk);
-    }
-    TopK<K> top;
-    top.init();
-    if constexpr (K == 1) {
-        // the minimum over the splits, eight loads in flight at a time
-        int s = 0;
-        for (; s + 8 <= splits; s += 8) {
-            double d[8];
-            int32_t id[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                d[u] = pd[(int64_t)(s + u) * nq + qi];
-                id[u] = pi[(int64_t)(s + u) * nq + qi];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (better(d[u], id[u], top.d[0], top.i[0])) {
-                    top.d[0] = d[u];
-                    top.i[0] = id[u];
-                }
-        }
-        for (; s < splits; ++s) {
-            const double d = pd[(int64_t)s * nq + qi];
-            const int32_t id = pi[(int64_t)s * nq + qi];
-            if (better(d, id, top.d[0], top.i[0])) {
-                top.d[0] = d;
-                top.i[0] = id;
-            }
-        }
-    } else {
-        for (int s = 0; s < splits; ++s) {
-            const int64_t base = ((int64_t)s * nq + qi) * K;
-            for (int j = 0; j < K; ++j) {
-                double d = pd[base + j];
-                int32_t id = pi[base + j];
-                if (id == INT_MAX) break;
-                top.insert(d, id);
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        if (j < k) {
-            bool have = top.i[j] != INT_MAX;
-            out_d[qi * k + j] = have ? top.d[j] : __builtin_inf();
-            out_i[qi * k + j] = have ? top.i[j] : -1;
-        }
-    }
-}
-
 // k = 1: the nearest over the splits.  kMergeLanes lanes share a query,
 // each reading every kMergeLanes-th split's partial result, then a shuffle
 // minimum by (distance, node id), which is exact in any order.
@@ -769,19 +597,16 @@ __global__ __launch_bounds__(kBlock) void knn_merge1(const double* __restrict__ 
     }
 }
 
-template <int K>
+// One split: its result is the answer.
 __global__ __launch_bounds__(kBlock) void knn_finish(const double* __restrict__ pd, const int32_t* __restrict__ pi,
-                                                     int64_t nq, int k, double* __restrict__ out_d,
+                                                     int64_t nq, double* __restrict__ out_d,
                                                      int32_t* __restrict__ out_i, const int32_t* skip,
                                                      const uint32_t* nq_dev) {
     const int64_t qi = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (qi >= nq || (skip && *skip) || (nq_dev && qi >= (int64_t)*nq_dev)) return;
-    for (int j = 0; j < k; ++j) {
-        int32_t id = pi[qi * K + j];
-        bool have = id != INT_MAX;
-        out_d[qi * k + j] = have ? pd[qi * K + j] : __builtin_inf();
-        out_i[qi * k + j] = have ? id : -1;
-    }
+    const bool have = pi[qi] != INT_MAX;
+    out_d[qi] = have ? pd[qi] : __builtin_inf();
+    out_i[qi] = have ? pi[qi] : -1;
 }
 
 // ---- k > 1 over large trees: bound, collect, select -------------------------
@@ -961,8 +786,8 @@ __global__ __launch_bounds__(64 * W) void knn_wave_se3(const double* __restrict_
                                                        double w_so3, double w_l2, double inf,
                                                        double* __restrict__ out_d, int32_t* __restrict__ out_i,
                                                        const int64_t* n_dev, const int32_t* skip) {
-    __shared__ double sd[W * kWaveMaxK];
-    __shared__ int32_t si[W * kWaveMaxK];
+    __shared__ double sd[W * kWaveListMax];
+    __shared__ int32_t si[W * kWaveListMax];
     __shared__ int real_s[W];
     if (skip && *skip) return;
     if (n_dev) n = *n_dev;
@@ -1026,10 +851,10 @@ struct ScanExtent {
     int64_t q8_target;       // byte prefilter: blocks its device-side split aims at
 };
 
-template <int D, int METRIC, int K>
+template <int D, int METRIC>
 void launch_scan(mptg_ctx* ctx, dim3 grid, const ScanExtent& x, const double* q, int64_t nq, double radius,
                  double* pd, int32_t* pi) {
-    if constexpr (K == 1 && METRIC == MPTG_METRIC_L1 && D >= 8) {
+    if constexpr (METRIC == MPTG_METRIC_L1 && D >= 8) {
         if (x.q8) {
             // the seed buffer (nq doubles) holds the queries' shared byte
             // bounds instead
@@ -1043,38 +868,37 @@ void launch_scan(mptg_ctx* ctx, dim3 grid, const ScanExtent& x, const double* q,
             return;
         }
     }
-    if (K == 1 && x.seed)
+    if (x.seed)
         hipLaunchKernelGGL((knn_seed<D, METRIC>), dim3((unsigned)((nq * kSeedLanes + kBlock - 1) / kBlock)),
                            dim3(kBlock), 0, ctx->stream, ctx->x64, x.n, q, nq, x.seed, x.n_dev, x.skip, x.nq_dev);
-    hipLaunchKernelGGL((knn_scan<D, METRIC, K>), grid, dim3(kBlock), 0, ctx->stream, ctx->x32, ctx->x64, x.n, x.chunk,
-                       q, nq, radius, ctx->coord_bound, pd, pi, x.n_dev, x.skip, (const double*)(K == 1 ? x.seed : nullptr),
+    hipLaunchKernelGGL((knn_scan<D, METRIC>), grid, dim3(kBlock), 0, ctx->stream, ctx->x32, ctx->x64, x.n, x.chunk,
+                       q, nq, radius, ctx->coord_bound, pd, pi, x.n_dev, x.skip, (const double*)x.seed,
                        x.nq_dev);
 }
 
-template <int D, int K>
+template <int D>
 bool dispatch_metric(mptg_ctx* ctx, dim3 grid, const ScanExtent& x, const double* q, int64_t nq, double radius,
                      double* pd, int32_t* pi) {
-    if (ctx->metric == MPTG_METRIC_L1) launch_scan<D, MPTG_METRIC_L1, K>(ctx, grid, x, q, nq, radius, pd, pi);
-    else launch_scan<D, MPTG_METRIC_L2, K>(ctx, grid, x, q, nq, radius, pd, pi);
+    if (ctx->metric == MPTG_METRIC_L1) launch_scan<D, MPTG_METRIC_L1>(ctx, grid, x, q, nq, radius, pd, pi);
+    else launch_scan<D, MPTG_METRIC_L2>(ctx, grid, x, q, nq, radius, pd, pi);
     return true;
 }
 
-template <int K>
 bool dispatch_dim(mptg_ctx* ctx, dim3 grid, const ScanExtent& x, const double* q, int64_t nq, double radius,
                   double* pd, int32_t* pi) {
     switch (ctx->dim) {
-        case 1: return dispatch_metric<1, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 2: return dispatch_metric<2, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 3: return dispatch_metric<3, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 4: return dispatch_metric<4, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 5: return dispatch_metric<5, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 6: return dispatch_metric<6, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 7: return dispatch_metric<7, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 8: return dispatch_metric<8, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 10: return dispatch_metric<10, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 12: return dispatch_metric<12, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 16: return dispatch_metric<16, K>(ctx, grid, x, q, nq, radius, pd, pi);
-        case 20: return dispatch_metric<20, K>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 1: return dispatch_metric<1>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 2: return dispatch_metric<2>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 3: return dispatch_metric<3>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 4: return dispatch_metric<4>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 5: return dispatch_metric<5>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 6: return dispatch_metric<6>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 7: return dispatch_metric<7>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 8: return dispatch_metric<8>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 10: return dispatch_metric<10>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 12: return dispatch_metric<12>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 16: return dispatch_metric<16>(ctx, grid, x, q, nq, radius, pd, pi);
+        case 20: return dispatch_metric<20>(ctx, grid, x, q, nq, radius, pd, pi);
         default: return false;
     }
 }
@@ -1083,59 +907,53 @@ bool dispatch_dim(mptg_ctx* ctx, dim3 grid, const ScanExtent& x, const double* q
 
 // Chooses the number of tree chunks so that a launch has ~8 waves per SIMD
 // worth of work, with at least kMinSplitNodes nodes per chunk.
-static int64_t choose_splits(mptg_ctx* ctx, int64_t nq, int64_t n, int K) {
+static int64_t choose_splits(mptg_ctx* ctx, int64_t nq, int64_t n) {
     int64_t qblocks = (nq + kBlock - 1) / kBlock;
     int64_t want_blocks = (int64_t)ctx->cus * ctx->tune.knn_blocks_per_cu;
     int64_t s = (want_blocks + qblocks - 1) / qblocks;
     int64_t max_s = (n + kMinSplitNodes - 1) / kMinSplitNodes;
     if (s > max_s) s = max_s;
     if (s < 1) s = 1;
-    // the merge reads splits * K candidates per query, one latency each
-    const int64_t cap = K == 1 ? 4096 : 64;
-    if (s > cap) s = cap;
-    return s;
+    return s > 4096 ? 4096 : s;
 }
 
-static int64_t plan_splits(mptg_ctx* ctx, int64_t nq, int64_t n, int64_t* chunk, int K = 1) {
-    int64_t splits = n > 0 ? choose_splits(ctx, nq, n, K) : 1;
+static int64_t plan_splits(mptg_ctx* ctx, int64_t nq, int64_t n, int64_t* chunk) {
+    int64_t splits = n > 0 ? choose_splits(ctx, nq, n) : 1;
     *chunk = n > 0 ? (n + splits - 1) / splits : 0;
     return n > 0 ? (n + *chunk - 1) / *chunk : 1;
 }
 
-int knn_reserve(mptg_ctx* ctx, int64_t nq, int k, int64_t tree_n) {
-    const int K = k_bucket(k);
+int knn_reserve(mptg_ctx* ctx, int64_t nq, int64_t tree_n) {
     int64_t chunk;
-    // k = 1 launches with a device query count plan for half the slots,
-    // which never takes fewer splits
-    const int64_t splits = plan_splits(ctx, K == 1 ? (nq + 1) / 2 : nq, tree_n, &chunk, K);
+    // launches with a device query count plan for half the slots, which
+    // never takes fewer splits
+    const int64_t splits = plan_splits(ctx, (nq + 1) / 2, tree_n, &chunk);
     int rc;
-    if ((rc = ensure(ctx, ctx->scratch[4], sizeof(double) * K * nq * splits))) return rc;
-    if (K == 1 && (rc = ensure(ctx, ctx->scratch[3], sizeof(double) * nq))) return rc;
-    return ensure(ctx, ctx->scratch[5], sizeof(int32_t) * K * nq * splits);
+    if ((rc = ensure(ctx, ctx->scratch[4], sizeof(double) * nq * splits))) return rc;
+    if ((rc = ensure(ctx, ctx->scratch[3], sizeof(double) * nq))) return rc;
+    return ensure(ctx, ctx->scratch[5], sizeof(int32_t) * nq * splits);
 }
 
-// The k-list scan: each lane keeps its query's k best in registers.
-static int knn_scan_path(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radius, int32_t* d_idx,
-                         double* d_dist, int64_t tree_n, const int64_t* n_dev, const int32_t* skip,
+// The k = 1 scan: one lane per query, the tree in chunks.
+static int knn_scan_path(mptg_ctx* ctx, const double* d_q, int64_t nq, double radius, int32_t* d_idx, double* d_dist,
+                         int64_t tree_n, const int64_t* n_dev, const int32_t* skip,
                          const uint32_t* nq_dev = nullptr) {
-    const int K = k_bucket(k);
     // with n_dev, tree_n is only the size the split count is planned for;
-    // with nq_dev (live queries on the device, k = 1) the split is planned
-    // for half of the nq slots
+    // with nq_dev (live queries on the device) the split is planned for half
+    // of the nq slots
     int64_t n = tree_n, chunk;
-    const int64_t splits = plan_splits(ctx, nq_dev ? (nq + 1) / 2 : nq, n, &chunk, K);
-    size_t pbytes_d = sizeof(double) * K * nq * splits, pbytes_i = sizeof(int32_t) * K * nq * splits;
+    const int64_t splits = plan_splits(ctx, nq_dev ? (nq + 1) / 2 : nq, n, &chunk);
     int rc;
-    if ((rc = ensure(ctx, ctx->scratch[4], pbytes_d))) return rc;
-    if ((rc = ensure(ctx, ctx->scratch[5], pbytes_i))) return rc;
+    if ((rc = ensure(ctx, ctx->scratch[4], sizeof(double) * nq * splits))) return rc;
+    if ((rc = ensure(ctx, ctx->scratch[5], sizeof(int32_t) * nq * splits))) return rc;
     // a seed bound pays off when the tree is split many ways: every chunk
     // starts from it
     double* seed = nullptr;
-    if (K == 1 && splits >= 8 && ctx->metric != MPTG_METRIC_SE3) {
+    if (splits >= 8 && ctx->metric != MPTG_METRIC_SE3) {
         if ((rc = ensure(ctx, ctx->scratch[3], sizeof(double) * nq))) return rc;
         seed = (double*)ctx->scratch[3].p;
     }
-    // k = 1 under L1 in 8 or more dimensions: the byte prefilter
+    // L1 in 8 or more dimensions: the byte prefilter
     const bool q8 = seed && ctx->metric == MPTG_METRIC_L1 && ctx->dim >= 8 && ctx->tune.knn_q8 &&
                     ctx->coord_bound > 0 && ctx->coord_bound < 1e300;
     // the byte prefilter's blocks (4 waves, 4 resident per CU) re-split on
@@ -1145,34 +963,33 @@ static int knn_scan_path(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, do
     double* pd = (double*)ctx->scratch[4].p;
     int32_t* pi = (int32_t*)ctx->scratch[5].p;
     dim3 grid((unsigned)((nq + kBlock - 1) / kBlock), (unsigned)splits);
-    bool ok;
-    if (K == 1) ok = dispatch_dim<1>(ctx, grid, ext, d_q, nq, radius, pd, pi);
-    else if (K == 20) ok = dispatch_dim<20>(ctx, grid, ext, d_q, nq, radius, pd, pi);
-    else if (K == 32) ok = dispatch_dim<32>(ctx, grid, ext, d_q, nq, radius, pd, pi);
-    else ok = dispatch_dim<64>(ctx, grid, ext, d_q, nq, radius, pd, pi);
-    if (!ok) return fail(ctx, MPTG_E_ARG, "unsupported dimension for the nearest-neighbour kernel");
+    if (!dispatch_dim(ctx, grid, ext, d_q, nq, radius, pd, pi))
+        return fail(ctx, MPTG_E_ARG, "unsupported dimension for the nearest-neighbour kernel");
     MPTG_HIP(ctx, hipGetLastError());
-    dim3 g1((unsigned)((nq + kBlock - 1) / kBlock));
-    if (splits > 1) {
-        if (K == 1) hipLaunchKernelGGL(knn_merge1, dim3((unsigned)((nq * kMergeLanes + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream, pd, pi, (int)splits, nq, d_dist, d_idx, skip, n_dev, std::numeric_limits<double>::infinity(), nq_dev, n, q8_target);
-        else if (K == 20) hipLaunchKernelGGL((knn_merge<20>), g1, dim3(kBlock), 0, ctx->stream, pd, pi, (int)splits, nq, k, d_dist, d_idx, skip, n_dev);
-        else if (K == 32) hipLaunchKernelGGL((knn_merge<32>), g1, dim3(kBlock), 0, ctx->stream, pd, pi, (int)splits, nq, k, d_dist, d_idx, skip, n_dev);
-        else hipLaunchKernelGGL((knn_merge<64>), g1, dim3(kBlock), 0, ctx->stream, pd, pi, (int)splits, nq, k, d_dist, d_idx, skip, n_dev);
-    } else {
-        if (K == 1) hipLaunchKernelGGL((knn_finish<1>), g1, dim3(kBlock), 0, ctx->stream, pd, pi, nq, k, d_dist, d_idx, skip, nq_dev);
-        else if (K == 20) hipLaunchKernelGGL((knn_finish<20>), g1, dim3(kBlock), 0, ctx->stream, pd, pi, nq, k, d_dist, d_idx, skip, nq_dev);
-        else if (K == 32) hipLaunchKernelGGL((knn_finish<32>), g1, dim3(kBlock), 0, ctx->stream, pd, pi, nq, k, d_dist, d_idx, skip, nq_dev);
-        else hipLaunchKernelGGL((knn_finish<64>), g1, dim3(kBlock), 0, ctx->stream, pd, pi, nq, k, d_dist, d_idx, skip, nq_dev);
-    }
+    if (splits > 1)
+        hipLaunchKernelGGL(knn_merge1, dim3((unsigned)((nq * kMergeLanes + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                           ctx->stream, pd, pi, (int)splits, nq, d_dist, d_idx, skip, n_dev,
+                           std::numeric_limits<double>::infinity(), nq_dev, n, q8_target);
+    else
+        hipLaunchKernelGGL(knn_finish, dim3((unsigned)((nq + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream, pd,
+                           pi, nq, d_dist, d_idx, skip, nq_dev);
     MPTG_HIP(ctx, hipGetLastError());
     return MPTG_OK;
+}
+
+// The scan for k neighbours: one lane per query at k = 1, one wave or more
+// per query beyond (knn_wave.hip).
+static int knn_brute(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radius, int32_t* d_idx,
+                     double* d_dist, int64_t n) {
+    return k == 1 ? knn_scan_path(ctx, d_q, nq, radius, d_idx, d_dist, n, nullptr, nullptr)
+                  : knn_wave_path(ctx, d_q, nq, k, radius, d_idx, d_dist, n);
 }
 
 // SE(3): one workgroup of W waves per query, W a power of two up to 16 for
 // about 4096 waves per launch, and no more waves than 64-node groups.
 static int knn_wave_se3_path(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radius, int32_t* d_idx,
                              double* d_dist, int64_t tree_n, const int64_t* n_dev, const int32_t* skip) {
-    if (k < 1 || k > kWaveMaxK) return fail(ctx, MPTG_E_RANGE, "SE(3) nearest neighbours: k must be 1..64");
+    if (k < 1 || k > kWaveListMax) return fail(ctx, MPTG_E_RANGE, "SE(3) nearest neighbours: k must be 1..64");
     if (nq >= ((int64_t)1 << 31)) return fail(ctx, MPTG_E_RANGE, "at most 2^31 - 1 queries");
     if (nq == 0) return MPTG_OK;
     const int64_t want = (4096 + nq - 1) / nq, groups = std::max<int64_t>(1, (tree_n + 63) / 64);
@@ -1279,7 +1096,7 @@ static int knn_refine(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, doubl
     int32_t* gi = (int32_t*)(gd + (size_t)m * k);
     hipLaunchKernelGGL(knn_gather, dim3((unsigned)(((int64_t)m * D + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                        ctx->stream, d_q, D, (const int64_t*)over, (int64_t)m, gq);
-    if ((rc = knn_scan_path(ctx, gq, m, k, radius, gi, gd, n, nullptr, nullptr))) return rc;
+    if ((rc = knn_brute(ctx, gq, m, k, radius, gi, gd, n))) return rc;
     hipLaunchKernelGGL(knn_scatter, dim3((unsigned)(((int64_t)m * k + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                        ctx->stream, (const double*)gd, (const int32_t*)gi, (const int64_t*)over, (int64_t)m, k, out_d,
                        out_i);
@@ -1304,7 +1121,7 @@ static int knn_select_path(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, 
     int32_t* sub_i = (int32_t*)(sub_d + (size_t)nq * k);
     double* tau = (double*)b[1].p;
     const unsigned g1 = (unsigned)((nq + kBlock - 1) / kBlock);
-    if ((rc = knn_scan_path(ctx, d_q, nq, k, radius, sub_i, sub_d, n / 256, nullptr, nullptr))) return rc;
+    if ((rc = knn_brute(ctx, d_q, nq, k, radius, sub_i, sub_d, n / 256))) return rc;
     hipLaunchKernelGGL(knn_bound, dim3(g1), dim3(kBlock), 0, ctx->stream, (const double*)sub_d, nq, k, radius, tau);
     if ((rc = knn_refine(ctx, d_q, nq, k, radius, tau, n / 16, sub_d, sub_i))) return rc;
     hipLaunchKernelGGL(knn_bound, dim3(g1), dim3(kBlock), 0, ctx->stream, (const double*)sub_d, nq, k, radius, tau);
@@ -1321,7 +1138,7 @@ int launch_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radiu
     if (nq_dev) {  // live queries known only on the device: the k = 1 scans
         if (k != 1 || ctx->metric == MPTG_METRIC_SE3)
             return fail(ctx, MPTG_E_STATE, "a device query count needs k = 1 and an L1/L2 space");
-        return knn_scan_path(ctx, d_q, nq, k, radius, d_idx, d_dist, tree_n, n_dev, skip, nq_dev);
+        return knn_scan_path(ctx, d_q, nq, radius, d_idx, d_dist, tree_n, n_dev, skip, nq_dev);
     }
     if (ctx->metric == MPTG_METRIC_SE3) return knn_wave_se3_path(ctx, d_q, nq, k, radius, d_idx, d_dist, tree_n, n_dev, skip);
     const bool sel_dim = ctx->dim <= 8 || ctx->dim == 10 || ctx->dim == 20;
@@ -1348,7 +1165,7 @@ int launch_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radiu
         // the select path streams the tree three times whatever the batch:
         // few queries take the k-list scan
         rc = select && m >= 2048 ? knn_select_path(ctx, gq, m, k, radius, gi, gd, tree_n)
-                                 : knn_scan_path(ctx, gq, m, k, radius, gi, gd, tree_n, nullptr, nullptr);
+                                 : knn_brute(ctx, gq, m, k, radius, gi, gd, tree_n);
         if (rc) return rc;
         hipLaunchKernelGGL(knn_scatter, dim3((unsigned)(((int64_t)m * k + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                            ctx->stream, (const double*)gd, (const int32_t*)gi, (const int64_t*)over, (int64_t)m, k,
@@ -1357,7 +1174,10 @@ int launch_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radiu
         return MPTG_OK;
     }
     if (select) return knn_select_path(ctx, d_q, nq, k, radius, d_idx, d_dist, tree_n);
-    return knn_scan_path(ctx, d_q, nq, k, radius, d_idx, d_dist, tree_n, n_dev, skip);
+    if (k == 1) return knn_scan_path(ctx, d_q, nq, radius, d_idx, d_dist, tree_n, n_dev, skip);
+    // (only k = 1 searches run inside captured iterations)
+    if (n_dev || skip) return fail(ctx, MPTG_E_STATE, "a device tree size needs k = 1");
+    return knn_wave_path(ctx, d_q, nq, k, radius, d_idx, d_dist, tree_n);
 }
 
 }  // namespace mptg

@@ -569,7 +569,7 @@ int mptg_prrt_run(mptg_ctx* ctx, int64_t target_size, int64_t max_iters, mptg_pr
                 ctx->size + span > s.g_plan) {
                 prrt_graph_drop(ctx);
                 const int64_t plan = std::min<int64_t>(ctx->cap, 2 * (ctx->size + span));
-                if ((rc = knn_reserve(ctx, B, 1, plan))) break;
+                if ((rc = knn_reserve(ctx, B, plan))) break;
                 if ((rc = capture_iterations(ctx, pd, G, plan, pre, &s.g_exec))) break;
                 s.g_epoch = ctx->epoch;
                 s.g_iters = G;

@@ -9,6 +9,8 @@
 
 namespace mptg {
 
+constexpr int kWaveListMax = 64;  // one entry per lane
+
 __device__ __forceinline__ bool wl_before(double a, int ia, double b, int ib) {
     return a < b || (a == b && ia < ib);
 }
@@ -17,6 +19,11 @@ __device__ __forceinline__ double wl_readlane(double v, int l) {
     const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
     const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
     return __hiloint2double(hi, lo);
+}
+
+// Lane l's value moved to lane l + 1 (lane 0 keeps its own): one DPP move.
+__device__ __forceinline__ int32_t wl_up(int32_t v) {
+    return __builtin_amdgcn_update_dpp(v, v, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
 }
 
 // (kd, ki) mirror lane k - 1's entry (the k-th best) as wave-uniform values.
@@ -37,26 +44,26 @@ struct WaveList {
         ki = INT_MAX;
         k = k_;
     }
-    // Inserts a wave-uniform candidate that beats (kd, ki): every entry
-    // after it moves one lane up.
+    // Inserts a wave-uniform candidate that beats (kd, ki): the first entry
+    // it beats and every one after it move one lane up (wl_up, a DPP move in
+    // the VALU; a shuffle is an LDS round trip).
     __device__ __forceinline__ void insert(double cd, int32_t ci, int lane) {
-        const double pd = __shfl_up(ld, 1);
-        const int32_t pi = __shfl_up(li, 1);
-        const bool shift = lane != 0 && wl_before(cd, ci, pd, pi);
-        const bool here = !shift && wl_before(cd, ci, ld, li);
-        ld = shift ? pd : (here ? cd : ld);
-        li = shift ? pi : (here ? ci : li);
+        const double pd = __hiloint2double(wl_up(__double2hiint(ld)), wl_up(__double2loint(ld)));
+        const int32_t pi = wl_up(li);
+        const int pos = __builtin_ctzll(__ballot(wl_before(cd, ci, ld, li)));  // never empty: lane k - 1 is beaten
+        ld = lane > pos ? pd : (lane == pos ? cd : ld);
+        li = lane > pos ? pi : (lane == pos ? ci : li);
         kd = wl_readlane(ld, k - 1);
         ki = __builtin_amdgcn_readlane(li, k - 1);
     }
-    // Offers every lane's (d, id) where `pass` holds, in lane order; only
-    // those that still beat the k-th best go in.
+    // Offers every lane's (d, id) where `pass` holds, in lane order; after
+    // each insert only those that still beat the k-th best stay.
     __device__ __forceinline__ void offer(bool pass, double d, int32_t id, int lane) {
-        for (unsigned long long m = __ballot(pass); m; m &= m - 1) {
+        unsigned long long m = __ballot(pass && wl_before(d, id, kd, ki));
+        while (m) {
             const int b = __builtin_ctzll(m);
-            const double cd = wl_readlane(d, b);
-            const int32_t ci = __builtin_amdgcn_readlane(id, b);
-            if (wl_before(cd, ci, kd, ki)) insert(cd, ci, lane);
+            insert(wl_readlane(d, b), __builtin_amdgcn_readlane(id, b), lane);
+            m = __ballot(pass && lane > b && wl_before(d, id, kd, ki));
         }
     }
 };

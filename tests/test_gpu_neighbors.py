@@ -166,3 +166,30 @@ def test_default_prrt_star_grows_1e5_nodes_in_se3(ctx_factory):
         anc = anc[anc]
     assert (anc == 0).all()
     assert st["rewires"] > 0
+
+
+# wave lists (knn_wave.hip): rows shorter than a wave, one row either side of
+# a wave's 64 nodes, the tree sizes where a query gets 4 and 16 waves, and
+# enough queries (an odd count) for four per wave
+@pytest.mark.parametrize("metric,dim,k,n,nq", [
+    (scenes.METRIC_L2, 2, 2, 1, 3), (scenes.METRIC_L2, 2, 20, 63, 100), (scenes.METRIC_L1, 3, 64, 64, 70),
+    (scenes.METRIC_L2, 7, 64, 65, 70), (scenes.METRIC_L1, 1, 5, 1023, 64), (scenes.METRIC_L2, 12, 33, 1024, 1),
+    (scenes.METRIC_L2, 2, 45, 4095, 1000), (scenes.METRIC_L1, 20, 20, 4097, 33), (scenes.METRIC_L2, 16, 7, 5000, 40),
+    (scenes.METRIC_L2, 2, 20, 900, 32769), (scenes.METRIC_L1, 8, 11, 700, 40001), (scenes.METRIC_L2, 10, 3, 300, 33001),
+])
+def test_knn_wave_lists_equal_oracle(ctx_factory, metric, dim, k, n, nq):
+    _say("knn wave lists", metric, dim, k, n, nq)
+    ctx = ctx_factory()
+    rng = np.random.default_rng(dim * 1000 + n)
+    pts = rng.uniform(-2, 2, (n, dim))
+    pts[n // 2:n // 2 + 3] = pts[0]  # equal distances: ascending ids
+    q = rng.uniform(-2.5, 2.5, (nq, dim))
+    q[0] = pts[0]
+    ctx.space(metric, dim)
+    ctx.tree_insert(pts)
+    o = oracle.Oracle(_plain(metric, dim))
+    some = np.unique(np.concatenate([[0, nq - 1], rng.integers(0, nq, 400)]))
+    for radius in (math.inf, 1.0):
+        gi, gd = ctx.knn(q, k, radius=radius)
+        oi, od = o.knn(pts, q[some], k, radius=radius, threads=8)
+        assert np.array_equal(gi[some], oi) and np.array_equal(gd[some], od), radius
