@@ -40,12 +40,13 @@ HBM_PEAK = 8.0e12        # B/s
 FP64_PEAK = 78.6e12      # FLOP/s (vector and matrix)
 FP32_PEAK = 157.3e12     # FLOP/s
 BF16_PEAK = 2.5e15       # FLOP/s, dense matrix
-# FP64 FLOP prices of the arm check's units of work
-FLOP_FK_LINK = 50        # angle add, pm::sincos (reduction + both kernels), 2 mul + 2 add
-FLOP_GROUP = 8           # group circle test: 2 sub, 3 mul, 2 add
-FLOP_LINK_FAR = 10       # link test settled by the far bound
-FLOP_LINK_EXACT = 24     # distPointSegmentSquared incl. the division
+# FLOP prices of the reference check's units of work (FP64)
+FLOP_FK_LINK = 50        # angle add, sine and cosine (reduction + both kernels), 2 mul + 2 add
 FLOP_REF_TEST = 20       # reference: one segment-disk test
+# and of the kernels' own (FP32, the angle in FP64)
+FLOP_NEAR_LINK = 10      # angle FMA and reduction, v_sin, v_cos, two joint FMAs
+FLOP_NEAR_CELL = 8       # midpoint and cell of a link
+FLOP_NEAR_TEST = 15      # one link-disk test
 
 
 def log(*a):
@@ -132,9 +133,9 @@ def arm_link_traffic():
     return None
 
 
-def fk_flops(wk):
-    return (FLOP_FK_LINK * wk["fk"] + FLOP_GROUP * wk["group"] + FLOP_LINK_FAR * wk["far"]
-            + FLOP_LINK_EXACT * wk["exact"])
+def executed_flops(wk):
+    return (FLOP_NEAR_LINK * wk["fk"] + FLOP_NEAR_CELL * wk["group"] + FLOP_NEAR_TEST * wk["far"]
+            + 20 * FLOP_FK_LINK * wk["exact"])
 
 
 def bench_arm(ctx, args, timer):
@@ -204,8 +205,8 @@ def bench_arm(ctx, args, timer):
     t_free = timer.time(lambda: ctx.link_dev(fa.ptr, fb.ptr, nf, mpt_amd.ORDER_REFERENCE, True, vf.ptr, cf.ptr), 5)
     for x in (fa, fb, vf, cf):
         x.free()
-    flops_p, flops_s = fk_flops(wk_p), fk_flops(wk_s)
-    # the dominant kernels: the packed head round + the continuation, surrogate order
+    flops_p, flops_s = executed_flops(wk_p), executed_flops(wk_s)
+    # the dominant kernels: the link kernel + the checks it leaves, surrogate order
     t_kernel = (phases["surrogate"]["head"] + phases["surrogate"]["tail"]) / 1e3
     t_kernel_p = (phases["plain"]["head"] + phases["plain"]["tail"]) / 1e3
     edge_batch = {
@@ -228,14 +229,14 @@ def bench_arm(ctx, args, timer):
         "reference_checks_on_collision_free_edges": int(out["plain"]["checks"][~coll].sum()),
         "gpu_waypoint_checks_plain": wk_p["calls"],
         "gpu_waypoint_checks_surrogate": wk_s["calls"],
-        "plain_kernel_fp64_tflops": flops_p / t_kernel_p / 1e12,
-        "surrogate_link_fp64_tflops": flops_s / t_kernel / 1e12,
+        "plain_kernel_tflops": flops_p / t_kernel_p / 1e12,
+        "surrogate_link_tflops": flops_s / t_kernel / 1e12,
         "score_rows": rows,
         "score_mfma_tflops": mlp_flops / t_score / 1e12,
         "score_frac_bf16": mlp_flops / t_score / BF16_PEAK,
     }
-    # roofline of the dominant kernels, the reference-order link (packed round
-    # + continuation + finish, one HIP-event span on the context stream).
+    # roofline of the dominant kernels, the reference-order link (one kernel and
+    # the checks it leaves, one HIP-event span on the context stream).
     # Algorithmic work: the reference loop's forward kinematics (every link of
     # every reference-order waypoint check up to the first hit) plus the
     # segment-disk tests whose disk lies within link length + r + R of the
@@ -250,15 +251,15 @@ def bench_arm(ctx, args, timer):
     roof = {"bound": "fp64-valu", "pipe": "FP64 vector ALU (the kernels issue no MFMA); peak = MI355X FP64 vector",
             "achieved": alg_flops / t_kernel_p / 1e12, "peak": FP64_PEAK / 1e12,
             "unit": "TFLOP/s", "frac": alg_flops / t_kernel_p / FP64_PEAK, "traffic": arm_link_traffic(),
-            "kernel": "arm_link_head + arm_link_tail <20, reference order>, 8192 planner edges (the 5 us "
-                      "arm_link_finish is outside launch_ms)",
+            "kernel": "arm_link + arm_link_rest <20, reference order>, 8192 planner edges",
             "launch_ms": t_kernel_p * 1e3, "flops_per_launch": alg_flops,
             "work_unit": "per reference-order waypoint check: 20 FK links x 50 flop, plus 20 flop per segment-disk "
                          "test whose disk lies within link length + r + R of the link's start joint",
             "effective_tflops": ref_flops / t_kernel_p / 1e12,
             "effective_unit": "reference brute force: 20 FK links x 50 flop + every disk tested until the first "
                               "hit x 20 flop",
-            "executed_tflops": flops_p / t_kernel_p / 1e12, "executed_frac": flops_p / t_kernel_p / FP64_PEAK,
+            "executed_tflops": flops_p / t_kernel_p / 1e12, "executed_frac": flops_p / t_kernel_p / FP32_PEAK,
+            "executed_unit": "the kernels' own FP32 bounds (angles in FP64) on the FP32 peak",
             "work": wk_p}
     res = {"plain": plain, "surrogate": sur, "tail_autotune": tune_link,
            "launch_shapes": ctx.tune_get(),

@@ -346,9 +346,9 @@ typedef struct mptg_tune_params {
     int32_t knn_blocks_per_cu;      /* kNN scan blocks per CU the tree split aims at (1..256) */
     int32_t dmv_long_waves_per_cu;  /* grid of the persistent DMV long-edge kernel (1..256) */
     int32_t mesh_waves_per_cu;      /* grid of the persistent mesh kernels (1..256) */
-    int32_t arm_tail_waves;         /* waves sharing one arm edge's continuation rounds (1..8) */
-    int32_t arm_cull;               /* arm link disk culling: 0 one walk per wave over the wave's
-                                       box, 1 each lane over its own grid cells */
+    int32_t arm_tail_waves;         /* kept for callers that set it (1..8); the arm link kernels
+                                       choose their waves from the batch size */
+    int32_t arm_cull;               /* likewise (0 or 1) */
     int32_t mesh_edge_waves;        /* waves sharing one mesh edge's waypoints (1..32) */
     int32_t knn_select;             /* k > 1 on trees of 2^16 nodes or more: 1 bound, collect and
                                        select (registers of k = 1 in the scan), 0 the k-list scan */
@@ -392,9 +392,8 @@ int mptg_tune_set(mptg_ctx* ctx, const mptg_tune_params* p);
 int mptg_autotune_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, mptg_tune_report* rep);
 /* Times link() of n device edges (reference order) for each candidate of the
    scene's link launch shape -- for DMV scenes the lanes per edge and then
-   the grid of the persistent long-edge kernel, for meshes the grid and then the waves per edge, for the arm the
-   disk culling and then the waves per continued edge (rep: the last knob
-   swept) -- and keeps the fastest;
+   the grid of the persistent long-edge kernel, for meshes the grid and then the waves per edge, for the arm
+   arm_tail_waves (rep: the last knob swept) -- and keeps the fastest;
    the per-edge bisection kernels have none (MPTG_E_STATE). */
 int mptg_autotune_link(mptg_ctx* ctx, const double* d_from, const double* d_to, int64_t n,
                        mptg_tune_report* rep);
@@ -407,8 +406,8 @@ int mptg_autotune_prrt(mptg_ctx* ctx, int64_t target_size, mptg_tune_report* rep
 
 /* one arm-scene link() call (as mptg_link_dev) timed phase by phase with HIP
  * events on the context stream: h_ms[0] surrogate scoring of every edge's
- * picks (surrogate order; one kernel), [1] packed head round, [2] the gap
- * before the continuation, [3] continuation, [4] irregular-edge walk (ms) */
+ * picks (surrogate order; one kernel), [1] the link kernel, [2] the gap
+ * before the next, [3] the checks and edges it left, [4] nothing (ms) */
 int mptg_link_phases(mptg_ctx* ctx, const double* d_from, const double* d_to, int64_t n, int order,
                      int endpoints_known_valid, uint8_t* d_verdict, uint32_t* d_checks, float* h_ms);
 /* plain device-to-device copy kernel of `bytes` (multiple of 16, 16-byte
@@ -416,10 +415,10 @@ int mptg_link_phases(mptg_ctx* ctx, const double* d_from, const double* d_to, in
 int mptg_diag_copy(mptg_ctx* ctx, void* d_dst, const void* d_src, uint64_t bytes);
 /* Work of a link() batch on the arm scene in the given order, from untimed
  * instrumented copies of the kernels (used to price a launch in FLOPs):
- *   h_work[0..4] = the GPU kernel's executed work: valid() calls, forward-
- *                  kinematics links, group broad-phase tests, link tests
- *                  resolved by the far-disk bound, link tests that ran the
- *                  exact expression;
+ *   h_work[0..4] = the GPU kernels' executed work: waypoint checks, forward-
+ *                  kinematics links, cell lookups (one per link), FP32
+ *                  link-disk tests, checks repeated exactly by arm_link_rest's
+ *                  edge walks;
  *   h_work[5..8] = the reference algorithm's work on the same edges: valid()
  *                  calls, FK links, segment-disk tests (every disk until the
  *                  first hit), and those of the tests whose disk centre lies

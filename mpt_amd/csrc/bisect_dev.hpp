@@ -91,16 +91,10 @@ __host__ __device__ __forceinline__ double coord_mid(double lo, double hi, uint3
 }
 
 
-// Height h and perfect-tree test of link(a, b) (see arm.hip for the bound).
-// Returns false when the edge needs more than kMaxArmDepth levels.
-template <int D>
-__device__ __forceinline__ bool bisect_shape(const double* a, const double* b, double tol, int* h_out, bool* regular) {
-    double wmax = 0.0, M = 0.0;
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-        wmax = __builtin_fmax(wmax, __builtin_fabs(a[j] - b[j]));
-        M = __builtin_fmax(M, __builtin_fmax(__builtin_fabs(a[j]), __builtin_fabs(b[j])));
-    }
+// Height h and perfect-tree test of link(a, b) from its widest coordinate
+// difference and largest |coordinate| (see arm.hip for the bound).  Returns
+// false when the edge needs more than kMaxArmDepth levels.
+__device__ __forceinline__ bool bisect_height(double wmax, double M, double tol, int* h_out, bool* regular) {
     int h = 0;
     double wd = wmax;  // w_max / 2^h, exact scaling
     while (!(wd < tol) && h <= kMaxArmDepth) {
@@ -113,6 +107,17 @@ __device__ __forceinline__ bool bisect_shape(const double* a, const double* b, d
     *regular = (h == 0) || ((2.0 * wd - err >= tol) && (wd + err < tol));
     *h_out = h;
     return true;
+}
+
+template <int D>
+__device__ __forceinline__ bool bisect_shape(const double* a, const double* b, double tol, int* h_out, bool* regular) {
+    double wmax = 0.0, M = 0.0;
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+        wmax = __builtin_fmax(wmax, __builtin_fabs(a[j] - b[j]));
+        M = __builtin_fmax(M, __builtin_fmax(__builtin_fabs(a[j]), __builtin_fabs(b[j])));
+    }
+    return bisect_height(wmax, M, tol, h_out, regular);
 }
 
 // Sort key of a waypoint in surrogate order: ascending key = descending

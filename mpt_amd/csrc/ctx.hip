@@ -150,6 +150,76 @@ int tree_reserve(mptg_ctx* ctx, int64_t cap) {
     return grow_tree(ctx, c);
 }
 
+// Disk lists of the arm's FP32 clearance bounds (arm_near.hpp): per cell of an
+// n x n grid over the square the joints can reach, every disk a link whose
+// midpoint lies in the cell may touch, with the squared distances below and
+// above which the FP32 test is certain.  disks: [cx, cy, (r+R)^2, r+R].
+// near_n = 0 (no lists) for arms and disks outside the bounds' assumptions.
+static void near_lists(const double* len, int nlinks, const std::vector<double>& disks, int ndisks, SceneDev* sd,
+                       std::vector<uint2>* cells, std::vector<float4>* out, std::vector<int32_t>* ids) {
+    sd->near_n = 0;
+    double T = 0.0, longest = 0.0, rmax = 0.0;
+    for (int i = 0; i < nlinks; ++i) {
+        if (!(len[i] >= 0.0) || !std::isfinite(len[i])) return;
+        T += len[i];
+        longest = std::max(longest, len[i]);
+    }
+    for (int i = 0; i < ndisks; ++i) {
+        const double* d = &disks[4 * (size_t)i];
+        if (!std::isfinite(d[0]) || !std::isfinite(d[1]) || !(d[3] >= 0.0) || !std::isfinite(d[3])) return;
+        rmax = std::max(rmax, d[3]);
+    }
+    // the FP32 squares stay clear of overflow and of denormals
+    if (!(T > 1e-6) || !(T + rmax < 1e6)) return;
+    const double margin = kNearMargin * (T + longest + 2.0 * rmax);
+    // cells half a link wide: the lists are then within a third of the
+    // shortest possible, and 64 x 64 cells of the 20-link arm stay in L2
+    const int n = std::max(1, std::min(kNearCells, (int)std::ceil(4.0 * T / longest)));
+    const double size = 2.0 * T / n;
+    // the midpoint's error is a joint's; its cell coordinate's FP32 rounding
+    // is within 1e-6 T
+    const double slack = 2.0 * margin + 8e-6 * T;
+    cells->assign((size_t)n * n, make_uint2(0, 0));
+    auto visit = [&](auto&& take) {
+        for (int i = 0; i < ndisks; ++i) {
+            const double* d = &disks[4 * (size_t)i];
+            const double reach = longest / 2 + d[3] + slack;
+            if (std::fabs(d[0]) > T + reach || std::fabs(d[1]) > T + reach) continue;
+            auto cell = [&](double v) { return std::max(0, std::min(n - 1, (int)std::floor((v + T) / size))); };
+            const int x0 = cell(d[0] - reach) - 1, x1 = cell(d[0] + reach) + 1;
+            const int y0 = cell(d[1] - reach) - 1, y1 = cell(d[1] + reach) + 1;
+            for (int y = std::max(0, y0); y <= std::min(n - 1, y1); ++y)
+                for (int x = std::max(0, x0); x <= std::min(n - 1, x1); ++x) {
+                    const double lx = -T + x * size, ly = -T + y * size;
+                    const double gx = std::max({lx - d[0], d[0] - (lx + size), 0.0});
+                    const double gy = std::max({ly - d[1], d[1] - (ly + size), 0.0});
+                    if (gx * gx + gy * gy <= reach * reach) take((size_t)y * n + x, i);
+                }
+        }
+    };
+    visit([&](size_t c, int) { (*cells)[c].y++; });
+    uint64_t total = 0;
+    for (uint2& c : *cells) {
+        c.x = (uint32_t)total;
+        total += c.y;
+        c.y = 0;
+    }
+    if (total > (uint64_t)kNearMaxEntries) return;
+    out->assign((size_t)std::max<uint64_t>(total, 1), make_float4(0, 0, 0, 0));
+    ids->assign(out->size(), 0);
+    visit([&](size_t c, int i) {
+        const double* d = &disks[4 * (size_t)i];
+        const double lo = std::max(d[3] - margin, 0.0), hi = d[3] + margin;
+        const size_t at = (*cells)[c].x + (*cells)[c].y++;
+        (*ids)[at] = i;
+        (*out)[at] = make_float4((float)d[0], (float)d[1], std::nextafterf((float)(lo * lo), 0.0f),
+                                 std::nextafterf((float)(hi * hi), INFINITY));
+    });
+    sd->near_n = n;
+    sd->near_extent = (float)T;
+    sd->near_inv = (float)(n / (2.0 * T));
+}
+
 }  // namespace mptg
 
 using namespace mptg;
@@ -195,6 +265,9 @@ void mptg_destroy(mptg_ctx* ctx) {
     (void)hipFree(ctx->scene.arm_disks.p);
     (void)hipFree(ctx->scene.arm_lim.p);
     (void)hipFree(ctx->scene.arm_index.p);
+    (void)hipFree(ctx->scene.near_cells.p);
+    (void)hipFree(ctx->scene.near_disks.p);
+    (void)hipFree(ctx->scene.near_ids.p);
     (void)hipFree(ctx->scene.mesh_nodes.p);
     (void)hipFree(ctx->scene.mesh_tris.p);
     (void)hipFree(ctx->scene.mesh_robot.p);
@@ -576,6 +649,21 @@ int mptg_scene_arm(mptg_ctx* ctx, const double* h_lengths, int nlinks, double ro
                                  hipMemcpyHostToDevice, ctx->stream));
     MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.arm_lim.p, lim.data(), sizeof(double) * lim.size(),
                                  hipMemcpyHostToDevice, ctx->stream));
+    std::vector<uint2> cells;
+    std::vector<float4> near;
+    std::vector<int32_t> near_ids;
+    near_lists(h_lengths, nlinks, ad, ndisks, &ctx->scene, &cells, &near, &near_ids);
+    if (ctx->scene.near_n > 0) {
+        if ((rc = ensure(ctx, ctx->scene.near_cells, sizeof(uint2) * cells.size()))) return rc;
+        if ((rc = ensure(ctx, ctx->scene.near_disks, sizeof(float4) * near.size()))) return rc;
+        if ((rc = ensure(ctx, ctx->scene.near_ids, sizeof(int32_t) * near_ids.size()))) return rc;
+        MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.near_ids.p, near_ids.data(), sizeof(int32_t) * near_ids.size(),
+                                     hipMemcpyHostToDevice, ctx->stream));
+        MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.near_cells.p, cells.data(), sizeof(uint2) * cells.size(),
+                                     hipMemcpyHostToDevice, ctx->stream));
+        MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.near_disks.p, near.data(), sizeof(float4) * near.size(),
+                                     hipMemcpyHostToDevice, ctx->stream));
+    }
     MPTG_HIP(ctx, hipStreamSynchronize(ctx->stream));
     ctx->scene.kind = MPTG_SCENE_ARM;
     ctx->valid_upto = 0;  // valid() changed: every node is checked again

@@ -41,6 +41,11 @@ struct SceneDev {
     DevBuf arm_disks, arm_lim;  // kernel layout of the disks (ascending cx), per-link bounds
     DevBuf arm_index;           // [xmin, 1/bucket width, max (r+R), 0] + int32 bucket starts
     double total_length = 0;    // sum of link lengths (feature scale)
+    // FP32 clearance bounds: cells and disk lists (arm_near.hpp); near_n = 0:
+    // the scene has none (every check is exact)
+    DevBuf near_cells, near_disks, near_ids;
+    float near_extent = 0, near_inv = 0;
+    int near_n = 0;
     // mesh (SE(3) rigid body): env BVH nodes, env triangles, robot triangles
     DevBuf mesh_nodes, mesh_tris, mesh_robot;
     int mesh_nnodes = 0, mesh_nrobot = 0;
@@ -145,7 +150,10 @@ struct mptg_ctx {
     // unsorted pairs and sort scratch; staged host queries; sorted results
     mptg::DevBuf rnn_buf, rnn_pairs, rnn_q, rnn_out;
     mptg::DevBuf scratch[12];  // 0-2 host staging, 3 kNN seed bounds, 4-5 kNN partials, 6 DMV table, 7 edge lists, 8 scores,
-                               // 9 surrogate picks, 10 continuation list
+                               // 9 surrogate picks, 10 arm link counters and lists
+    // the arm link's list counters are zero (its second kernel clears them);
+    // false after an allocation or a failed launch
+    bool arm_lists_clean = false;
     // pinned host staging
     void* pinned = nullptr;
     size_t pinned_bytes = 0;
@@ -163,9 +171,8 @@ struct mptg_ctx {
     // graph is replayed only while the epoch it was captured at holds
     uint64_t epoch = 0;
     // launch shapes (mptg_autotune_*): kNN blocks per CU, waves per CU of the
-    // persistent DMV long-edge kernel and of the mesh kernels, waves per edge
-    // of the arm continuation, arm link disk culling (0 wave box, 1 per lane),
-    // waves per mesh edge, kNN select and grid paths, lanes per DMV edge, the
+    // persistent DMV long-edge kernel and of the mesh kernels, two that the
+    // arm link no longer reads, waves per mesh edge, kNN select and grid paths, lanes per DMV edge, the
     // byte prefilter of the k = 1 L1 scan
     mptg_tune_params tune{8, 16, 32, 2, 0, 2, 1, 1, 8, 1};
     hipEvent_t phase_ev[6] = {};
@@ -272,10 +279,9 @@ int launch_mesh_link(mptg_ctx* ctx, const uint8_t* d_table, const double* d_from
 int launch_mesh_filter(mptg_ctx* ctx, const double* d_states, int64_t n, uint8_t* d_mask, uint8_t* d_status,
                        int invalid_code);
 // Arm link kernels in `order`; with the surrogate order every edge's picks
-// are scored first, and the packed round checks them.
+// are scored first and checked first.  MPTG_E_STATE: no kernel for this arm.
 int launch_arm_link(mptg_ctx* ctx, const double* from, const double* to, int64_t n, int known_valid,
-                    const uint8_t* mask, uint8_t* verdict, uint32_t* checks, int64_t* irr, uint32_t* nirr,
-                    unsigned long long* work, int order);
+                    const uint8_t* mask, uint8_t* verdict, uint32_t* checks, unsigned long long* work, int order);
 // surrogate scores of every waypoint of every (masked) arm edge:
 // scores[e * 512 + reference ordinal]
 int surrogate_score_edges(mptg_ctx* ctx, const double* from, const double* to, int64_t n, const uint8_t* mask,

@@ -331,19 +331,19 @@ int enqueue_iteration(mptg_ctx* ctx, const PrrtDev& pd, int64_t it, int64_t plan
     uint8_t* skip = nullptr;  // custom sampler: slots without a sample (eager iterations only)
     if (s.sampler && (rc = take_host_samples(ctx, it, (double*)pb.q.p, dcnt, &skip))) return rc;
     if (pre) {
-        const bool arm8 = ctx->scene.kind == MPTG_SCENE_ARM && ctx->scene.nlinks == D && (D == 5 || D == 10 || D == 20);
+        const bool arm = ctx->scene.kind == MPTG_SCENE_ARM && ctx->scene.nlinks == D && (D == 5 || D == 10 || D == 20);
         dispatch_dim(D, [&]<int DD>() {
             if constexpr (DD == 5 || DD == 10 || DD == 20) {
-                if (arm8) {
-                    hipLaunchKernelGGL((prrt_prevalid<DD, kPrevalidLanes>),
-                                       dim3((unsigned)(((int64_t)B * kPrevalidLanes + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                if (arm) {
+                    hipLaunchKernelGGL((prrt_prevalid<DD, true>),
+                                       dim3((unsigned)(((int64_t)B * near_lanes<DD>() + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                                        ctx->stream, scene_args(ctx), D, B, (const double*)pb.q.p,
                                        (uint8_t*)pb.status.p, (uint8_t*)pb.mask.p, (double*)pb.qv.p,
                                        (int32_t*)pb.vidx.p, vcnt, (const Counters*)dcnt);
                     return;
                 }
             }
-            hipLaunchKernelGGL((prrt_prevalid<DD, 1>), dim3((unsigned)((B + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+            hipLaunchKernelGGL((prrt_prevalid<DD, false>), dim3((unsigned)((B + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                                ctx->stream, scene_args(ctx), D, B, (const double*)pb.q.p, (uint8_t*)pb.status.p,
                                (uint8_t*)pb.mask.p, (double*)pb.qv.p, (int32_t*)pb.vidx.p, vcnt,
                                (const Counters*)dcnt);

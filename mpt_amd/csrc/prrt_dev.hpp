@@ -3,7 +3,7 @@
 // src/mpt/impl/prrt_star/prrt_star.hpp:470-540).
 #pragma once
 #include "sample_hd.hpp"
-#include "space_dev.hpp"
+#include "arm_near.hpp"
 
 namespace mptg {
 namespace {
@@ -175,12 +175,8 @@ __global__ __launch_bounds__(kBlock) void prrt_steer(SpaceArgs sp, SceneArgs sc,
     linkmask[b] = 1;
 }
 
-// prrt_steer for arm scenes with D = nlinks: kArmLanes lanes per sample
-// share its disk tests (arm_ok_split); lane 0 of each group writes.  Same
-// outputs as prrt_steer.
-constexpr int kArmLanes = 8;
-constexpr int kPrevalidLanes = 4;  // lanes per sample in prrt_prevalid on arm scenes
-
+// prrt_steer for arm scenes with D = nlinks: five links of a sample per lane
+// (arm_ok_near).  Same outputs as prrt_steer.
 template <int D>
 __global__ __launch_bounds__(kBlock) void prrt_steer_arm(SpaceArgs sp, SceneArgs sc, double range, int B,
                                                          const double* __restrict__ x64, const double* __restrict__ q,
@@ -189,22 +185,22 @@ __global__ __launch_bounds__(kBlock) void prrt_steer_arm(SpaceArgs sp, SceneArgs
                                                          double* __restrict__ to, uint8_t* __restrict__ status,
                                                          uint8_t* __restrict__ linkmask, double* dnear,
                                                          const Counters* __restrict__ cnt) {
+    constexpr int L = near_lanes<D>(), N = kNearLinks;
     const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int b = (int)(t / kArmLanes);
-    const bool lead = (t % kArmLanes) == 0;
+    const int b = (int)(t / L), u = (int)(t % L);
+    const bool lead = u == 0;
     const bool inb = b < B;
-    bool need = false;
-    double s[D];
-#pragma unroll
-    for (int i = 0; i < D; ++i) s[i] = 0.0;
+    bool need = false, cut = false;
+    double d = 0.0;
+    int32_t nn = 0;
     if (inb && cnt->done) {
         if (lead) {
             linkmask[b] = 0;
             if (dnear) dnear[b] = ndist[b];
         }
     } else if (inb) {
-        const double d = ndist[b];
-        const int32_t nn = near[b];
+        d = ndist[b];
+        nn = near[b];
         if (dnear && lead) dnear[b] = d;  // replaced below when the step is cut to range
         if (d == 0 || nn < 0) {
             if (lead) {
@@ -212,30 +208,40 @@ __global__ __launch_bounds__(kBlock) void prrt_steer_arm(SpaceArgs sp, SceneArgs
                 status[b] = ST_ZERO;
             }
         } else {
-            double a[D], r[D];
-#pragma unroll
-            for (int i = 0; i < D; ++i) {
-                a[i] = x64[(int64_t)nn * D + i];
-                r[i] = q[(int64_t)b * D + i];
-            }
-            if (d > range) {
-                space_interp_t<D>(sp, a, r, range / d, s);
-                if (dnear && lead) dnear[b] = space_dist_t<D>(sp, a, s);
-            } else {
-#pragma unroll
-                for (int i = 0; i < D; ++i) s[i] = r[i];
-            }
-            if (lead) {
-#pragma unroll
-                for (int i = 0; i < D; ++i) {
-                    from[(int64_t)b * D + i] = a[i];
-                    to[(int64_t)b * D + i] = s[i];
-                }
-            }
             need = true;
+            cut = d > range;
         }
     }
-    const bool ok = arm_ok_split<D, kArmLanes>(sc, [&](int i) { return s[i]; }, need);
+    const double* a = x64 + (int64_t)(need ? nn : 0) * D;
+    const double* r = q + (int64_t)(inb ? b : 0) * D;
+    const double f = cut ? range / d : 0.0;
+    // coordinate i of the new state: the sample, or space_interp_t's
+    // expression at range / d
+    auto state = [&](int i) { return cut ? (r[i] - a[i]) * f + a[i] : r[i]; };
+    if (need) {
+        if (cut && dnear && lead) {
+            double av[D], sv[D];
+#pragma unroll
+            for (int i = 0; i < D; ++i) {
+                av[i] = a[i];
+                sv[i] = state(i);
+            }
+            dnear[b] = space_dist_t<D>(sp, av, sv);
+        }
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int i = u * N + k;
+            from[(int64_t)b * D + i] = a[i];
+            to[(int64_t)b * D + i] = state(i);
+        }
+    }
+    double turn[N];
+    float len[N];
+    state_turns<D>(sc, state, turn, len);
+    // (a lane reads its group's row of `to` as its neighbours just wrote it)
+    __threadfence_block();
+    const double* s = need ? to + (int64_t)b * D : r;
+    const bool ok = arm_ok_near<D>(sc, turn, len, s, s, 0u, -1, need);
     if (need && lead) {
         status[b] = ok ? ST_LINK_FAIL : ST_INVALID;  // ST_LINK_FAIL until link() says otherwise
         linkmask[b] = ok ? 1 : 0;
@@ -250,31 +256,42 @@ __global__ __launch_bounds__(kBlock) void prrt_steer_arm(SpaceArgs sp, SceneArgs
 // (:427), which needs a tree node equal to it, hence an invalid tree node.
 // The host takes this path only while every tree node is known valid; then
 // only the valid samples are searched.  prrt_prevalid checks each sample
-// (L lanes per sample: the arm's split disk tests, else one), marks invalid
-// ones and lists the valid ones compactly (queries qv, sample ids vidx,
-// count *vcnt; list order is immaterial: every query is independent).
-template <int D, int L>
+// (ARM: five links per lane, arm_ok_near; else one lane per sample), marks
+// invalid ones and lists the valid ones compactly (queries qv, sample ids
+// vidx, count *vcnt; list order is immaterial: every query is independent).
+template <int D, bool ARM>
 __global__ __launch_bounds__(kBlock) void prrt_prevalid(SceneArgs sc, int dim, int B, const double* __restrict__ q,
                                                         uint8_t* __restrict__ status, uint8_t* __restrict__ linkmask,
                                                         double* __restrict__ qv, int32_t* __restrict__ vidx,
                                                         uint32_t* __restrict__ vcnt,
                                                         const Counters* __restrict__ cnt) {
     constexpr int DA = D > 0 ? D : kMaxDim;
+    constexpr int L = [] {
+        if constexpr (ARM) return near_lanes<D>();
+        else return 1;
+    }();
     const int dd = D > 0 ? D : dim;
     const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int b = (int)(t / L);
-    const bool lead = (t % L) == 0;
+    const int b = (int)(t / L), u = (int)(t % L);
+    const bool lead = u == 0;
     const bool inb = b < B;
     if (cnt->done) {  // nothing to link in an iteration past the stop
         if (inb && lead) linkmask[b] = 0;
         return;
     }
+    const double* row = q + (int64_t)(inb ? b : 0) * dd;
     double s[DA];
-#pragma unroll
-    for (int i = 0; i < DA; ++i) s[i] = (inb && i < dd) ? q[(int64_t)b * dd + i] : 0.0;
     bool ok;
-    if constexpr (L > 1) ok = arm_ok_split<D, L>(sc, [&](int i) { return s[i]; }, inb);
-    else ok = inb && state_valid_t<D>(sc, s);
+    if constexpr (ARM) {
+        double turn[kNearLinks];
+        float len[kNearLinks];
+        state_turns<D>(sc, [&](int i) { return row[i]; }, turn, len);
+        ok = arm_ok_near<D>(sc, turn, len, row, row, 0u, -1, inb);
+    } else {
+#pragma unroll
+        for (int i = 0; i < DA; ++i) s[i] = (inb && i < dd) ? row[i] : 0.0;
+        ok = inb && state_valid_t<D>(sc, s);
+    }
     const bool list = inb && lead && ok;
     if (inb && lead && !ok) {
         status[b] = ST_INVALID;
@@ -288,7 +305,16 @@ __global__ __launch_bounds__(kBlock) void prrt_prevalid(SceneArgs sc, int dim, i
         if (lane == __builtin_ctzll(m)) base = atomicAdd(vcnt, (uint32_t)__popcll(m));
         base = __shfl(base, __builtin_ctzll(m));
     }
-    if (list) {
+    if constexpr (ARM) {  // the group's lanes copy five coordinates each
+        const int first = lane & ~(L - 1);
+        if (inb && ok) {
+            const uint32_t k = base + (uint32_t)__popcll(m & (first ? (~0ull >> (64 - first)) : 0ull));
+            if (lead) vidx[k] = b;
+#pragma unroll
+            for (int i = 0; i < kNearLinks; ++i)
+                qv[(int64_t)k * D + u * kNearLinks + i] = row[u * kNearLinks + i];
+        }
+    } else if (list) {
         const uint32_t k = base + (uint32_t)__popcll(m & (lane ? (~0ull >> (64 - lane)) : 0ull));
         vidx[k] = b;
 #pragma unroll
@@ -370,7 +396,7 @@ void launch_steer(mptg_ctx* ctx, double range, int B, const double* q, const int
                   double* from, double* to, uint8_t* status, uint8_t* linkmask, double* dnear, const Counters* cnt) {
     if constexpr (D == 5 || D == 10 || D == 20) {
         if (ctx->scene.kind == MPTG_SCENE_ARM && ctx->scene.nlinks == D) {
-            const unsigned g = (unsigned)(((int64_t)B * kArmLanes + kBlock - 1) / kBlock);
+            const unsigned g = (unsigned)(((int64_t)B * near_lanes<D>() + kBlock - 1) / kBlock);
             hipLaunchKernelGGL((prrt_steer_arm<D>), dim3(g), dim3(kBlock), 0, ctx->stream, space_args(ctx),
                                scene_args(ctx), range, B, (const double*)ctx->x64, q, near, ndist, from, to, status,
                                linkmask, dnear, cnt);

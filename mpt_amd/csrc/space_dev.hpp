@@ -39,6 +39,16 @@ struct SceneArgs {
     const double* arm_index;   // disk grid, see ArmGrid
     const double* circles;     // shapes: [cx, cy, r^2, r] per circle
     int ncircles;
+    // arm, FP32 clearance bounds (arm_near.hpp): near_n x near_n cells over
+    // [-near_extent, near_extent]^2, each a run {first, count} of near_disks
+    // [cx, cy, squared distance below which a link surely hits, above which
+    // it surely clears] and of near_ids, their places in arm_disks;
+    // near_n = 0: none
+    const uint2* near_cells;
+    const float4* near_disks;
+    const int32_t* near_ids;
+    float near_extent, near_inv;
+    int near_n;
 };
 
 // Uniform grid over the disk centres.  Disks are stored by cell, row-major
@@ -55,6 +65,12 @@ MPTG_HD int arm_cell(double v, double v0, double inv, int n) {
     const double t = (v - v0) * inv;
     return t < 0.0 ? 0 : (t >= (double)n ? n - 1 : (int)t);
 }
+
+// FP32 clearance bounds of the arm (arm_near.hpp): cells per axis at most,
+// list entries at most (64 MiB), certainty margin relative to the scene.
+constexpr int kNearCells = 64;
+constexpr int kNearMaxEntries = 1 << 22;
+constexpr double kNearMargin = 0x1.0p-18;
 
 struct ArmGrid {
     double x0, y0, ix, iy, rtmax;
@@ -73,7 +89,8 @@ inline SceneArgs scene_args(const mptg_ctx* ctx) {
     return SceneArgs{s.kind,    s.boxes,  s.nboxes, s.grid,   s.width,
                      s.height,  s.grid_tx, s.lengths, s.nlinks, s.disks, s.ndisks,
                      (const ArmDisk*)s.arm_disks.p, (const double*)s.arm_lim.p, (const double*)s.arm_index.p,
-                     s.circles, s.ncircles};
+                     s.circles, s.ncircles, (const uint2*)s.near_cells.p, (const float4*)s.near_disks.p,
+                     (const int32_t*)s.near_ids.p, s.near_extent, s.near_inv, s.near_n};
 }
 
 __device__ __forceinline__ double so3_dist(const double* a, const double* b) {
@@ -304,213 +321,23 @@ __device__ __forceinline__ bool disk_clear(const ArmDisk& dk, double fx, double 
 //     links at a time (group-major keeps only that group's joints live);
 //   * a group's points all lie within its
 //     half-length S_g/2 of m_g = (p_first + p_last)/2 (triangle inequality);
-//   * for every disk, a group whose circle (m_g, rho_g + r + R) misses the
-//     disk centre is skipped; rho_g = S_g/2 (1 + 2^-30) + 1e-12 dominates the
-//     FK rounding, so every skipped (disk, link) pair would have passed the
-//     exact test;
+//   * a group whose circle (m_g, rho_g + r + R) misses a disk's centre passes
+//     it; rho_g = S_g/2 (1 + 2^-30) + 1e-12 dominates the FK rounding, so
+//     every skipped (disk, link) pair would have passed the exact test;
+//   * only the disks whose centre lies within (group half-length + the
+//     largest r + R) (1 + 2^-40) + 1e-12 of the group-circle centre, per
+//     axis, can fail that test (the margin dominates the rounding of
+//     dx*dx + dy*dy > R*R for coordinates below 10^3); they sit in the grid
+//     cells that box covers, one contiguous run per cell row;
 //   * the remaining pairs run disk_clear (the reference expression).
 // coord(i) yields the state's i-th coordinate, so callers can generate the
-// coordinates on the fly instead of holding the state in registers.
+// coordinates on the fly instead of holding the state in registers.  No
+// cross-lane operation: lanes may call it divergently.
 constexpr int kArmGroup = 5;
 
-// Work tally of arm_ok_fn (instrumented builds only): FK links, group tests,
-// link tests resolved by the far bound, link tests that ran the exact
-// expression, valid() calls.
-struct ArmWork {
-    uint32_t fk, group, far, exact, calls;
-};
-
-template <int D, bool COUNT = false, typename Coord>
-__device__ __forceinline__ bool arm_ok_fn(const SceneArgs& sc, Coord&& coord, ArmWork* wk = nullptr) {
+template <int D, typename Coord>
+__device__ __forceinline__ bool arm_ok_lane(const SceneArgs& sc, Coord&& coord) {
     constexpr int G = (D + kArmGroup - 1) / kArmGroup;
-    if constexpr (COUNT) wk->calls += 1;
-    double px = 0.0, py = 0.0, angle = 0.0;  // first joint of the current group
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        constexpr int GS = kArmGroup;
-        const int i0 = g * GS;
-        const int n = (i0 + GS <= D) ? GS : D - i0;
-        double jx[GS + 1], jy[GS + 1];
-        jx[0] = px;
-        jy[0] = py;
-#pragma unroll
-        for (int k = 0; k < GS; ++k) {
-            if (k < n) {
-                angle += coord(i0 + k);
-                double s, c;
-                pm::sincos(angle, &s, &c);
-                double L = sc.lengths[i0 + k];
-                jx[k + 1] = jx[k] + L * c;
-                jy[k + 1] = jy[k] + L * s;
-                if constexpr (COUNT) wk->fk += 1;
-            }
-        }
-        double last_x = jx[0], last_y = jy[0];
-#pragma unroll
-        for (int k = 1; k <= GS; ++k)
-            if (k <= n) {
-                last_x = jx[k];
-                last_y = jy[k];
-            }
-        const double mx = (jx[0] + last_x) / 2, my = (jy[0] + last_y) / 2;
-        const double rho = sc.arm_lim[D + g];
-        for (int j = 0; j < sc.ndisks; ++j) {
-            const ArmDisk dk = sc.arm_disks[j];
-            double dx = dk.cx - mx, dy = dk.cy - my;
-            double R = rho + dk.rt;
-            if constexpr (COUNT) wk->group += 1;
-            if (dx * dx + dy * dy > R * R) continue;
-#pragma unroll
-            for (int k = 0; k < GS; ++k) {
-                if (k < n) {
-                    double vx = jx[k + 1] - jx[k], vy = jy[k + 1] - jy[k];
-                    if constexpr (COUNT) {
-                        double wx = dk.cx - jx[k], wy = dk.cy - jy[k];
-                        double far = sc.arm_lim[i0 + k] + dk.rt;
-                        if (wx * wx + wy * wy > far * far) wk->far += 1;
-                        else wk->exact += 1;
-                    }
-                    if (!disk_clear(dk, jx[k], jy[k], jx[k + 1], jy[k + 1], vx, vy, sc.arm_lim[i0 + k]))
-                        return false;
-                }
-            }
-        }
-        px = last_x;
-        py = last_y;
-    }
-    return true;
-}
-
-__device__ __forceinline__ double wave_min_f64(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const double w = __shfl_xor(v, o);
-        v = w < v ? w : v;
-    }
-    return v;
-}
-__device__ __forceinline__ double wave_max_f64(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const double w = __shfl_xor(v, o);
-        v = w > v ? w : v;
-    }
-    return v;
-}
-
-// arm_ok_fn for a whole wave whose lanes check nearby states (one edge's
-// waypoints): every lane must call it (lanes with active == false compute on
-// any valid coordinates and return true).  Per group, the lanes' group-circle
-// centres span a box; a disk farther than (group half-length + r + R)
-// (1 + 2^-40) + 1e-12 outside that box fails every lane's own group test
-// (the margin dominates the rounding of dx*dx + dy*dy > R*R for coordinates
-// below 10^3), so the wave skips it with one uniform branch.  Other disks go
-// through the per-lane tests of arm_ok_fn unchanged.  Lanes that already
-// found a collision leave the box; the verdicts equal arm_ok_fn's.
-template <int D, bool COUNT = false, typename Coord>
-__device__ __forceinline__ bool arm_ok_wave(const SceneArgs& sc, Coord&& coord, bool active, ArmWork* wk = nullptr) {
-    constexpr int G = (D + kArmGroup - 1) / kArmGroup;
-    if constexpr (COUNT) wk->calls += active ? 1 : 0;
-    bool ok = true;
-    double px = 0.0, py = 0.0, angle = 0.0;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        constexpr int GS = kArmGroup;
-        const int i0 = g * GS;
-        const int n = (i0 + GS <= D) ? GS : D - i0;
-        double jx[GS + 1], jy[GS + 1];
-        jx[0] = px;
-        jy[0] = py;
-#pragma unroll
-        for (int k = 0; k < GS; ++k) {
-            if (k < n) {
-                angle += coord(i0 + k);
-                double s, c;
-                pm::sincos(angle, &s, &c);
-                double L = sc.lengths[i0 + k];
-                jx[k + 1] = jx[k] + L * c;
-                jy[k + 1] = jy[k] + L * s;
-                if constexpr (COUNT) wk->fk += (active && ok) ? 1 : 0;
-            }
-        }
-        double last_x = jx[0], last_y = jy[0];
-#pragma unroll
-        for (int k = 1; k <= GS; ++k)
-            if (k <= n) {
-                last_x = jx[k];
-                last_y = jy[k];
-            }
-        const double mx = (jx[0] + last_x) / 2, my = (jy[0] + last_y) / 2;
-        const bool live = active && ok;
-        if (__ballot(live) == 0) break;  // wave-uniform
-        const double inf = __builtin_inf();
-        const double bx0 = wave_min_f64(live ? mx : inf), bx1 = wave_max_f64(live ? mx : -inf);
-        const double by0 = wave_min_f64(live ? my : inf), by1 = wave_max_f64(live ? my : -inf);
-        const double rho = sc.arm_lim[D + g];
-        // disks whose centre lies within the box widened by the largest
-        // (group half-length + r + R) sit in the grid cells that box covers,
-        // one contiguous run per cell row; every other disk is farther than
-        // its own bound below
-        const ArmGrid ag = arm_grid(sc.arm_index);
-        const double Rmax = (rho + ag.rtmax) * (1.0 + 0x1.0p-40) + 1e-12;
-        const int gx0 = arm_cell(bx0 - Rmax, ag.x0, ag.ix, ag.nx), gx1 = arm_cell(bx1 + Rmax, ag.x0, ag.ix, ag.nx);
-        const int gy0 = arm_cell(by0 - Rmax, ag.y0, ag.iy, ag.ny), gy1 = arm_cell(by1 + Rmax, ag.y0, ag.iy, ag.ny);
-        for (int gy = gy0; gy <= gy1; ++gy) {
-        const int j0 = ag.starts[gy * ag.nx + gx0];
-        const int j1 = ag.starts[gy * ag.nx + gx1 + 1];
-        for (int jb = j0; jb < j1; jb += kDiskBatch) {
-            ArmDisk batch[kDiskBatch];
-#pragma unroll
-            for (int u = 0; u < kDiskBatch; ++u) batch[u] = sc.arm_disks[jb + u < j1 ? jb + u : j1 - 1];
-#pragma unroll
-            for (int u = 0; u < kDiskBatch; ++u) {
-                if (jb + u >= j1) break;  // uniform
-                const ArmDisk dk = batch[u];
-                const double Rw = (rho + dk.rt) * (1.0 + 0x1.0p-40) + 1e-12;
-                if (dk.cx < bx0 - Rw || dk.cx > bx1 + Rw || dk.cy < by0 - Rw || dk.cy > by1 + Rw) continue;  // uniform
-                if (!(active && ok)) continue;
-                double dx = dk.cx - mx, dy = dk.cy - my;
-                double R = rho + dk.rt;
-                if constexpr (COUNT) wk->group += 1;
-                if (dx * dx + dy * dy > R * R) continue;
-#pragma unroll
-                for (int k = 0; k < GS; ++k) {
-                    if (k < n && ok) {
-                        double vx = jx[k + 1] - jx[k], vy = jy[k + 1] - jy[k];
-                        if constexpr (COUNT) {
-                            double wx = dk.cx - jx[k], wy = dk.cy - jy[k];
-                            double far = sc.arm_lim[i0 + k] + dk.rt;
-                            if (wx * wx + wy * wy > far * far) wk->far += 1;
-                            else wk->exact += 1;
-                        }
-                        if (!disk_clear(dk, jx[k], jy[k], jx[k + 1], jy[k + 1], vx, vy, sc.arm_lim[i0 + k]))
-                            ok = false;
-                    }
-                }
-            }
-        }
-        }  // grid rows
-        px = last_x;
-        py = last_y;
-    }
-    return ok;
-}
-
-// arm_ok_fn for one lane on its own (states unrelated to their neighbours'):
-// per group, only the disks whose centre lies within (group half-length +
-// the largest r + R) (1 + 2^-40) + 1e-12 of the lane's group-circle centre,
-// per axis, can pass the group test; they sit in the grid cells that box
-// covers, one contiguous run per cell row.  Every other disk fails
-// arm_ok_fn's group test (the margin dominates the rounding of
-// dx*dx + dy*dy > R*R for coordinates below 10^3), so the verdict equals
-// arm_ok_fn's.  No cross-lane operation: lanes may call it divergently;
-// active == false returns true at once.
-template <int D, bool COUNT = false, typename Coord>
-__device__ __forceinline__ bool arm_ok_lane(const SceneArgs& sc, Coord&& coord, bool active = true,
-                                            ArmWork* wk = nullptr) {
-    if (!active) return true;
-    constexpr int G = (D + kArmGroup - 1) / kArmGroup;
-    if constexpr (COUNT) wk->calls += 1;
     const ArmGrid ag = arm_grid(sc.arm_index);
     double px = 0.0, py = 0.0, angle = 0.0;
 #pragma unroll
@@ -530,7 +357,6 @@ __device__ __forceinline__ bool arm_ok_lane(const SceneArgs& sc, Coord&& coord, 
                 double L = sc.lengths[i0 + k];
                 jx[k + 1] = jx[k] + L * c;
                 jy[k + 1] = jy[k] + L * s;
-                if constexpr (COUNT) wk->fk += 1;
             }
         }
         double last_x = jx[0], last_y = jy[0];
@@ -551,18 +377,11 @@ __device__ __forceinline__ bool arm_ok_lane(const SceneArgs& sc, Coord&& coord, 
                 const ArmDisk dk = sc.arm_disks[j];
                 double dx = dk.cx - mx, dy = dk.cy - my;
                 double R = rho + dk.rt;
-                if constexpr (COUNT) wk->group += 1;
                 if (dx * dx + dy * dy > R * R) continue;
 #pragma unroll
                 for (int k = 0; k < GS; ++k) {
                     if (k < n) {
                         double vx = jx[k + 1] - jx[k], vy = jy[k + 1] - jy[k];
-                        if constexpr (COUNT) {
-                            double wx = dk.cx - jx[k], wy = dk.cy - jy[k];
-                            double far = sc.arm_lim[i0 + k] + dk.rt;
-                            if (wx * wx + wy * wy > far * far) wk->far += 1;
-                            else wk->exact += 1;
-                        }
                         if (!disk_clear(dk, jx[k], jy[k], jx[k + 1], jy[k + 1], vx, vy, sc.arm_lim[i0 + k]))
                             return false;
                     }

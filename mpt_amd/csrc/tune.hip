@@ -135,8 +135,6 @@ int mptg_autotune_link(mptg_ctx* ctx, const double* d_from, const double* d_to, 
         return launch_link_masked(ctx, d_from, d_to, n, MPTG_ORDER_REFERENCE, 0, nullptr, verdict, checks);
     };
     if (arm_wave) {
-        if ((rc = sweep(ctx, MPTG_TUNE_ARM_CULL, {0, 1}, [&](int v) { ctx->tune.arm_cull = v; }, call, nullptr)))
-            return rc;
         return sweep(ctx, MPTG_TUNE_ARM_TAIL, {1, 2, 4, 8}, [&](int v) { ctx->tune.arm_tail_waves = v; }, call, rep);
     }
     if (ctx->scene.kind == MPTG_SCENE_MESH) {

@@ -42,7 +42,7 @@
 #include <utility>
 #include <vector>
 
-#include "space_dev.hpp"
+#include "arm_near.hpp"
 
 namespace mptg {
 namespace {
@@ -60,18 +60,19 @@ __host__ __device__ constexpr int64_t table16_row(int64_t m) {
 constexpr int64_t kMaxDmvWaypoints = (int64_t)1 << 24;
 constexpr int kMaxBisectDepth = 30;
 
-// valid() of n arm states, 8 lanes per state (arm_ok_split).
+// valid() of n arm states, five links per lane (arm_ok_near).
 template <int D>
 __global__ __launch_bounds__(kBlock) void valid_kernel_arm(SceneArgs sc, const double* __restrict__ q, int64_t n,
                                                            uint8_t* __restrict__ ok) {
-    constexpr int L = 8;
+    constexpr int L = near_lanes<D>();
     const int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int64_t i = t / L;
     const bool active = i < n;
-    double s[D];
-#pragma unroll
-    for (int j = 0; j < D; ++j) s[j] = active ? q[i * D + j] : 0.0;
-    const bool v = arm_ok_split<D, L>(sc, [&](int j) { return s[j]; }, active);
+    const double* s = q + (active ? i : 0) * D;
+    double turn[kNearLinks];
+    float len[kNearLinks];
+    state_turns<D>(sc, [&](int j) { return s[j]; }, turn, len);
+    const bool v = arm_ok_near<D>(sc, turn, len, s, s, 0u, -1, active);
     if (active && (t % L) == 0) ok[i] = v ? 1 : 0;
 }
 
@@ -470,19 +471,6 @@ __global__ __launch_bounds__(kBlock) void link_bisect(int D, SceneArgs sc, doubl
     bisect_edge<L2>(D, sc, tol, from, to, e, known_valid, verdict, checks);
 }
 
-// Exact walk of the edges the wave kernel listed (grid-stride over the list).
-__global__ __launch_bounds__(kBlock) void link_bisect_list(int D, SceneArgs sc, double tol,
-                                                           const double* __restrict__ from,
-                                                           const double* __restrict__ to, int known_valid,
-                                                           const int64_t* __restrict__ list,
-                                                           const uint32_t* __restrict__ list_count,
-                                                           uint8_t* __restrict__ verdict,
-                                                           uint32_t* __restrict__ checks) {
-    const int64_t cnt = *list_count;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * kBlock)
-        bisect_edge<false>(D, sc, tol, from, to, list[i], known_valid, verdict, checks);
-}
-
 // Instrumented bisection link (not timed): same walk and verdicts, and
 // accumulates [waypoint valid() calls, FK links, segment-disk tests, tests
 // within the per-link reach bound] for the arm scene into work[0..3].
@@ -640,7 +628,7 @@ int launch_valid(mptg_ctx* ctx, const double* d_q, int64_t n, uint8_t* d_ok) {
     if (ctx->scene.kind == MPTG_SCENE_HOST) return host_valid_dev(ctx, d_q, n, d_ok);
     if (ctx->scene.kind == MPTG_SCENE_ARM && ctx->scene.nlinks == ctx->dim &&
         (ctx->dim == 5 || ctx->dim == 10 || ctx->dim == 20)) {
-        const unsigned g = (unsigned)((n * 8 + kBlock - 1) / kBlock);
+        const unsigned g = (unsigned)((n * (ctx->dim / kNearLinks) + kBlock - 1) / kBlock);
         switch (ctx->dim) {
             case 5: hipLaunchKernelGGL(valid_kernel_arm<5>, dim3(g), dim3(kBlock), 0, ctx->stream, scene_args(ctx), d_q, n, d_ok); break;
             case 10: hipLaunchKernelGGL(valid_kernel_arm<10>, dim3(g), dim3(kBlock), 0, ctx->stream, scene_args(ctx), d_q, n, d_ok); break;
@@ -684,23 +672,8 @@ int launch_link_masked(mptg_ctx* ctx, const double* d_from, const double* d_to, 
         return fail(ctx, MPTG_E_STATE, "mesh scenes use the discrete motion validator link");
     if (ctx->link_mode == MPTG_LINK_BISECT) {
         if (ctx->scene.kind == MPTG_SCENE_ARM && !ctx->force_generic) {
-            int rc;
-            if ((rc = ensure(ctx, ctx->scratch[7], sizeof(int64_t) * n + 256))) return rc;
-            uint32_t* nirr = (uint32_t*)ctx->scratch[7].p;
-            int64_t* irr = (int64_t*)((char*)ctx->scratch[7].p + 256);
-            rc = launch_arm_link(ctx, d_from, d_to, n, known_valid, d_mask, d_verdict, d_checks, irr, nirr, nullptr,
-                                 order);
-            if (rc == MPTG_OK) {
-                phase_mark(ctx, 4);
-                // listed (irregular) edges: exact per-edge walk; usually an empty launch
-                hipLaunchKernelGGL(link_bisect_list, dim3(16), dim3(kBlock), 0, ctx->stream, ctx->dim,
-                                   scene_args(ctx), ctx->link_param, d_from, d_to, known_valid, (const int64_t*)irr,
-                                   (const uint32_t*)nirr, d_verdict, d_checks);
-                MPTG_HIP(ctx, hipGetLastError());
-                phase_mark(ctx, 5);
-                return MPTG_OK;
-            }
-            if (rc != MPTG_E_STATE) return rc;  // E_STATE: no wave kernel for this arm, use the generic one
+            const int rc = launch_arm_link(ctx, d_from, d_to, n, known_valid, d_mask, d_verdict, d_checks, nullptr, order);
+            if (rc != MPTG_E_STATE) return rc;  // E_STATE: no kernel for this arm, use the generic one
         }
         hipLaunchKernelGGL(link_bisect<false>, dim3(blocks), dim3(kBlock), 0, ctx->stream, ctx->dim,
                            scene_args(ctx), ctx->link_param, d_from, d_to, n, known_valid, d_mask, d_verdict,
@@ -765,12 +738,8 @@ int launch_link_work(mptg_ctx* ctx, const double* d_from, const double* d_to, in
                      unsigned long long* d_work, uint8_t* d_verdict, uint32_t* d_checks) {
     if (ctx->scene.kind != MPTG_SCENE_ARM || ctx->link_mode != MPTG_LINK_BISECT)
         return fail(ctx, MPTG_E_STATE, "work counting is implemented for the arm scene with bisection links");
-    int rc;
-    if ((rc = ensure(ctx, ctx->scratch[7], sizeof(int64_t) * n + 256))) return rc;
-    uint32_t* nirr = (uint32_t*)ctx->scratch[7].p;
-    int64_t* irr = (int64_t*)((char*)ctx->scratch[7].p + 256);
     MPTG_HIP(ctx, hipMemsetAsync(d_work, 0, 9 * sizeof(unsigned long long), ctx->stream));
-    rc = launch_arm_link(ctx, d_from, d_to, n, known_valid, nullptr, d_verdict, d_checks, irr, nirr, d_work, order);
+    const int rc = launch_arm_link(ctx, d_from, d_to, n, known_valid, nullptr, d_verdict, d_checks, d_work, order);
     if (rc) return rc == MPTG_E_STATE ? fail(ctx, rc, "no wave kernel for this arm") : rc;
     hipLaunchKernelGGL(link_bisect_work, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
                        ctx->dim, scene_args(ctx), ctx->link_param, d_from, d_to, n, known_valid, d_work + 5);

@@ -2,6 +2,7 @@
 
 Bar: bit-exact — node ids, FP64 distances, verdicts, check counts and whole
 trees must equal the oracle's on the same seeded inputs."""
+import dataclasses
 import math
 import sys
 
@@ -233,6 +234,61 @@ def test_arm_link_work_counts_equal_oracle(ctx_factory):
             (ow["calls"], ow["fk"], ow["tests"], ow["near_tests"]), kv
     da.free()
     db.free()
+
+
+def _tangent_arm(links, seed):
+    """An arm state whose second link lies at distance d of a point, and d."""
+    base = scenes.arm_scene(links=links, ndisks=3)
+    rng = np.random.default_rng(seed)
+    q0 = rng.uniform(-1.0, 1.0, links)
+    ang = np.cumsum(q0)
+    x1, y1 = base.lengths[0] * math.cos(ang[0]), base.lengths[0] * math.sin(ang[0])
+    ux, uy = math.cos(ang[1]), math.sin(ang[1])
+    d = 2.0
+    mid = 0.5 * base.lengths[1]
+    return base, q0, (x1 + mid * ux - d * uy, y1 + mid * uy + d * ux), d
+
+
+@pytest.mark.parametrize("links", [5, 10, 20])
+@pytest.mark.parametrize("n,span", [(70, 0.1), (70, 3.0), (2100, 0.3)])
+def test_arm_checks_at_the_bounds_are_exact(ctx_factory, links, n, span):
+    """Disks that touch a link which no edge moves, their radius within a few
+    ulps of the distance: every check is too close for the FP32 bounds, few
+    edges with few checks, then more checks than their list holds.  Also
+    states of thousands of turns.  Verdicts and counts equal the oracle's."""
+    base, q0, c, d = _tangent_arm(links, 50 + links)
+    rng = np.random.default_rng(51)
+    a = np.tile(q0, (n, 1))
+    b = a.copy()
+    b[:, -1] += rng.uniform(0.05, span, n)  # the last joint alone: the second link stays
+    for ulps in (-40, -1, 0, 1, 40):
+        r = d * (1.0 + ulps * 2.0 ** -52) - base.robot_radius
+        _say("arm at the bounds", links, n, span, ulps)
+        sc = dataclasses.replace(base, disks=np.array([[c[0], c[1], r]]))
+        ctx = ctx_factory()
+        ctx.scene(sc)
+        o = oracle.Oracle(sc)
+        q = np.concatenate([a[:50], b[:50]])
+        assert np.array_equal(ctx.valid(q), o.valid(q))
+        for kv in (False, True):
+            gv, gc = ctx.link(a, b, endpoints_known_valid=kv)
+            ov, oc = o.link(a, b, known_valid=kv, threads=16)
+            assert np.array_equal(gv, ov) and np.array_equal(gc, oc), (ulps, kv)
+    # a scene too small for the bounds takes the exact checks alone
+    for r in (0.4, 0.6):
+        tiny = dataclasses.replace(base, lengths=np.full(links, 1e-8), disks=np.array([[1.0, 0.0, r]]))
+        ctx.scene(tiny)
+        ot = oracle.Oracle(tiny)
+        assert np.array_equal(ctx.valid(q), ot.valid(q))
+        gv, gc = ctx.link(a, b)
+        ov, oc = ot.link(a, b, threads=16)
+        assert np.array_equal(gv, ov) and np.array_equal(gc, oc), r
+    ctx.scene(sc)
+    q = rng.uniform(-3000.0, 3000.0, (500, links))  # beyond the bounds' angles
+    assert np.array_equal(ctx.valid(q), o.valid(q))
+    gv, gc = ctx.link(q[:250], q[:250] + 0.3)
+    ov, oc = o.link(q[:250], q[:250] + 0.3, threads=16)
+    assert np.array_equal(gv, ov) and np.array_equal(gc, oc)
 
 
 # ---- whole trees -------------------------------------------------------------
