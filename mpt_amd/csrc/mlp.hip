@@ -4,20 +4,18 @@
 // orders the waypoint checks of link() so that likely collisions are tested
 // first — every verdict still comes from the exact checker.
 //
-// Matrix products use v_mfma_f32_16x16x32_bf16, one wave per 16x16 output
-// tile.  Operand layout (checked on the device): lane l supplies row l%16 of
-// A and column l%16 of B, k = 8*(l/16) .. +7; it receives column l%16 and
-// rows 4*(l/16) .. +3 of D.  Every product is written C = A * Bt^T with A and
-// Bt row-major, so both operands are contiguous 16-byte loads.  Epilogues:
-//   FWD  : + bias, ReLU, store H (BF16) and H^T (BF16, for the weight grads)
-//   DX   : zero where the layer input was 0 (ReLU'), store dH and dH^T (BF16)
-//   F32  : store FP32 (weight gradients)
-// Rounding points are those of the CPU oracle (oracle/orc_mlp.cpp).
+// Matrix products use v_mfma_f32_16x16x32_bf16.  Operand layout (checked on
+// the device): lane l supplies row l%16 of A and column l%16 of B, k =
+// 8*(l/16) .. +7; it receives column l%16 and rows 4*(l/16) .. +3 of D.
+// Every product is written C = A * Bt^T with A and Bt row-major, so both
+// operands are contiguous 16-byte loads.  Rounding points are those of the
+// CPU oracle (oracle/orc_mlp.cpp).
 //
 // Parameter layout (FP32 master copy, same as the oracle):
 //   W1[64][128] b1[128] W2[128][128] b2[128] W3[128][128] b3[128] w4[128] b4
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "bisect_dev.hpp"
@@ -34,145 +32,227 @@ constexpr int64_t OFF_W1 = 0, OFF_B1 = OFF_W1 + IN * HID, OFF_W2 = OFF_B1 + HID,
                   OFF_W3 = OFF_B2 + HID, OFF_B3 = OFF_W3 + HID * HID, OFF_W4 = OFF_B3 + HID,
                   OFF_B4 = OFF_W4 + HID, NPARAM = OFF_B4 + 1;
 
-enum { EPI_FWD = 0, EPI_DX = 1, EPI_F32 = 2 };
-
 __device__ __forceinline__ bf16x8 load8(const uint16_t* p) {
     uint4 v = *reinterpret_cast<const uint4*>(p);
     return __builtin_bit_cast(bf16x8, v);
 }
 
-struct Epi {
-    const float* bias;     // FWD
-    const uint16_t* mask;  // DX: layer input, [M][N]
-    uint16_t* out;         // FWD/DX: [M][N] BF16
-    uint16_t* out_t;       // FWD/DX: [N][M] BF16 (may be null)
-    float* out_f;          // F32: [M][N]
+// ---- forward and backward pass ---------------------------------------------
+// A batch is two launches.  mlp_pass: a block of 8 waves takes 16 rows at a
+// time through all layers, forward and back, with the activations in LDS;
+// wave w owns units 16 w .. 16 w + 15 of every hidden layer, so the ReLU masks
+// stay in its registers.  It leaves the transposed activations and their
+// gradients in memory.  mlp_update: a wave per 16 x 16 tile of a weight matrix
+// (and one per bias or output weight) sums the rows' products, sixteen
+// chunks of 32 rows in flight, and makes the Adam step and its BF16 copies from the
+// registers that hold the sum.
+//
+// The sums run over the rows in one chain each, as they always have: weights
+// are rounded to BF16 after every step, so a gradient that differs in its
+// last bit becomes another training run within a few steps (partial sums per
+// block, as fast, moved the weights by 5e-3 after 32 steps).
+//
+// What it replaced: one launch per product, transposition and sum, 19 for a
+// batch, every load of the sums waited for in turn.  A batch of 1024 rows
+// took 107 us, against 0.3 us of matrix instructions; now 11 + 9.5 us, the
+// chain of small layers and the trip of their operands between the XCDs' L2s.
+constexpr int kPassWaves = 8, kPassRows = 16;  // 1024 rows: 13.3 us in blocks of 32, 10.9 us of 16
+constexpr int kXS = IN + 8, kHS = HID + 8;  // row strides of [row][unit] arrays in LDS
+
+struct PassLds {
+    uint16_t x[kPassRows * kXS], h1[kPassRows * kHS], h2[kPassRows * kHS], h3[kPassRows * kHS];
+};
+struct PassLdsTrain : PassLds {
+    uint16_t d3[kPassRows * kHS], d2[kPassRows * kHS];
+    float z[kPassRows], dz[kPassRows];
 };
 
-// C[M][N] = A[M][K] * Bt[N][K]^T; M, N multiples of 16, K multiple of 32.
-template <int MODE>
-__global__ __launch_bounds__(256) void gemm_nt(int M, int N, int K, const uint16_t* __restrict__ A,
-                                               const uint16_t* __restrict__ Bt, Epi ep) {
-    const int lane = threadIdx.x & 63;
-    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int tiles_n = N / 16;
-    const int tm = tile / tiles_n, tn = tile % tiles_n;
-    if (tm * 16 >= M) return;
-    const int r = lane & 15, kq = lane >> 4;
-    const uint16_t* pa = A + (int64_t)(tm * 16 + r) * K + 8 * kq;
-    const uint16_t* pb = Bt + (int64_t)(tn * 16 + r) * K + 8 * kq;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < K; k0 += 32) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(pa + k0), load8(pb + k0), acc, 0, 0, 0);
-    const int n = tn * 16 + r;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = tm * 16 + 4 * kq + i;
-        float v = acc[i];
-        if constexpr (MODE == EPI_F32) {
-            ep.out_f[(int64_t)m * N + n] = v;
-        } else {
-            if constexpr (MODE == EPI_FWD) {
-                v = v + ep.bias[n];
-                v = v > 0.f ? v : 0.f;
-            } else {
-                if (ep.mask[(int64_t)m * N + n] == 0) v = 0.f;  // ReLU output is 0 or positive
-            }
-            uint16_t h = float_to_bf16(v);
-            ep.out[(int64_t)m * N + n] = h;
-            if (ep.out_t) ep.out_t[(int64_t)n * M + m] = h;
-        }
-    }
+// Transposed activations and gradients of a batch, [unit][Mp] BF16 (Mp = M
+// rounded up to 32; columns past M hold zero gradients), the logits' gradients
+// and the loss of each block.
+struct PassOut {
+    uint16_t *xt, *h1t, *h2t, *h3t, *d3t, *d2t, *d1t;
+    float *dz, *loss;
+    int64_t Mp;
+};
+
+// Block barrier for LDS alone: the transposed copies' stores stay in flight
+// across it (a full barrier waits for them, 7 times a tile).
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Output layer and loss: z = H3 . w4 + b4; dz = (sigmoid(z) - y) / N;
-// dH3 = bf16(dz * w4 where H3 > 0).  A block takes 64 rows, each wave 16 of
-// them in turn: lanes hold 2 of the 128 hidden units (coalesced row loads), a
-// wave reduction gives the logit, and the gradient row goes to dH3 directly
-// and to dH3^T through an LDS tile so both stores are coalesced.
-constexpr int kHeadRows = 64;
+// Rows [0, M) of X; logits to z (if not null).  TRAIN: labels y; the mean
+// loss's gradients (scaled by inv_n) to out.
+// Round to nearest even in hardware (finite values as float_to_bf16).
+__device__ __forceinline__ uint16_t to_bf16(float v) { return __builtin_bit_cast(uint16_t, (__bf16)v); }
 
-__global__ __launch_bounds__(256) void head_kernel(int M, const uint16_t* __restrict__ H3,
-                                                   const uint16_t* __restrict__ w4, const float* __restrict__ b4,
-                                                   const float* __restrict__ y, float inv_n, float* __restrict__ z,
-                                                   float* __restrict__ dz, uint16_t* __restrict__ dH3,
-                                                   uint16_t* __restrict__ dH3t, float* __restrict__ loss) {
-    __shared__ uint16_t tile[HID][kHeadRows + 2];
-    __shared__ float wl[4];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int r0 = blockIdx.x * kHeadRows;
-    const float wa = bf16_to_float(w4[2 * lane]), wb = bf16_to_float(w4[2 * lane + 1]);
-    float lsum = 0.f;
-    // all 16 row loads of this wave in flight before any is used
-    constexpr int kRowsPerWave = kHeadRows / 4;
-    uint32_t pairs[kRowsPerWave];
-    float ys[kRowsPerWave];
+template <bool TRAIN>
+__global__ __launch_bounds__(64 * kPassWaves) void mlp_pass(const uint16_t* __restrict__ X,
+                                                            const float* __restrict__ y, int64_t M, float inv_n,
+                                                            const uint16_t* __restrict__ wt,
+                                                            const uint16_t* __restrict__ wb,
+                                                            const float* __restrict__ p, float* __restrict__ z,
+                                                            PassOut out) {
+    __shared__ __attribute__((aligned(16))) std::conditional_t<TRAIN, PassLdsTrain, PassLds> S;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int r = lane & 15, q = lane >> 4;
+    const int unit = 16 * w + r;
+    constexpr int MT = kPassRows / 16;
+    // this wave's weights: B operands of the three layers (W^T rows, one per
+    // unit) and of the two products back (W rows)
+    bf16x8 w1[2], w2[4], w3[4], v3[TRAIN ? 4 : 1], v2[TRAIN ? 4 : 1];
 #pragma unroll
-    for (int j = 0; j < kRowsPerWave; ++j) {
-        const int r = r0 + wid + 4 * j;
-        pairs[j] = r < M ? reinterpret_cast<const uint32_t*>(H3 + (int64_t)r * HID)[lane] : 0u;
-        ys[j] = (y && r < M) ? y[r] : 0.f;
+    for (int k = 0; k < 2; ++k) w1[k] = load8(wt + unit * IN + 32 * k + 8 * q);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        w2[k] = load8(wt + IN * HID + unit * HID + 32 * k + 8 * q);
+        w3[k] = load8(wt + IN * HID + HID * HID + unit * HID + 32 * k + 8 * q);
+        if constexpr (TRAIN) {
+            v3[k] = load8(wb + IN * HID + HID * HID + unit * HID + 32 * k + 8 * q);
+            v2[k] = load8(wb + IN * HID + unit * HID + 32 * k + 8 * q);
+        }
     }
+    const float b1 = p[OFF_B1 + unit], b2 = p[OFF_B2 + unit], b3 = p[OFF_B3 + unit], b4 = p[OFF_B4];
+    const uint16_t* w4 = wb + IN * HID + 2 * HID * HID;
+    const float wa = bf16_to_float(w4[2 * lane]), wc = bf16_to_float(w4[2 * lane + 1]), wu = bf16_to_float(w4[unit]);
+    float lsum = 0.f;
+    // rows 16 mt .. of A (LDS, stride as) times this wave's 16 columns
+    auto product = [&](const uint16_t* A, int as, int mt, const bf16x8* B, int ks) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < ks; ++k)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load8(A + (16 * mt + r) * as + 32 * k + 8 * q), B[k], acc, 0, 0, 0);
+        return acc;
+    };
+    const int64_t tiles = (TRAIN ? out.Mp : M + kPassRows - 1) / kPassRows;
+    for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {  // block-uniform
+        const int64_t r0 = tile * kPassRows;
+        // four rows of this lane's unit: row-major in LDS, transposed in memory
+        auto store = [&](uint16_t* rows, uint16_t* cols, int mt, const uint16_t (&h)[4]) {
+            if (rows)
 #pragma unroll
-    for (int j = 0; j < kRowsPerWave; ++j) {
-        const int i = wid + 4 * j;
-        const int r = r0 + i;
-        uint16_t g0 = 0, g1 = 0;
-        if (r < M) {  // wave-uniform
-            const uint16_t h0 = (uint16_t)(pairs[j] & 0xffffu), h1 = (uint16_t)(pairs[j] >> 16);
-            float acc = bf16_to_float(h0) * wa + bf16_to_float(h1) * wb;
+                for (int i = 0; i < 4; ++i) rows[(16 * mt + 4 * q + i) * kHS + unit] = h[i];
+            if constexpr (TRAIN)
+                *reinterpret_cast<uint2*>(cols + (int64_t)unit * out.Mp + r0 + 16 * mt + 4 * q) =
+                    make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+        };
+        auto relu_layer = [&](const f32x4& acc, float bias, uint16_t (&h)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float v = acc[i] + bias;
+                h[i] = to_bf16(v > 0.f ? v : 0.f);
+            }
+        };
+        const int xrow = t / (IN / 8), xc = t % (IN / 8);  // threads below kPassRows * IN / 8
+        uint4 xv = make_uint4(0, 0, 0, 0);
+        if (xrow < kPassRows && r0 + xrow < M) xv = *reinterpret_cast<const uint4*>(X + (r0 + xrow) * IN + 8 * xc);
+        constexpr int kWaveRows = kPassRows / kPassWaves;
+        float ys[kWaveRows];
+        if constexpr (TRAIN) {
+#pragma unroll
+            for (int i = 0; i < kWaveRows; ++i) {
+                const int64_t gr = r0 + w * kWaveRows + i;
+                ys[i] = gr < M ? y[gr] : 0.f;
+            }
+        }
+        lds_barrier();  // the previous tile's operands have been read
+        if (xrow < kPassRows) *reinterpret_cast<uint4*>(S.x + xrow * kXS + 8 * xc) = xv;
+        lds_barrier();
+        if constexpr (TRAIN) {  // features transposed: 8 rows of one feature per thread
+            if (t < IN * kPassRows / 8) {
+                const int f = t / (kPassRows / 8), g = t % (kPassRows / 8);
+                uint32_t e[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    e[i] = (uint32_t)S.x[(8 * g + 2 * i) * kXS + f] | ((uint32_t)S.x[(8 * g + 2 * i + 1) * kXS + f] << 16);
+                *reinterpret_cast<uint4*>(out.xt + (int64_t)f * out.Mp + r0 + 8 * g) = make_uint4(e[0], e[1], e[2], e[3]);
+            }
+        }
+        uint16_t h1[MT][4], h2[MT][4], h3[MT][4];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            relu_layer(product(S.x, kXS, mt, w1, 2), b1, h1[mt]);
+            store(S.h1, out.h1t, mt, h1[mt]);
+        }
+        lds_barrier();
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            relu_layer(product(S.h1, kHS, mt, w2, 4), b2, h2[mt]);
+            store(S.h2, out.h2t, mt, h2[mt]);
+        }
+        lds_barrier();
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            relu_layer(product(S.h2, kHS, mt, w3, 4), b3, h3[mt]);
+            store(S.h3, out.h3t, mt, h3[mt]);
+        }
+        lds_barrier();
+        // the output unit: four rows per wave, two units per lane
+#pragma unroll
+        for (int i = 0; i < kWaveRows; ++i) {
+            const int row = w * kWaveRows + i;
+            const int64_t gr = r0 + row;
+            const uint32_t pair = *reinterpret_cast<const uint32_t*>(S.h3 + row * kHS + 2 * lane);
+            float acc = bf16_to_float((uint16_t)(pair & 0xffffu)) * wa + bf16_to_float((uint16_t)(pair >> 16)) * wc;
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-            const float zz = acc + b4[0];
-            if (z && lane == 0) z[r] = zz;
-            if (y) {
-                const float yy = ys[j];
-                const float d = (1.f / (1.f + expf(-zz)) - yy) * inv_n;
-                if (lane == 0) {
+            const float zz = acc + b4;
+            if (z && lane == 0 && gr < M) z[gr] = zz;
+            if constexpr (TRAIN) {
+                float dz = 0.f;
+                if (gr < M) {
+                    const float yy = ys[i];
+                    dz = (1.f / (1.f + expf(-zz)) - yy) * inv_n;
                     lsum += fmaxf(zz, 0.f) - zz * yy + log1pf(expf(-fabsf(zz)));
-                    dz[r] = d;
                 }
-                g0 = float_to_bf16(h0 != 0 ? d * wa : 0.f);
-                g1 = float_to_bf16(h1 != 0 ? d * wb : 0.f);
-                reinterpret_cast<uint32_t*>(dH3 + (int64_t)r * HID)[lane] = (uint32_t)g0 | ((uint32_t)g1 << 16);
+                if (lane == 0) {
+                    S.dz[row] = dz;
+                    out.dz[gr] = dz;
+                }
             }
         }
-        tile[2 * lane][i] = g0;
-        tile[2 * lane + 1][i] = g1;
+        if constexpr (TRAIN) {
+            lds_barrier();
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                uint16_t d[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    d[i] = to_bf16(h3[mt][i] != 0 ? S.dz[16 * mt + 4 * q + i] * wu : 0.f);
+                store(S.d3, out.d3t, mt, d);
+            }
+            lds_barrier();
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const f32x4 acc = product(S.d3, kHS, mt, v3, 4);
+                uint16_t d[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[i] = to_bf16(h2[mt][i] != 0 ? acc[i] : 0.f);
+                store(S.d2, out.d2t, mt, d);
+            }
+            lds_barrier();
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const f32x4 acc = product(S.d2, kHS, mt, v2, 4);
+                uint16_t d[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[i] = to_bf16(h1[mt][i] != 0 ? acc[i] : 0.f);
+                store(nullptr, out.d1t, mt, d);
+            }
+        }
     }
-    if (!y) return;  // block-uniform
-    if (lane == 0) wl[wid] = lsum;
-    __syncthreads();
-    // dH3^T rows k, columns r0 .. r0 + 63: 64 consecutive rows per k
-    for (int idx = threadIdx.x; idx < HID * kHeadRows; idx += 256) {
-        const int k = idx / kHeadRows, i = idx % kHeadRows;
-        if (r0 + i < M) dH3t[(int64_t)k * M + r0 + i] = tile[k][i];
+    if constexpr (TRAIN) {
+        lds_barrier();
+        if (lane == 0) S.z[w] = lsum;
+        lds_barrier();
+        if (t == 0) {
+            float l = 0.f;
+            for (int k = 0; k < kPassWaves; ++k) l += S.z[k];
+            out.loss[blockIdx.x] = l * inv_n;
+        }
     }
-    if (threadIdx.x == 0) atomicAdd(loss, (wl[0] + wl[1] + wl[2] + wl[3]) * inv_n);
-}
-
-// out[row] = sum_j X[row][j] * (w ? w[j] : 1), X BF16 [rows][len]: bias
-// gradients from dH^T rows, and dw4 from H3^T rows weighted by dz.
-__global__ __launch_bounds__(256) void row_sums(const uint16_t* __restrict__ X, int len, const float* __restrict__ w,
-                                                float* __restrict__ out) {
-    const uint16_t* x = X + (int64_t)blockIdx.x * len;
-    float acc = 0.f;
-    for (int j = threadIdx.x; j < len; j += blockDim.x) acc += bf16_to_float(x[j]) * (w ? w[j] : 1.f);
-    __shared__ float red[256];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[blockIdx.x] = red[0];
-}
-
-// Transpose of a BF16 matrix [rows][cols] -> [cols][rows].
-__global__ void transpose_bf16(const uint16_t* __restrict__ X, int rows, int cols, uint16_t* __restrict__ Xt) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)rows * cols) return;
-    int r = (int)(i / cols), c = (int)(i % cols);
-    Xt[(int64_t)c * rows + r] = X[i];
 }
 
 // BF16 operand copies of the FP32 master weights: W[in][out] and W^T[out][in].
@@ -199,17 +279,107 @@ __global__ void cast_weights(const float* __restrict__ p, uint16_t* __restrict__
     }
 }
 
-__global__ void adam_kernel(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                            const float* __restrict__ g, int64_t n, float lr, float b1, float b2, float eps, float c1,
-                            float c2) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float gi = g[i];
-    float mi = b1 * m[i] + (1.f - b1) * gi;
-    float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+// The gradient's sums and (adam) the step they make; loss_sum += the blocks'
+// losses.  One wave per item: the 16 x 16 tiles of W3, W2 and W1, then the
+// output weights, the biases of layers 3, 2 and 1, and the output bias.
+struct AdamArgs {
+    float *p, *m, *v;
+    uint16_t *wb, *wtb;
+    float lr, b1, b2, eps, c1, c2;
+};
+constexpr int kTilesH = (HID / 16) * (HID / 16), kTilesX = (IN / 16) * (HID / 16);
+constexpr int kUpdateItems = 2 * kTilesH + kTilesX + 4 * HID + 1;
+
+// sum_j x[j] * (wgt ? wgt[j] : 1) over [0, M): 256 strided sums, then a
+// pairwise tree; the total on lane 0.
+template <typename Value>
+__device__ __forceinline__ float strided_sum(int64_t M, int lane, Value&& value) {
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int64_t j = lane; j < M; j += 256) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (j + 64 * k < M) v[k] += value(j + 64 * k);
+    }
+    float x = (v[0] + v[2]) + (v[1] + v[3]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o);
+    return x;
+}
+
+__global__ __launch_bounds__(64) void mlp_update(PassOut in, int64_t M, int blocks, float* __restrict__ loss_sum,
+                                                  float* __restrict__ grad, int adam, AdamArgs A) {
+    const int lane = threadIdx.x;
+    int item = (int)blockIdx.x;
+    // parameter i, its gradient, and where its BF16 copies go (-1: none)
+    auto apply = [&](int64_t i, float g, int64_t copy, int64_t copy_t) {
+        if (!adam) {
+            grad[i] = g;
+            return;
+        }
+        const float mi = A.b1 * A.m[i] + (1.f - A.b1) * g;
+        const float vi = A.b2 * A.v[i] + (1.f - A.b2) * g * g;
+        A.m[i] = mi;
+        A.v[i] = vi;
+        const float w = A.p[i] - A.lr * (mi / A.c1) / (sqrtf(vi / A.c2) + A.eps);
+        A.p[i] = w;
+        if (copy >= 0) A.wb[copy] = float_to_bf16(w);
+        if (copy_t >= 0) A.wtb[copy_t] = float_to_bf16(w);
+    };
+    if (item < 2 * kTilesH + kTilesX) {
+        const int layer = item < kTilesH ? 3 : (item < 2 * kTilesH ? 2 : 1);
+        if (layer < 3) item -= layer == 2 ? kTilesH : 2 * kTilesH;
+        const int ti = item / (HID / 16), tj = item % (HID / 16);
+        const int r = lane & 15, q = lane >> 4;
+        const uint16_t* a = (layer == 3 ? in.h2t : (layer == 2 ? in.h1t : in.xt)) + (int64_t)(16 * ti + r) * in.Mp + 8 * q;
+        const uint16_t* b = (layer == 3 ? in.d3t : (layer == 2 ? in.d2t : in.d1t)) + (int64_t)(16 * tj + r) * in.Mp + 8 * q;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        int64_t k = 0;
+        auto chunks = [&]<int U>() {  // U chunks of 32 rows in flight
+            for (; k + 32 * U <= in.Mp; k += 32 * U) {
+                bf16x8 fa[U], fb[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    fa[u] = load8(a + k + 32 * u);
+                    fb[u] = load8(b + k + 32 * u);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // every load issued before the chain starts
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[u], fb[u], acc, 0, 0, 0);
+            }
+        };
+        chunks.template operator()<16>();
+        chunks.template operator()<4>();
+        chunks.template operator()<1>();
+        const int rows = layer == 1 ? IN : HID;
+        const int64_t off = layer == 3 ? OFF_W3 : (layer == 2 ? OFF_W2 : OFF_W1);
+        const int64_t copy = layer == 3 ? IN * HID + HID * HID : (layer == 2 ? IN * HID : 0);
+        const int o = 16 * tj + r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int in_u = 16 * ti + 4 * q + i;
+            apply(off + in_u * HID + o, acc[i], copy + in_u * HID + o, copy + (int64_t)o * rows + in_u);
+        }
+        return;
+    }
+    item -= 2 * kTilesH + kTilesX;
+    const int kind = item / HID, u = item % HID;  // 0: w4, 1..3: biases of layers 3..1, 4: b4
+    if (kind == 4) {
+        const float g = strided_sum(M, lane, [&](int64_t j) { return in.dz[j]; });
+        if (lane == 0) {
+            float l = 0.f;
+            for (int k = 0; k < blocks; ++k) l += in.loss[k];
+            *loss_sum += l;
+            apply(OFF_B4, g, -1, -1);
+        }
+        return;
+    }
+    const uint16_t* x = (kind == 0 ? in.h3t : (kind == 1 ? in.d3t : (kind == 2 ? in.d2t : in.d1t))) + (int64_t)u * in.Mp;
+    const float g = kind == 0 ? strided_sum(M, lane, [&](int64_t j) { return bf16_to_float(x[j]) * in.dz[j]; })
+                              : strided_sum(M, lane, [&](int64_t j) { return bf16_to_float(x[j]); });
+    if (lane == 0) {
+        if (kind == 0) apply(OFF_W4 + u, g, IN * HID + 2 * HID * HID + u, -1);
+        else apply((kind == 1 ? OFF_B3 : (kind == 2 ? OFF_B2 : OFF_B1)) + u, g, -1, -1);
+    }
 }
 
 __global__ void init_params(float* __restrict__ p, uint64_t seed) {
@@ -261,19 +431,6 @@ __device__ __forceinline__ void arm_features(const double* q, const double* leng
 
 namespace mptg {
 namespace {
-
-__global__ void sum_f32(const float* __restrict__ x, int n, float* __restrict__ out) {
-    float acc = 0.f;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) acc += x[j];
-    __shared__ float red[256];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = red[0];
-}
 
 template <int D>
 __global__ void features_kernel(const double* __restrict__ q, int64_t n, const double* __restrict__ lengths,
@@ -703,10 +860,10 @@ __global__ __launch_bounds__(256) void sample_waypoints(const double* __restrict
 // Device state of the surrogate (owned by the context).
 struct Surrogate {
     bool init = false;
-    int64_t cap = 0;  // rows the batch buffers hold
     int32_t adam_t = 0;
     DevBuf params, m, v, grad, wb, wtb, loss;
-    DevBuf x, xt, y, h1, h1t, h2, h2t, h3, h3t, z, dz, dh3, dh3t, dh2, dh2t, dh1, dh1t;
+    DevBuf pass;  // a batch's transposed activations and gradients (PassOut)
+    DevBuf x, y;  // a batch of features or labels whose own address is not aligned
 };
 
 Surrogate& surrogate(mptg_ctx* ctx) {
@@ -717,29 +874,12 @@ Surrogate& surrogate(mptg_ctx* ctx) {
 void surrogate_free(mptg_ctx* ctx) {
     if (!ctx->surrogate) return;
     Surrogate& S = *ctx->surrogate;
-    for (DevBuf* b : {&S.params, &S.m, &S.v, &S.grad, &S.wb, &S.wtb, &S.loss, &S.x, &S.xt, &S.y, &S.h1, &S.h1t,
-                      &S.h2, &S.h2t, &S.h3, &S.h3t, &S.z, &S.dz, &S.dh3, &S.dh3t, &S.dh2, &S.dh2t, &S.dh1, &S.dh1t})
-        (void)hipFree(b->p);
+    for (DevBuf* b : {&S.params, &S.m, &S.v, &S.grad, &S.wb, &S.wtb, &S.loss, &S.pass, &S.x, &S.y}) (void)hipFree(b->p);
     delete ctx->surrogate;
     ctx->surrogate = nullptr;
 }
 
 static constexpr int64_t kWb = IN * HID + 2 * HID * HID + HID;  // BF16 weight copies
-
-static int sur_reserve(mptg_ctx* ctx, Surrogate& S, int64_t rows) {
-    if (rows <= S.cap) return MPTG_OK;
-    int rc;
-    const size_t bh = sizeof(uint16_t) * HID * rows;
-    if ((rc = ensure(ctx, S.x, sizeof(uint16_t) * IN * rows))) return rc;
-    if ((rc = ensure(ctx, S.xt, sizeof(uint16_t) * IN * rows))) return rc;
-    if ((rc = ensure(ctx, S.y, sizeof(float) * rows))) return rc;
-    for (DevBuf* b : {&S.h1, &S.h1t, &S.h2, &S.h2t, &S.h3, &S.h3t, &S.dh3, &S.dh3t, &S.dh2, &S.dh2t, &S.dh1, &S.dh1t})
-        if ((rc = ensure(ctx, *b, bh))) return rc;
-    if ((rc = ensure(ctx, S.z, sizeof(float) * rows))) return rc;
-    if ((rc = ensure(ctx, S.dz, sizeof(float) * rows))) return rc;
-    S.cap = rows;
-    return MPTG_OK;
-}
 
 static int sur_alloc(mptg_ctx* ctx, Surrogate& S) {
     int rc;
@@ -758,60 +898,65 @@ static int sur_cast(mptg_ctx* ctx, Surrogate& S) {
     return MPTG_OK;
 }
 
-static void gemm(mptg_ctx* ctx, int mode, int M, int N, int K, const void* A, const void* Bt, Epi ep) {
-    unsigned blocks = (unsigned)(((int64_t)(M / 16) * (N / 16) + 3) / 4);
-    if (mode == EPI_FWD)
-        hipLaunchKernelGGL(gemm_nt<EPI_FWD>, dim3(blocks), dim3(256), 0, ctx->stream, M, N, K, (const uint16_t*)A,
-                           (const uint16_t*)Bt, ep);
-    else if (mode == EPI_DX)
-        hipLaunchKernelGGL(gemm_nt<EPI_DX>, dim3(blocks), dim3(256), 0, ctx->stream, M, N, K, (const uint16_t*)A,
-                           (const uint16_t*)Bt, ep);
-    else
-        hipLaunchKernelGGL(gemm_nt<EPI_F32>, dim3(blocks), dim3(256), 0, ctx->stream, M, N, K, (const uint16_t*)A,
-                           (const uint16_t*)Bt, ep);
+// The pass kernel reads feature rows as 16-byte words and labels as floats:
+// rows at another alignment are copied to a buffer first.
+static int sur_rows(mptg_ctx* ctx, Surrogate& S, const uint16_t* feat, const float* label, int64_t n,
+                    const uint16_t** x, const float** y) {
+    int rc;
+    *x = feat;
+    *y = label;
+    if ((uintptr_t)feat % 16) {
+        if ((rc = ensure(ctx, S.x, sizeof(uint16_t) * IN * (size_t)n))) return rc;
+        MPTG_HIP(ctx, hipMemcpyAsync(S.x.p, feat, sizeof(uint16_t) * IN * (size_t)n, hipMemcpyDeviceToDevice, ctx->stream));
+        *x = (const uint16_t*)S.x.p;
+    }
+    if ((uintptr_t)label % 4) {
+        if ((rc = ensure(ctx, S.y, sizeof(float) * (size_t)n))) return rc;
+        MPTG_HIP(ctx, hipMemcpyAsync(S.y.p, label, sizeof(float) * (size_t)n, hipMemcpyDeviceToDevice, ctx->stream));
+        *y = (const float*)S.y.p;
+    }
+    return MPTG_OK;
 }
 
-// Forward over M rows of S.x (M multiple of 16); logits to S.z.  With
-// labels (S.y) also the loss, dz and dH3.
-static void sur_forward(mptg_ctx* ctx, Surrogate& S, int M, bool with_loss) {
-    const uint16_t* wt = (const uint16_t*)S.wtb.p;
-    const float* p = (const float*)S.params.p;
-    gemm(ctx, EPI_FWD, M, HID, IN, S.x.p, wt, Epi{p + OFF_B1, nullptr, (uint16_t*)S.h1.p, (uint16_t*)S.h1t.p, nullptr});
-    gemm(ctx, EPI_FWD, M, HID, HID, S.h1.p, wt + IN * HID,
-         Epi{p + OFF_B2, nullptr, (uint16_t*)S.h2.p, (uint16_t*)S.h2t.p, nullptr});
-    gemm(ctx, EPI_FWD, M, HID, HID, S.h2.p, wt + IN * HID + HID * HID,
-         Epi{p + OFF_B3, nullptr, (uint16_t*)S.h3.p, (uint16_t*)S.h3t.p, nullptr});
-    hipLaunchKernelGGL(head_kernel, dim3((unsigned)((M + kHeadRows - 1) / kHeadRows)), dim3(256), 0, ctx->stream, M,
-                       (const uint16_t*)S.h3.p, (const uint16_t*)S.wb.p + IN * HID + 2 * HID * HID, p + OFF_B4,
-                       with_loss ? (const float*)S.y.p : nullptr, 1.0f / (float)M, (float*)S.z.p, (float*)S.dz.p,
-                       (uint16_t*)S.dh3.p, (uint16_t*)S.dh3t.p, (float*)S.loss.p);
-}
-
-// Gradient of the mean loss over the M rows already forwarded; into S.grad.
-static void sur_backward(mptg_ctx* ctx, Surrogate& S, int M) {
-    float* g = (float*)S.grad.p;
-    const uint16_t* wb = (const uint16_t*)S.wb.p;
-    hipLaunchKernelGGL(row_sums, dim3(HID), dim3(256), 0, ctx->stream, (const uint16_t*)S.h3t.p, M,
-                       (const float*)S.dz.p, g + OFF_W4);
-    hipLaunchKernelGGL(sum_f32, dim3(1), dim3(256), 0, ctx->stream, (const float*)S.dz.p, M, g + OFF_B4);
-    // layer 3
-    gemm(ctx, EPI_F32, HID, HID, M, S.h2t.p, S.dh3t.p, Epi{nullptr, nullptr, nullptr, nullptr, g + OFF_W3});
-    hipLaunchKernelGGL(row_sums, dim3(HID), dim3(256), 0, ctx->stream, (const uint16_t*)S.dh3t.p, M,
-                       (const float*)nullptr, g + OFF_B3);
-    gemm(ctx, EPI_DX, M, HID, HID, S.dh3.p, wb + IN * HID + HID * HID,
-         Epi{nullptr, (const uint16_t*)S.h2.p, (uint16_t*)S.dh2.p, (uint16_t*)S.dh2t.p, nullptr});
-    // layer 2
-    gemm(ctx, EPI_F32, HID, HID, M, S.h1t.p, S.dh2t.p, Epi{nullptr, nullptr, nullptr, nullptr, g + OFF_W2});
-    hipLaunchKernelGGL(row_sums, dim3(HID), dim3(256), 0, ctx->stream, (const uint16_t*)S.dh2t.p, M,
-                       (const float*)nullptr, g + OFF_B2);
-    gemm(ctx, EPI_DX, M, HID, HID, S.dh2.p, wb + IN * HID,
-         Epi{nullptr, (const uint16_t*)S.h1.p, (uint16_t*)S.dh1.p, (uint16_t*)S.dh1t.p, nullptr});
-    // layer 1
-    hipLaunchKernelGGL(transpose_bf16, dim3((unsigned)(((int64_t)M * IN + 255) / 256)), dim3(256), 0, ctx->stream,
-                       (const uint16_t*)S.x.p, M, IN, (uint16_t*)S.xt.p);
-    gemm(ctx, EPI_F32, IN, HID, M, S.xt.p, S.dh1t.p, Epi{nullptr, nullptr, nullptr, nullptr, g + OFF_W1});
-    hipLaunchKernelGGL(row_sums, dim3(HID), dim3(256), 0, ctx->stream, (const uint16_t*)S.dh1t.p, M,
-                       (const float*)nullptr, g + OFF_B1);
+// Gradient and loss of the mean over n rows, the gradient to S.grad or (step)
+// into an Adam step; the loss is added to S.loss.
+static int sur_batch(mptg_ctx* ctx, Surrogate& S, const uint16_t* feat, const float* label, int64_t n, bool step,
+                     float lr) {
+    int rc;
+    const int64_t Mp = (n + 31) / 32 * 32;  // whole chunks of the sums
+    // a block reads the weights once for all its rows: no more blocks than
+    // the chip holds at once
+    const int blocks = (int)std::min<int64_t>((int64_t)ctx->cus * 2, Mp / kPassRows);
+    const size_t col = sizeof(uint16_t) * (size_t)Mp;
+    if ((rc = ensure(ctx, S.pass, col * (IN + 6 * HID) + sizeof(float) * (size_t)(Mp + ctx->cus * 2)))) return rc;
+    PassOut o;
+    o.Mp = Mp;
+    o.xt = (uint16_t*)S.pass.p;
+    o.h1t = o.xt + (size_t)IN * Mp;
+    o.h2t = o.h1t + (size_t)HID * Mp;
+    o.h3t = o.h2t + (size_t)HID * Mp;
+    o.d3t = o.h3t + (size_t)HID * Mp;
+    o.d2t = o.d3t + (size_t)HID * Mp;
+    o.d1t = o.d2t + (size_t)HID * Mp;
+    o.dz = (float*)(o.d1t + (size_t)HID * Mp);
+    o.loss = o.dz + Mp;
+    const uint16_t* x;
+    const float* y;
+    if ((rc = sur_rows(ctx, S, feat, label, n, &x, &y))) return rc;
+    hipLaunchKernelGGL(mlp_pass<true>, dim3((unsigned)blocks), dim3(64 * kPassWaves), 0, ctx->stream, x, y, n,
+                       1.0f / (float)n, (const uint16_t*)S.wtb.p, (const uint16_t*)S.wb.p, (const float*)S.params.p,
+                       (float*)nullptr, o);
+    AdamArgs A{(float*)S.params.p, (float*)S.m.p, (float*)S.v.p, (uint16_t*)S.wb.p, (uint16_t*)S.wtb.p,
+               lr, 0.9f, 0.999f, 1e-8f, 1.f, 1.f};
+    if (step) {
+        S.adam_t += 1;
+        A.c1 = 1.f - std::pow(A.b1, (float)S.adam_t);
+        A.c2 = 1.f - std::pow(A.b2, (float)S.adam_t);
+    }
+    hipLaunchKernelGGL(mlp_update, dim3((unsigned)kUpdateItems), dim3(64), 0, ctx->stream, o, n, blocks,
+                       (float*)S.loss.p, (float*)S.grad.p, step ? 1 : 0, A);
+    MPTG_HIP(ctx, hipGetLastError());
+    return MPTG_OK;
 }
 
 static int sur_check(mptg_ctx* ctx, bool need_init) {
@@ -985,18 +1130,15 @@ int mptg_surrogate_forward(mptg_ctx* ctx, const uint16_t* d_feat, int64_t n, flo
     int rc = check_device(ctx);
     if (rc || (rc = sur_check(ctx, true))) return rc;
     if (n < 0 || (n > 0 && (!d_feat || !d_logits))) return fail(ctx, MPTG_E_ARG, "bad buffers");
+    if (n == 0) return MPTG_OK;
     Surrogate& S = surrogate(ctx);
-    const int64_t chunk = 1 << 16;
-    for (int64_t r0 = 0; r0 < n; r0 += chunk) {
-        int64_t m = std::min(chunk, n - r0);
-        int M = (int)((m + 15) / 16 * 16);
-        if ((rc = sur_reserve(ctx, S, M))) return rc;
-        MPTG_HIP(ctx, hipMemsetAsync(S.x.p, 0, sizeof(uint16_t) * IN * M, ctx->stream));
-        MPTG_HIP(ctx, hipMemcpyAsync(S.x.p, d_feat + r0 * IN, sizeof(uint16_t) * IN * m, hipMemcpyDeviceToDevice,
-                                     ctx->stream));
-        sur_forward(ctx, S, M, false);
-        MPTG_HIP(ctx, hipMemcpyAsync(d_logits + r0, S.z.p, sizeof(float) * m, hipMemcpyDeviceToDevice, ctx->stream));
-    }
+    const uint16_t* x;
+    const float* y;
+    if ((rc = sur_rows(ctx, S, d_feat, nullptr, n, &x, &y))) return rc;
+    const int64_t blocks = std::min<int64_t>((n + kPassRows - 1) / kPassRows, (int64_t)ctx->cus * 4);
+    hipLaunchKernelGGL(mlp_pass<false>, dim3((unsigned)blocks), dim3(64 * kPassWaves), 0, ctx->stream, x, y, n, 0.f,
+                       (const uint16_t*)S.wtb.p, (const uint16_t*)S.wb.p, (const float*)S.params.p, d_logits,
+                       PassOut{});
     MPTG_HIP(ctx, hipGetLastError());
     return MPTG_OK;
 }
@@ -1009,13 +1151,8 @@ int mptg_surrogate_loss_grad(mptg_ctx* ctx, const uint16_t* d_feat, const float*
     if (n <= 0 || n % 16 || n > (1 << 20) || !d_feat || !d_label)
         return fail(ctx, MPTG_E_ARG, "batch rows must be a positive multiple of 16 (at most 2^20)");
     Surrogate& S = surrogate(ctx);
-    if ((rc = sur_reserve(ctx, S, n))) return rc;
-    MPTG_HIP(ctx, hipMemcpyAsync(S.x.p, d_feat, sizeof(uint16_t) * IN * n, hipMemcpyDeviceToDevice, ctx->stream));
-    MPTG_HIP(ctx, hipMemcpyAsync(S.y.p, d_label, sizeof(float) * n, hipMemcpyDeviceToDevice, ctx->stream));
     MPTG_HIP(ctx, hipMemsetAsync(S.loss.p, 0, sizeof(float), ctx->stream));
-    sur_forward(ctx, S, (int)n, true);
-    sur_backward(ctx, S, (int)n);
-    MPTG_HIP(ctx, hipGetLastError());
+    if ((rc = sur_batch(ctx, S, d_feat, d_label, n, false, 0.f))) return rc;
     if (h_loss) MPTG_HIP(ctx, hipMemcpyAsync(h_loss, S.loss.p, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
     if (h_grad)
         MPTG_HIP(ctx, hipMemcpyAsync(h_grad, S.grad.p, sizeof(float) * NPARAM, hipMemcpyDeviceToHost, ctx->stream));
@@ -1033,27 +1170,11 @@ int mptg_surrogate_train(mptg_ctx* ctx, const uint16_t* d_feat, const float* d_l
     if (batch <= 0 || batch % 16 || batch > (1 << 16)) return fail(ctx, MPTG_E_ARG, "batch must be a multiple of 16");
     if (n < batch || epochs < 1 || !(lr > 0) || !d_feat || !d_label) return fail(ctx, MPTG_E_ARG, "bad training args");
     Surrogate& S = surrogate(ctx);
-    if ((rc = sur_reserve(ctx, S, batch))) return rc;
     const int64_t nb = n / batch;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     for (int ep = 0; ep < epochs; ++ep) {
         MPTG_HIP(ctx, hipMemsetAsync(S.loss.p, 0, sizeof(float) * 2, ctx->stream));
-        for (int64_t bi = 0; bi < nb; ++bi) {
-            const int64_t r0 = bi * batch;
-            MPTG_HIP(ctx, hipMemcpyAsync(S.x.p, d_feat + r0 * IN, sizeof(uint16_t) * IN * batch,
-                                         hipMemcpyDeviceToDevice, ctx->stream));
-            MPTG_HIP(ctx, hipMemcpyAsync(S.y.p, d_label + r0, sizeof(float) * batch, hipMemcpyDeviceToDevice,
-                                         ctx->stream));
-            sur_forward(ctx, S, batch, true);
-            sur_backward(ctx, S, batch);
-            S.adam_t += 1;
-            float c1 = 1.f - std::pow(b1, (float)S.adam_t), c2 = 1.f - std::pow(b2, (float)S.adam_t);
-            hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((NPARAM + 255) / 256)), dim3(256), 0, ctx->stream,
-                               (float*)S.params.p, (float*)S.m.p, (float*)S.v.p, (const float*)S.grad.p,
-                               (int64_t)NPARAM, lr, b1, b2, eps, c1, c2);
-            if ((rc = sur_cast(ctx, S))) return rc;
-        }
-        MPTG_HIP(ctx, hipGetLastError());
+        for (int64_t bi = 0; bi < nb; ++bi)
+            if ((rc = sur_batch(ctx, S, d_feat + bi * batch * IN, d_label + bi * batch, batch, true, lr))) return rc;
         if (h_losses) {
             float tot = 0.f;
             MPTG_HIP(ctx, hipMemcpyAsync(&tot, S.loss.p, sizeof(float), hipMemcpyDeviceToHost, ctx->stream));

@@ -100,6 +100,35 @@ def test_adam_step_parity(ctx_factory):
     assert np.mean(np.abs(p1 - e1) <= 1e-6) > 0.999
 
 
+@pytest.mark.parametrize("n", [16, 32, 48, 256, 4112, 16432])
+def test_pass_sizes_parity(ctx_factory, n):
+    """A half tile of rows, whole tiles, tiles that end half full, a sum's
+    unrolled chunks (256 rows) with and without a rest, and more tiles than
+    blocks (16384 rows), from aligned rows and from rows the pass
+    kernel has to copy (2-byte offset): loss and gradient against the oracle
+    with test_loss_grad_parity's bounds, and the logits of the same rows."""
+    _say("surrogate pass", n)
+    ctx = ctx_factory()
+    p = _net(18)
+    X, y = _data(19, n)
+    ctx.surrogate_set(p)
+    ol, og, oz = oracle.mlp_loss_grad(p, X, y)
+    dy, dz = ctx.to_device(y), ctx.array(n, np.float32)
+    for shift in (0, 1):
+        dX = ctx.to_device(np.concatenate([np.zeros(shift, np.uint16), X.ravel()]))
+        ptr = dX.ptr + 2 * shift
+        loss, g = ctx.surrogate_loss_grad(ptr, dy.ptr, n)
+        assert abs(loss - ol) <= 1e-4 * abs(ol)
+        for name, a, b in _tensor_slices():
+            gg, oo = g[a:b].astype(np.float64), og[a:b].astype(np.float64)
+            assert np.linalg.norm(gg - oo) <= 1e-2 * np.linalg.norm(oo) + 1e-7, (shift, name)
+        ctx.surrogate_forward(ptr, n, dz.ptr)
+        assert np.allclose(dz.numpy(), oz, rtol=2e-2, atol=2e-2), shift
+    # the sums' order is fixed: the same bits every time
+    l2, g2 = ctx.surrogate_loss_grad(ptr, dy.ptr, n)
+    assert l2 == loss and np.array_equal(g2, g)
+
+
 def test_features_match_forward_kinematics(ctx_factory):
     _say("surrogate features")
     ctx = ctx_factory()
