@@ -349,7 +349,7 @@ typedef struct mptg_tune_params {
     int32_t arm_tail_waves;         /* kept for callers that set it (1..8); the arm link kernels
                                        choose their waves from the batch size */
     int32_t arm_cull;               /* likewise (0 or 1) */
-    int32_t mesh_edge_waves;        /* waves sharing one mesh edge's waypoints (1..32) */
+    int32_t mesh_edge_waves;        /* kept likewise (1..32): a mesh edge's waypoints go to any wave */
     int32_t knn_select;             /* k > 1 on trees of 2^16 nodes or more: 1 bound, collect and
                                        select (registers of k = 1 in the scan), 0 the k-list scan */
     int32_t knn_grid;               /* L1/L2 in 2..8 dimensions on trees of 2^16 nodes or more: 1 a

@@ -582,14 +582,14 @@ int launch_arm_link(mptg_ctx* ctx, const double* from, const double* to, int64_t
     DevBuf& buf = ctx->scratch[10];
     const int64_t cap = n + 4096;  // checks in doubt
     const size_t need = kArmListsBytes + sizeof(int64_t) * (size_t)(2 * n + cap);
-    if (!buf.p || buf.bytes < need) ctx->arm_lists_clean = false;
+    if (!buf.p || buf.bytes < need) ctx->link_lists_clean = false;
     if ((rc = ensure(ctx, buf, need))) return rc;
     ArmLinkArgs A{from, to, n, known_valid, mask, ctx->link_param, scene_args(ctx), nullptr, verdict, checks,
                   (ArmLists*)buf.p, (int64_t*)((char*)buf.p + kArmListsBytes), nullptr, nullptr, (uint32_t)cap, work};
     A.irregular = A.open + n;
     A.doubt = (uint64_t*)(A.irregular + n);
-    if (!ctx->arm_lists_clean && (rc = launch_zero_u32(ctx, (uint32_t*)A.lists, kArmListsBytes / 4))) return rc;
-    ctx->arm_lists_clean = false;  // until both kernels are enqueued
+    if (!ctx->link_lists_clean && (rc = launch_zero_u32(ctx, (uint32_t*)A.lists, kArmListsBytes / 4))) return rc;
+    ctx->link_lists_clean = false;  // until both kernels are enqueued
     phase_mark(ctx, 0);
     switch (ctx->dim) {
         case 5: rc = launch_arm_d<5>(ctx, order, A); break;
@@ -598,7 +598,7 @@ int launch_arm_link(mptg_ctx* ctx, const double* from, const double* to, int64_t
     }
     if (rc) return rc;
     MPTG_HIP(ctx, hipGetLastError());
-    ctx->arm_lists_clean = true;
+    ctx->link_lists_clean = true;
     return MPTG_OK;
 }
 

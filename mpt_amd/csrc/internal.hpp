@@ -150,10 +150,10 @@ struct mptg_ctx {
     // unsorted pairs and sort scratch; staged host queries; sorted results
     mptg::DevBuf rnn_buf, rnn_pairs, rnn_q, rnn_out;
     mptg::DevBuf scratch[12];  // 0-2 host staging, 3 kNN seed bounds, 4-5 kNN partials, 6 DMV table, 7 edge lists, 8 scores,
-                               // 9 surrogate picks, 10 arm link counters and lists
-    // the arm link's list counters are zero (its second kernel clears them);
+                               // 9 surrogate picks, 10 arm / mesh link counters and lists
+    // the arm or mesh link's list counters are zero (its last kernel clears them);
     // false after an allocation or a failed launch
-    bool arm_lists_clean = false;
+    bool link_lists_clean = false;
     // pinned host staging
     void* pinned = nullptr;
     size_t pinned_bytes = 0;
@@ -171,10 +171,11 @@ struct mptg_ctx {
     // graph is replayed only while the epoch it was captured at holds
     uint64_t epoch = 0;
     // launch shapes (mptg_autotune_*): kNN blocks per CU, waves per CU of the
-    // persistent DMV long-edge kernel and of the mesh kernels, two that the
-    // arm link no longer reads, waves per mesh edge, kNN select and grid paths, lanes per DMV edge, the
-    // byte prefilter of the k = 1 L1 scan
-    mptg_tune_params tune{8, 16, 32, 2, 0, 2, 1, 1, 8, 1};
+    // persistent DMV long-edge kernel and of the mesh kernels (32 -> 128:
+    // see mesh_link), two that the arm link and one that the mesh link no
+    // longer reads, kNN select and grid paths, lanes per DMV edge, the byte
+    // prefilter of the k = 1 L1 scan
+    mptg_tune_params tune{8, 16, 128, 2, 0, 2, 1, 1, 8, 1};
     hipEvent_t phase_ev[6] = {};
 };
 
@@ -244,10 +245,6 @@ int rnn_fill(mptg_ctx* ctx, const double* d_q, int64_t nq, double r, int64_t tot
 bool rnn_dim_ok(int dim);
 // Zeroes n 32-bit words with a kernel (graph-capturable, unlike a memset).
 int launch_zero_u32(mptg_ctx* ctx, uint32_t* p, int64_t n);
-// Zeroes the 32-bit words *a and *b with one small kernel.
-int launch_zero_pair(mptg_ctx* ctx, uint32_t* a, uint32_t* b);
-// Sets n 32-bit words to v with a kernel.
-int launch_fill_u32(mptg_ctx* ctx, uint32_t* p, int64_t n, uint32_t v);
 // nq_dev (k = 1, L1/L2): only the first *nq_dev of the nq query slots are
 // live (nq stays the layout); the scans run, planned for half the slots.
 int launch_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radius, int32_t* d_idx,

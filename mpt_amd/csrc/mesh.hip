@@ -17,8 +17,8 @@
 //             consecutive triangles a lane owns are close together
 // Kernels (one 64-lane wave per block, one item per wave at a time):
 //   mesh_valid  one state per wave
-//   mesh_link   one edge per wave; waypoints in DMV order one at a time
-//               (reference checks_done counts), early exit on the first hit
+//   mesh_link   one waypoint of one edge per wave at a time (reference
+//               checks_done counts), nothing past an edge's first hit
 // Per state, lane l poses robot triangles [4l, 4l + 4) of each 256-triangle
 // chunk and takes their box; the wave walks the env BVH depth-first once with
 // one LDS stack, visiting a node when any lane's box overlaps it, and stops
@@ -292,8 +292,8 @@ __device__ __forceinline__ void load_env_tri(const float4* __restrict__ t, int i
     hi[0] = d.x; hi[1] = d.y; hi[2] = d.z;
 }
 
-// Does the robot at state q collide with the environment?  Whole wave; q is
-// the same on every lane.  stack: this wave's kStackSlots LDS slots.
+// Does the robot at `pose` collide with the environment?  Whole wave; the
+// pose is the same on every lane.  stack: this wave's kStackSlots LDS slots.
 //
 // Per 256-triangle chunk, lane l poses robot triangles [4l, 4l + 4) and takes
 // their box; the wave walks the environment BVH depth-first once, visiting a
@@ -303,10 +303,9 @@ __device__ __forceinline__ void load_env_tri(const float4* __restrict__ t, int i
 // tested only when the boxes overlap, as the predicate requires, and a lane
 // whose box overlaps a leaf overlaps every ancestor of it, so the pairs
 // tested are those a per-lane walk would test.
-__device__ bool mesh_collides(const MeshArgs& m, const double* q, int32_t* stack) {
+__device__ bool mesh_collides(const MeshArgs& m, const Pose32& pose, int32_t* stack) {
     const int lane = threadIdx.x & 63;
     if (m.nnodes == 0 || m.nrobot == 0) return false;
-    const Pose32 pose = pose_from_state(q);
     for (int c0 = 0; c0 < m.nrobot; c0 += kChunkTris) {
         const int first = c0 + lane * kLaneTris;
         const int cnt = max(0, min(kLaneTris, m.nrobot - first));
@@ -397,7 +396,7 @@ __global__ __launch_bounds__(64) void mesh_valid(MeshArgs m, const double* __res
         double s[7];
 #pragma unroll
         for (int j = 0; j < 7; ++j) s[j] = q[i * 7 + j];
-        const bool hit = mesh_collides(m, s, stack);
+        const bool hit = mesh_collides(m, pose_from_state(s), stack);
         if (threadIdx.x == 0) ok[i] = hit ? 0 : 1;
     }
 }
@@ -411,7 +410,7 @@ __global__ __launch_bounds__(64) void mesh_filter(MeshArgs m, const double* __re
         double s[7];
 #pragma unroll
         for (int j = 0; j < 7; ++j) s[j] = q[i * 7 + j];
-        const bool hit = mesh_collides(m, s, stack);
+        const bool hit = mesh_collides(m, pose_from_state(s), stack);
         if (threadIdx.x == 0 && hit) {
             mask[i] = 0;
             status[i] = (uint8_t)invalid_code;
@@ -419,144 +418,239 @@ __global__ __launch_bounds__(64) void mesh_filter(MeshArgs m, const double* __re
     }
 }
 
-// DMV link (src/mpt/discrete_motion_validator.hpp:71-130), one edge per wave:
-// valid(to) unless the caller vouches for it, then the interior waypoints in
-// the reference's ring order (table for up to 255, ring replay beyond).
-// link() of n edges, P waves per edge (P = waves_per_edge; each wave is one
-// workgroup, and the whole wave checks one waypoint at a time).  The check
-// sequence of an edge is valid(to) at position 0 (counted even when vouched
-// for, as the reference's validator counts it), then the DMV waypoints in
-// table order at positions 1..mw.  Wave p takes valid(to) (p = 0) and the
-// waypoints of rank p, p + P, ...; a failure lowers the edge's slot in
-// `checks` (set to ~0 beforehand) to its position with atomicMin, and a wave
-// stops when the slot is already below its next position.  The first
-// failing position lies in one wave's share, which that wave reaches, so the
-// slot ends at exactly the first failing position; no wave waits for
-// another.  Edges beyond 255 waypoints replay the 256-slot ring on wave 0
-// alone.  mesh_link_finish turns the slots into verdicts and check counts.
-__global__ __launch_bounds__(64) void mesh_link(SpaceArgs sp, MeshArgs m, double inv,
-                                                const uint8_t* __restrict__ table, const double* __restrict__ from,
-                                                const double* __restrict__ to, int64_t n, int known_valid,
-                                                const uint8_t* __restrict__ mask, int waves_per_edge,
-                                                uint32_t* __restrict__ slot) {
-    __shared__ int32_t stack[kStackSlots];
-    __shared__ uint64_t rmin[256], rmax[256];
-    __shared__ uint64_t emitted[64];
-    __shared__ int cnt_s;
-    // edge endpoints live in LDS (read back per waypoint) to keep them out of
-    // the registers the collision walk needs
-    __shared__ double ab_s[14];
-    volatile double* ab = ab_s;
-    const int lane = threadIdx.x;
-    const int64_t P = waves_per_edge;
-    auto current = [&](int64_t e) {  // the edge's slot, wave-uniform
-        return (uint32_t)__builtin_amdgcn_readfirstlane(
-            (int)__hip_atomic_load(&slot[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    };
-    for (int64_t item = blockIdx.x; item < n * P; item += gridDim.x) {
-        const int64_t e = item / P;
-        const int64_t p = item % P;
-        if (mask && !mask[e]) continue;
-        if (lane < 14) ab[lane] = lane < 7 ? from[e * 7 + lane] : to[e * 7 + lane - 7];
-        __syncthreads();
-        double a[7], b[7], q[7];
-        auto load_ab = [&]() {
+// DMV link (src/mpt/discrete_motion_validator.hpp:71-130) of n edges: one wave
+// checks one waypoint at a time.  The check sequence of an edge is valid(to)
+// at position 0 (counted even when vouched for, as the reference's validator
+// counts it), then the DMV waypoints in table order at positions 1..mw.
+//
+// mesh_link_prepare lists the live edges with their waypoint counts and sets
+// their slots in `checks` to ~0.  mesh_link deals (position, edge) items,
+// positions before edges, to its waves in turn; a wave tests 64 of its items
+// at once (not past the edge's last waypoint, nor past a position that has
+// failed already), each lane interpolates the pose of its own item, and the
+// wave checks those left one by one.  A failure lowers the edge's slot to its
+// position with atomicMin; every position below the final slot has been
+// checked, so it ends at exactly the first failing one.  No wave waits for
+// another.  mesh_link_finish turns the slots into verdicts and
+// check counts.
+//
+// Dealt this way a wave meets other edges from item to item.  When P waves
+// shared an edge's waypoints (2 of 8192 waves for 4096 edges), the waves of
+// the few long free edges checked up to a dozen waypoints in series while the
+// other waves had ended, and a larger P checked waypoints past failures; and
+// every lane of a wave computed the one pose, which was half of the registers.
+// 4096 edges, 15 600 waypoint checks against 50 000 triangles: 315 us before,
+// 197 now (312 with 32 waves dealt to each CU, 217 with 64).
+//
+// Edges beyond 255 waypoints replay the 256-slot ring on one wave, 64 indices
+// at a time.
+struct MeshWork {
+    uint32_t n_live, max_mw;  // zero between calls (mesh_link_finish clears them)
+};
+constexpr size_t kMeshWorkBytes = 256;
+
+__device__ __forceinline__ int64_t mesh_waypoints(const SpaceArgs& sp, const double* a, const double* b, double inv) {
+    const double x = __builtin_ceil(space_dist(sp, a, b) * inv);
+    int64_t steps = 0;
+    if (x >= 2.0) steps = x < 0x1.0p62 ? (int64_t)x : ((int64_t)1 << 62);
+    return steps > 0 ? steps - 1 : 0;
+}
+
+__global__ __launch_bounds__(256) void mesh_link_prepare(SpaceArgs sp, double inv, const double* __restrict__ from,
+                                                         const double* __restrict__ to, int64_t n,
+                                                         const uint8_t* __restrict__ mask, uint32_t* __restrict__ slot,
+                                                         MeshWork* __restrict__ work, uint2* __restrict__ live) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    int mw = -1;
+    if (e < n) {
+        slot[e] = 0xffffffffu;
+        if (!mask || mask[e]) {
+            double a[7], b[7];
 #pragma unroll
             for (int j = 0; j < 7; ++j) {
-                a[j] = ab[j];
-                b[j] = ab[7 + j];
+                a[j] = from[e * 7 + j];
+                b[j] = to[e * 7 + j];
             }
-        };
-        load_ab();
-        if (p == 0 && !known_valid && mesh_collides(m, b, stack)) {
-            if (lane == 0) atomicMin(&slot[e], 0u);
-            __syncthreads();
-            continue;
+            const int64_t w = mesh_waypoints(sp, a, b, inv);
+            if (w <= kMaxDmvWaypointsMesh) mw = (int)w;  // beyond: not checked, the finish kernel reports it
         }
-        load_ab();
-        double x = __builtin_ceil(space_dist(sp, a, b) * inv);
-        int64_t steps = 0;
-        if (x >= 2.0) steps = x < 0x1.0p62 ? (int64_t)x : ((int64_t)1 << 62);
-        const int64_t mw = steps > 0 ? steps - 1 : 0;
-        if (mw > kMaxDmvWaypointsMesh) {  // not checked; the finish kernel reports it
-            __syncthreads();
-            continue;
+    }
+    const uint64_t m = __ballot(mw >= 0);
+    if (m == 0) return;
+    int most = mw;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o));
+    uint32_t base = 0;
+    if (lane == 0) {
+        base = atomicAdd(&work->n_live, (uint32_t)__popcll(m));
+        atomicMax(&work->max_mw, (uint32_t)min(most, kTableMaxMesh));  // a ring edge is one item
+    }
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (mw >= 0) live[base + __popcll(m & ((1ull << lane) - 1ull))] = make_uint2((uint32_t)e, (uint32_t)mw);
+}
+
+// The next indices of an edge's 256-slot ring, in check order (lane 0).
+struct MeshRing {
+    uint64_t rmin[256], rmax[256], emitted[64];
+    uint64_t qs, qe, seq_cur, seq_end;
+    int seq, count, mw;
+
+    __device__ void start(int waypoints) {
+        mw = waypoints;
+        rmin[0] = 1;
+        rmax[0] = (uint64_t)waypoints;
+        qs = 0;
+        qe = 1;
+        seq = 0;
+    }
+    __device__ void emit() {
+        int c = 0;
+        while (c < 64 && (seq || qs != qe)) {
+            if (seq) {
+                emitted[c++] = seq_cur;
+                if (seq_cur == seq_end) seq = 0;
+                else ++seq_cur;
+                continue;
+            }
+            const uint64_t mn = rmin[qs % 256], mx = rmax[qs % 256];
+            ++qs;
+            if (mn == mx) {
+                emitted[c++] = mn;
+            } else if (qe + 2 < qs + 256) {
+                const uint64_t mid = (mn + mx) / 2;
+                emitted[c++] = mid;
+                if (mn < mid) {
+                    rmin[qe % 256] = mn;
+                    rmax[qe % 256] = mid - 1;
+                    ++qe;
+                }
+                if (mid < mx) {
+                    rmin[qe % 256] = mid + 1;
+                    rmax[qe % 256] = mx;
+                    ++qe;
+                }
+            } else {
+                seq = 1;
+                seq_cur = mn;
+                seq_end = mx;
+            }
         }
-        const double delta = steps > 0 ? 1.0 / (double)steps : 0.0;
-        if (mw <= kTableMaxMesh) {
-            const uint8_t* ord = table + (mw * (mw - 1)) / 2;
-            for (int64_t o = p; o < mw; o += P) {
-                const uint32_t pos = (uint32_t)(o + 1);
-                if (current(e) < pos) break;  // an earlier position already failed
-                load_ab();
-                space_interp(sp, a, b, (double)ord[o] * delta, q);
-                if (mesh_collides(m, q, stack)) {
-                    if (lane == 0) atomicMin(&slot[e], pos);
+        count = c;
+    }
+};
+
+__device__ __forceinline__ Pose32 lane_pose(const Pose32& p, int src) {
+    Pose32 o;
+    auto rl = [&](float v) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), src)); };
+#pragma unroll
+    for (int i = 0; i < 9; ++i) o.r[i] = rl(p.r[i]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) o.t[i] = rl(p.t[i]);
+    return o;
+}
+
+// Four waves per SIMD: 128 registers, none spilled (133 and three waves left
+// to itself; five spill 48 values).
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void mesh_link(
+    SpaceArgs sp, MeshArgs m, const uint8_t* __restrict__ table, const double* __restrict__ from,
+    const double* __restrict__ to, int known_valid, const MeshWork* __restrict__ work,
+    const uint2* __restrict__ live, uint32_t* __restrict__ slot) {
+    __shared__ int32_t stack[kStackSlots];
+    __shared__ MeshRing ring;
+    const int lane = threadIdx.x;
+    const uint32_t pos0 = known_valid ? 1u : 0u;  // the first position checked
+    uint64_t first = blockIdx.x;
+    // this lane's item of the batch: edge, waypoint count, position
+    uint32_t my_e = 0, my_pos = 0;
+    int my_mw = 0;
+    uint64_t rings = 0;  // the batch's items that are whole edges with a ring
+    bool in_ring = false;
+    uint32_t ring_e = 0, ring_at = 0;  // the edge in the ring, and its next position
+    while (true) {
+        // a batch of up to 64 positions, a lane each: `todo`
+        bool want = false;
+        uint32_t e = 0, pos = 0;
+        int mw = 0;
+        uint64_t index = 0;  // the waypoint, 0: valid(to)
+        if (in_ring) {
+            __syncthreads();  // the indices emitted last have been read
+            if (lane == 0) ring.emit();
+            __syncthreads();
+            const int c = ring.count;
+            if (c == 0) {
+                in_ring = false;
+                continue;
+            }
+            want = lane < c;
+            e = ring_e;
+            mw = ring.mw;
+            pos = ring_at + (uint32_t)lane;
+            index = want ? ring.emitted[lane] : 0;
+            ring_at += (uint32_t)c;
+        } else if (rings) {
+            const int src = __builtin_ctzll(rings);
+            rings &= rings - 1;
+            in_ring = true;
+            ring_e = (uint32_t)__builtin_amdgcn_readlane((int)my_e, src);
+            ring_at = 1;
+            __syncthreads();
+            if (lane == src) ring.start(my_mw);
+            __syncthreads();
+            if (known_valid) continue;
+            want = lane == 0;  // valid(to) first
+            e = ring_e;
+            mw = ring.mw;
+        } else {
+            const uint64_t n_live = work->n_live;
+            const uint64_t items = n_live * ((uint64_t)work->max_mw + 1u - pos0);
+            if (first >= items) break;
+            const uint64_t it = first + (uint64_t)lane * gridDim.x;
+            first += (uint64_t)gridDim.x * 64;
+            bool whole = false;
+            if (it < items) {
+                const uint64_t row = items < (1ull << 32) ? (uint64_t)((uint32_t)it / (uint32_t)n_live) : it / n_live;
+                const uint2 le = live[it - row * n_live];
+                my_e = le.x;
+                my_mw = (int)le.y;
+                my_pos = (uint32_t)row + pos0;
+                whole = my_mw > kTableMaxMesh && my_pos == pos0;
+                want = my_mw <= kTableMaxMesh && my_pos <= (uint32_t)my_mw && slot[my_e] >= my_pos;
+            }
+            rings = __ballot(whole);
+            e = my_e;
+            mw = my_mw;
+            pos = my_pos;
+            if (want && pos > 0) index = table[((int64_t)mw * (mw - 1)) / 2 + pos - 1];
+        }
+        Pose32 pose{};
+        if (want) {
+            double a[7], b[7], q[7];
+#pragma unroll
+            for (int j = 0; j < 7; ++j) {
+                a[j] = from[(int64_t)e * 7 + j];
+                b[j] = to[(int64_t)e * 7 + j];
+                q[j] = b[j];
+            }
+            if (index > 0) space_interp(sp, a, b, (double)index * (1.0 / (double)(mw + 1)), q);
+            pose = pose_from_state(q);
+        }
+        for (uint64_t todo = __ballot(want); todo; todo &= todo - 1) {  // wave-uniform, in position order
+            const int src = __builtin_ctzll(todo);
+            const uint32_t ee = (uint32_t)__builtin_amdgcn_readlane((int)e, src);
+            const uint32_t pp = (uint32_t)__builtin_amdgcn_readlane((int)pos, src);
+            // an earlier position has failed meanwhile
+            if ((uint32_t)__builtin_amdgcn_readfirstlane(
+                    (int)__hip_atomic_load(&slot[ee], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < pp)
+                continue;
+            if (mesh_collides(m, lane_pose(pose, src), stack)) {
+                if (lane == 0) atomicMin(&slot[ee], pp);
+                if (in_ring) {
+                    in_ring = false;
                     break;
                 }
             }
-        } else if (p == 0) {
-            // ring replay: lane 0 emits up to 64 indices at a time
-            bool failed = false;
-            int64_t done = 0;
-            uint64_t qs = 0, qe = 1, seq_cur = 0, seq_end = 0;
-            bool seq = false;
-            if (lane == 0) {
-                rmin[0] = 1;
-                rmax[0] = (uint64_t)mw;
-            }
-            while (!failed) {
-                if (lane == 0) {
-                    int c = 0;
-                    while (c < 64 && (seq || qs != qe)) {
-                        if (seq) {
-                            emitted[c++] = seq_cur;
-                            if (seq_cur == seq_end) seq = false;
-                            else ++seq_cur;
-                            continue;
-                        }
-                        const uint64_t mn = rmin[qs % 256], mx = rmax[qs % 256];
-                        ++qs;
-                        if (mn == mx) {
-                            emitted[c++] = mn;
-                        } else if (qe + 2 < qs + 256) {
-                            const uint64_t mid = (mn + mx) / 2;
-                            emitted[c++] = mid;
-                            if (mn < mid) {
-                                rmin[qe % 256] = mn;
-                                rmax[qe % 256] = mid - 1;
-                                ++qe;
-                            }
-                            if (mid < mx) {
-                                rmin[qe % 256] = mid + 1;
-                                rmax[qe % 256] = mx;
-                                ++qe;
-                            }
-                        } else {
-                            seq = true;
-                            seq_cur = mn;
-                            seq_end = mx;
-                        }
-                    }
-                    cnt_s = c;
-                }
-                __syncthreads();
-                const int c = cnt_s;
-                if (c == 0) break;
-                for (int o = 0; o < c; ++o) {
-                    load_ab();
-                    space_interp(sp, a, b, (double)emitted[o] * delta, q);
-                    ++done;
-                    if (mesh_collides(m, q, stack)) {
-                        failed = true;
-                        break;
-                    }
-                }
-                __syncthreads();
-            }
-            if (failed && lane == 0) atomicMin(&slot[e], (uint32_t)done);
         }
-        __syncthreads();
     }
 }
 
@@ -564,8 +658,10 @@ __global__ __launch_bounds__(64) void mesh_link(SpaceArgs sp, MeshArgs m, double
 __global__ __launch_bounds__(256) void mesh_link_finish(SpaceArgs sp, double inv, const double* __restrict__ from,
                                                         const double* __restrict__ to, int64_t n,
                                                         const uint8_t* __restrict__ mask,
-                                                        uint8_t* __restrict__ verdict, uint32_t* __restrict__ checks) {
+                                                        uint8_t* __restrict__ verdict, uint32_t* __restrict__ checks,
+                                                        MeshWork* __restrict__ work) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e == 0) work->n_live = work->max_mw = 0;
     if (e >= n || (mask && !mask[e])) return;
     const uint32_t s = checks[e];
     if (s != 0xffffffffu) {
@@ -579,10 +675,7 @@ __global__ __launch_bounds__(256) void mesh_link_finish(SpaceArgs sp, double inv
         a[j] = from[e * 7 + j];
         b[j] = to[e * 7 + j];
     }
-    const double x = __builtin_ceil(space_dist(sp, a, b) * inv);
-    int64_t steps = 0;
-    if (x >= 2.0) steps = x < 0x1.0p62 ? (int64_t)x : ((int64_t)1 << 62);
-    const int64_t mw = steps > 0 ? steps - 1 : 0;
+    const int64_t mw = mesh_waypoints(sp, a, b, inv);
     if (mw > kMaxDmvWaypointsMesh) {
         verdict[e] = 0;
         checks[e] = MPTG_CHECKS_OVER_LIMIT;
@@ -622,18 +715,27 @@ int launch_mesh_link(mptg_ctx* ctx, const uint8_t* d_table, const double* d_from
                      int known_valid, const uint8_t* d_mask, uint8_t* d_verdict, uint32_t* d_checks) {
     if (n <= 0) return MPTG_OK;
     int rc;
-    if ((rc = launch_fill_u32(ctx, d_checks, n, 0xffffffffu))) return rc;  // first-failure slots
-    // waves per edge: the tuned count, or more for a batch too small to fill
-    // the device (the rewire pass's late batches hold a few edges), up to 256
-    // (the verdicts and counts do not depend on it)
-    const int64_t fill = (int64_t)ctx->cus * ctx->tune.mesh_waves_per_cu;
-    const int P = (int)std::max<int64_t>(ctx->tune.mesh_edge_waves, std::min<int64_t>(256, fill / n));
-    const unsigned gp = (unsigned)std::min<int64_t>(n * P, fill);
-    hipLaunchKernelGGL(mesh_link, dim3(gp), dim3(64), 0, ctx->stream, space_args(ctx), mesh_args(ctx),
-                       1.0 / ctx->link_param, d_table, d_from, d_to, n, known_valid, d_mask, P, d_checks);
-    hipLaunchKernelGGL(mesh_link_finish, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, space_args(ctx),
-                       1.0 / ctx->link_param, d_from, d_to, n, d_mask, d_verdict, d_checks);
+    DevBuf& buf = ctx->scratch[10];
+    const size_t need = kMeshWorkBytes + sizeof(uint2) * (size_t)n;
+    if (!buf.p || buf.bytes < need) ctx->link_lists_clean = false;
+    if ((rc = ensure(ctx, buf, need))) return rc;
+    MeshWork* work = (MeshWork*)buf.p;
+    uint2* live = (uint2*)((char*)buf.p + kMeshWorkBytes);
+    if (!ctx->link_lists_clean && (rc = launch_zero_u32(ctx, (uint32_t*)work, kMeshWorkBytes / 4))) return rc;
+    ctx->link_lists_clean = false;  // until every kernel is enqueued
+    const unsigned g1 = (unsigned)((n + 255) / 256);
+    hipLaunchKernelGGL(mesh_link_prepare, dim3(g1), dim3(256), 0, ctx->stream, space_args(ctx), 1.0 / ctx->link_param,
+                       d_from, d_to, n, d_mask, d_checks, work, live);
+    // waves: as many as the device holds, or 256 per edge (every waypoint of
+    // a short edge at once) in a batch too small for that (the rewire pass's
+    // late batches hold a few edges)
+    const unsigned gp = (unsigned)std::min<int64_t>(n * 256, (int64_t)ctx->cus * ctx->tune.mesh_waves_per_cu);
+    hipLaunchKernelGGL(mesh_link, dim3(gp), dim3(64), 0, ctx->stream, space_args(ctx), mesh_args(ctx), d_table,
+                       d_from, d_to, known_valid, (const MeshWork*)work, (const uint2*)live, d_checks);
+    hipLaunchKernelGGL(mesh_link_finish, dim3(g1), dim3(256), 0, ctx->stream, space_args(ctx), 1.0 / ctx->link_param,
+                       d_from, d_to, n, d_mask, d_verdict, d_checks, work);
     MPTG_HIP(ctx, hipGetLastError());
+    ctx->link_lists_clean = true;
     return MPTG_OK;
 }
 

@@ -77,6 +77,35 @@ def test_mesh_link_parity(ctx_factory, se3):
     assert (oc > 256).sum() >= 20 and gv.sum() >= 10
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 700])
+@pytest.mark.parametrize("waves", [1, 128])
+def test_mesh_link_mixed_lengths_in_one_batch(ctx_factory, se3, n, waves):
+    """Zero-length, short, table-long and ring-long edges side by side in the
+    64-position batches of the link waves, for grids of few and many waves:
+    verdicts and first-failure check counts equal the oracle's."""
+    import dataclasses
+    _say("mesh link mixed", n, waves)
+    sparse = scenes.se3_scene(n_env_tris=1200, seed_env=7)
+    fine = dataclasses.replace(sparse, link_param=sparse.link_param / 6)
+    o = oracle.Oracle(fine)
+    rng = np.random.default_rng(43)
+    a = _states(rng, n)
+    b = _states(rng, n)  # ring: several hundred waypoints
+    near = a + 0.0
+    near[:, 4:] += rng.normal(0, 1.0, (n, 3))
+    b[0::4] = a[0::4]
+    b[1::4] = near[1::4]
+    b[2::4, :4] = a[2::4, :4]
+    b[2::4, 4:] = a[2::4, 4:] + rng.normal(0, 6.0, (len(b[2::4]), 3))
+    ctx = ctx_factory()
+    ctx.scene(fine)
+    ctx.tune_set(mesh_waves_per_cu=waves)
+    for kv in (False, True):
+        gv, gc = ctx.link(a, b, endpoints_known_valid=kv)
+        ov, oc = o.link(a, b, known_valid=kv, threads=8)
+        assert np.array_equal(gv, ov) and np.array_equal(gc, oc), kv
+
+
 def test_mesh_prrt_tree_parity(ctx_factory, se3):
     _say("mesh prrt")
     ctx = ctx_factory()
