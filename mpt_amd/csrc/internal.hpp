@@ -49,6 +49,7 @@ struct SceneDev {
     // mesh (SE(3) rigid body): env BVH nodes, env triangles, robot triangles
     DevBuf mesh_nodes, mesh_tris, mesh_robot;
     int mesh_nnodes = 0, mesh_nrobot = 0;
+    float mesh_reach = 0, mesh_env_reach = 0;  // largest coordinates in magnitude
     // shapes: circles [cx, cy, r^2, r]; the rectangles are `boxes`
     double* circles = nullptr;
     int ncircles = 0;
@@ -171,11 +172,11 @@ struct mptg_ctx {
     // graph is replayed only while the epoch it was captured at holds
     uint64_t epoch = 0;
     // launch shapes (mptg_autotune_*): kNN blocks per CU, waves per CU of the
-    // persistent DMV long-edge kernel and of the mesh kernels (32 -> 128:
+    // persistent DMV long-edge kernel and of the mesh kernels (64:
     // see mesh_link), two that the arm link and one that the mesh link no
     // longer reads, kNN select and grid paths, lanes per DMV edge, the byte
     // prefilter of the k = 1 L1 scan
-    mptg_tune_params tune{8, 16, 128, 2, 0, 2, 1, 1, 8, 1};
+    mptg_tune_params tune{8, 16, 64, 2, 0, 2, 1, 1, 8, 1};
     hipEvent_t phase_ev[6] = {};
 };
 

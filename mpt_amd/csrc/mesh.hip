@@ -9,20 +9,18 @@
 //
 // Layout in HBM (built on the host at upload):
 //   env BVH   binned-SAH binary tree (<= 4 triangles per leaf, depth <= 38)
-//             collapsed to MeshNode4[nnodes]: 128 B per node holding the
-//             boxes (by axis) and references of up to four nodes two levels
-//             below it, so one uniform load serves two levels of the walk
+//             collapsed to MeshNode16[nnodes]: 512 B per node holding the
+//             boxes and references of up to sixteen nodes four levels below
+//             it, 32 B each, so sixteen lanes read one node
 //   env tris  16 floats (64 B) per triangle in leaf order: v0 v1 v2, box lo, hi
-//   robot     9 floats per triangle, Morton-sorted by centroid so that the 4
-//             consecutive triangles a lane owns are close together
+//   robot     9 floats per triangle, Morton-sorted by centroid so that the
+//             consecutive triangles of a lane's group are close together;
+//             after them the groups' boxes (centre, half-sides)
 // Kernels (one 64-lane wave per block, one item per wave at a time):
 //   mesh_valid  one state per wave
 //   mesh_link   one waypoint of one edge per wave at a time (reference
 //               checks_done counts), nothing past an edge's first hit
-// Per state, lane l poses robot triangles [4l, 4l + 4) of each 256-triangle
-// chunk and takes their box; the wave walks the env BVH depth-first once with
-// one LDS stack, visiting a node when any lane's box overlaps it, and stops
-// at the first leaf where some lane finds a hit.
+// See mesh_collides for the check of one state.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -36,11 +34,8 @@ namespace mptg {
 
 namespace {
 
-constexpr int kLaneTris = 4;                    // robot triangles per lane
-constexpr int kChunkTris = 64 * kLaneTris;      // robot triangles per wave pass
+constexpr int kGroupShift = 3;                  // a lane's group: up to 2^3 robot triangles
 constexpr int kBuildDepth = 38;                 // BVH depth bound
-// LDS stack of a wave's walk: up to three (a, b) entries per four-wide level
-constexpr int kStackSlots = 2 * 3 * (kBuildDepth / 2 + 1);
 constexpr int kMaxDmvWaypointsMesh = 1 << 24;   // same limit as the other DMV kernels
 constexpr int kTableMaxMesh = 255;
 
@@ -163,76 +158,56 @@ int bvh_depth(const std::vector<MeshNode>& nodes, int n, int d) {
     return std::max(bvh_depth(nodes, nodes[n].a, d + 1), bvh_depth(nodes, nodes[n].b, d + 1));
 }
 
-// Four-wide node: slot k holds the box and reference of a binary node one or
-// two levels below (the children, with an internal child replaced by its two
-// children).  b[k] > 0: a[k] is a MeshNode4 index; b[k] <= 0: triangles
-// [a[k], a[k] - b[k]); an unused slot has an empty box (lo > hi).
-struct MeshNode4 {
-    float lo[3][4], hi[3][4];
-    int32_t a[4], b[4];
+// Sixteen-wide node: its slots hold the boxes and references of the binary
+// nodes four levels below (a leaf above that level takes one slot, and the
+// slots that such leaves leave free go to one more level of the first of the
+// others).  b > 0: a is a MeshNode16 index; b <= 0: triangles [a, a - b); an
+// unused slot has an empty box (lo > hi).
+constexpr int kWide = 16, kWideLevels = 4;
+struct MeshSlot {
+    float lo[3];
+    int32_t a;
+    float hi[3];
+    int32_t b;
 };
-static_assert(sizeof(MeshNode4) == 128, "four-wide node is 128 bytes");
+struct MeshNode16 {
+    MeshSlot slot[kWide];
+};
+static_assert(sizeof(MeshNode16) == 512, "sixteen-wide node is 512 bytes");
 
-// Collapse the binary subtree under internal node id into out (pre-order).
-int collapse4(const std::vector<MeshNode>& n2, int id, std::vector<MeshNode4>& out) {
+// Collapse the binary subtree under id (an internal node, or a leaf root) into
+// out (pre-order).
+int collapse16(const std::vector<MeshNode>& n2, int id, std::vector<MeshNode16>& out) {
     const int me = (int)out.size();
-    out.push_back(MeshNode4{});
-    int slot[4], ns = 0;
-    for (const int c : {n2[id].a, n2[id].b}) {
-        if (n2[c].b > 0) {
-            slot[ns++] = n2[c].a;
-            slot[ns++] = n2[c].b;
-        } else {
-            slot[ns++] = c;
+    out.push_back(MeshNode16{});
+    std::vector<int> slot{id};
+    for (int level = 0; level <= kWideLevels; ++level) {  // the last one as far as there is room
+        const std::vector<int> above = slot;
+        slot.clear();
+        for (size_t i = 0; i < above.size(); ++i) {
+            const MeshNode& g = n2[above[i]];
+            if (g.b > 0 && slot.size() + (above.size() - i) < (size_t)kWide) {
+                slot.push_back(g.a);
+                slot.push_back(g.b);
+            } else {
+                slot.push_back(above[i]);
+            }
         }
     }
-    MeshNode4 node;
-    for (int k = 0; k < 4; ++k) {
-        for (int i = 0; i < 3; ++i) {
-            node.lo[i][k] = INFINITY;
-            node.hi[i][k] = -INFINITY;
-        }
-        node.a[k] = 0;
-        node.b[k] = 0;
-    }
-    for (int k = 0; k < ns; ++k) {
+    MeshNode16 node;
+    for (MeshSlot& o : node.slot) o = {{INFINITY, INFINITY, INFINITY}, 0, {-INFINITY, -INFINITY, -INFINITY}, 0};
+    for (size_t k = 0; k < slot.size(); ++k) {
         const MeshNode& g = n2[slot[k]];
+        MeshSlot& o = node.slot[k];
         for (int i = 0; i < 3; ++i) {
-            node.lo[i][k] = g.lo[i];
-            node.hi[i][k] = g.hi[i];
+            o.lo[i] = g.lo[i];
+            o.hi[i] = g.hi[i];
         }
-        if (g.b > 0) {
-            node.a[k] = collapse4(n2, slot[k], out);
-            node.b[k] = 1;
-        } else {
-            node.a[k] = g.a;
-            node.b[k] = g.b;
-        }
+        o.a = g.b > 0 ? collapse16(n2, slot[k], out) : g.a;
+        o.b = g.b > 0 ? 1 : g.b;
     }
     out[(size_t)me] = node;
     return me;
-}
-
-// The four-wide tree of a binary BVH (root first); a leaf root becomes one
-// node with a single slot.
-std::vector<MeshNode4> collapse_bvh(const std::vector<MeshNode>& n2) {
-    std::vector<MeshNode4> out;
-    if (n2.empty()) return out;
-    if (n2[0].b > 0) {
-        collapse4(n2, 0, out);
-        return out;
-    }
-    MeshNode4 node;
-    for (int k = 0; k < 4; ++k) {
-        for (int i = 0; i < 3; ++i) {
-            node.lo[i][k] = k == 0 ? n2[0].lo[i] : INFINITY;
-            node.hi[i][k] = k == 0 ? n2[0].hi[i] : -INFINITY;
-        }
-        node.a[k] = k == 0 ? n2[0].a : 0;
-        node.b[k] = k == 0 ? n2[0].b : 0;
-    }
-    out.push_back(node);
-    return out;
 }
 
 uint32_t spread10(uint32_t v) {
@@ -248,142 +223,300 @@ uint32_t spread10(uint32_t v) {
 // device
 // ---------------------------------------------------------------------------
 struct MeshArgs {
-    const MeshNode4* nodes;
-    const float4* tris;   // 4 float4 per triangle
-    const float* robot;   // 9 floats per triangle
+    const float4* slots;   // 16 slots of 2 float4 per node
+    const float4* tris;    // 4 float4 per triangle
+    const float* robot;    // 9 floats per triangle
+    const float4* groups;  // 2 float4 per group: centre, half-sides
     int nnodes, nrobot;
+    int shift;    // a group is 2^shift robot triangles
+    float reach, env_reach;  // largest coordinate in magnitude
 };
 
-// The scene's BVH nodes are written only at upload, so the walk reads them
-// through the constant address space: its wave-uniform node loads then become
-// scalar loads also in kernels that store elsewhere (mesh_link).
-template <typename T>
-__device__ __forceinline__ const __attribute__((address_space(4))) T* scene_const(const T* p) {
-    return (const __attribute__((address_space(4))) T*)p;
+// Below this magnitude no coordinate's products overflow: an axis from a
+// normal is at most 2^5 kTameReach^3, its dot product 2^7 kTameReach^4.
+constexpr float kTameReach = 0x1p29f;
+
+// One wave's work lists in a check: BVH nodes to open, leaves met, (lane's
+// group, environment triangle) pairs and (robot triangle, environment
+// triangle) pairs whose boxes overlap.
+constexpr int kOpenNodes = 64 / kWide;  // nodes opened at a time, sixteen lanes each
+constexpr int kStackSoft = 64;          // above it one node at a time
+struct MeshLists {
+    // kStackSoft + 60 after the last step of several nodes, and then fifteen
+    // more per level of a depth-first descent
+    int32_t stack[kStackSoft + 60 + (kWide - 1) * (kBuildDepth / kWideLevels + 2)];
+    uint32_t leaf[128];  // first triangle | (count - 1) << 20
+    uint32_t pair[128];  // lane | environment triangle << 6
+    uint32_t sat[128];   // robot triangle of the chunk | environment triangle << 9
+};
+
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_or_self(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(
+        (int)__float_as_uint(v), (int)__float_as_uint(v), CTRL, ROWS, 0xf, false));
+}
+// Minimum over the wave (no NaN), the same on every lane.
+__device__ __forceinline__ float wave_min_f32(float v) {
+    v = __builtin_fminf(v, dpp_or_self<0x128, 0xf>(v));  // rows of 16: rotate by 8, 4, 2, 1
+    v = __builtin_fminf(v, dpp_or_self<0x124, 0xf>(v));
+    v = __builtin_fminf(v, dpp_or_self<0x122, 0xf>(v));
+    v = __builtin_fminf(v, dpp_or_self<0x121, 0xf>(v));
+    v = __builtin_fminf(v, dpp_or_self<0x142, 0xa>(v));  // lane 15 to row 1, 47 to row 3
+    v = __builtin_fminf(v, dpp_or_self<0x143, 0xc>(v));  // lane 31 to rows 2 and 3
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
 }
 
-// Four-wide node i, word by word (lo[3][4], hi[3][4], a[4], b[4]).
-__device__ __forceinline__ MeshNode4 load_node4(const MeshNode4* nodes, int i) {
-    const __attribute__((address_space(4))) uint32_t* w = scene_const((const uint32_t*)nodes) + 32 * (size_t)i;
-    MeshNode4 n;
+__device__ __forceinline__ float lane_f32(float v, int src) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), src));
+}
+
+// Slots of the lanes with `want` in a list that holds `at` entries; `at` grows.
+__device__ __forceinline__ int take_slot(bool want, int& at) {
+    const uint64_t b = __ballot(want);
+    const int mine = at + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0));
+    at += __popcll(b);
+    return mine;
+}
+
+__device__ __forceinline__ void load_posed(const MeshArgs& m, const Pose32& pose, int i, float* tri) {
+    const float* src = m.robot + (size_t)i * 9;
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            n.lo[k][j] = __uint_as_float(w[4 * k + j]);
-            n.hi[k][j] = __uint_as_float(w[12 + 4 * k + j]);
-        }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        n.a[j] = (int32_t)w[24 + j];
-        n.b[j] = (int32_t)w[28 + j];
+    for (int v = 0; v < 3; ++v) xform(pose, src + 3 * v, tri + 3 * v);
+}
+
+// Box of robot triangles [first, first + cnt) as posed, vertex by vertex.
+__device__ __forceinline__ void posed_box(const MeshArgs& m, const Pose32& pose, int first, int cnt, float* lo, float* hi) {
+    for (int i = 0; i < 3; ++i) {
+        lo[i] = INFINITY;
+        hi[i] = -INFINITY;
     }
-    return n;
+#pragma unroll 1
+    for (int t = 0; t < cnt; ++t) {
+        float tri[9], tlo[3], thi[3];
+        load_posed(m, pose, first + t, tri);
+        tri_box(tri, tlo, thi);
+        for (int i = 0; i < 3; ++i) {
+            lo[i] = tlo[i] < lo[i] ? tlo[i] : lo[i];
+            hi[i] = thi[i] > hi[i] ? thi[i] : hi[i];
+        }
+    }
 }
 
-// Triangle record i (16 floats: v0 v1 v2, box lo, box hi, one unused),
-// vector loads: as scalar loads the leaf tests ran slower in mesh_filter.
-__device__ __forceinline__ void load_env_tri(const float4* __restrict__ t, int i, float* v, float* lo, float* hi) {
-    const float4 a = t[4 * i], b = t[4 * i + 1], c = t[4 * i + 2], d = t[4 * i + 3];
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    v[8] = c.x;
-    lo[0] = c.y; lo[1] = c.z; lo[2] = c.w;
-    hi[0] = d.x; hi[1] = d.y; hi[2] = d.z;
+// tri_tri_overlap without its early returns: some lane of 64 pairs nearly
+// always needs the last axis, and seventeen nested exits hold as many masks.
+// For coordinates whose products cannot overflow there is no NaN, and the
+// minima and maxima are single instructions.
+__device__ __forceinline__ int apart_on_tame(const float* ax, const float* p, const float* q) {
+    const float p0 = dot3(ax, p), p1 = dot3(ax, p + 3), p2 = dot3(ax, p + 6);
+    const float q0 = dot3(ax, q), q1 = dot3(ax, q + 3), q2 = dot3(ax, q + 6);
+    const float pmax = __builtin_fmaxf(__builtin_fmaxf(p0, p1), p2), pmin = __builtin_fminf(__builtin_fminf(p0, p1), p2);
+    const float qmax = __builtin_fmaxf(__builtin_fmaxf(q0, q1), q2), qmin = __builtin_fminf(__builtin_fminf(q0, q1), q2);
+    return (int)(pmax < qmin) | (int)(qmax < pmin);
+}
+__device__ __forceinline__ bool tri_tri_overlap_wave(const float* p, const float* q, bool tame) {
+    float ep[3][3], eq[3][3], np[3], nq[3], ax[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        sub3(p + 3 * ((i + 1) % 3), p + 3 * i, ep[i]);
+        sub3(q + 3 * ((i + 1) % 3), q + 3 * i, eq[i]);
+    }
+    cross3(ep[0], ep[1], np);
+    cross3(eq[0], eq[1], nq);
+    if (!tame) {
+        // any coordinates: axis by axis in a loop, to hold few registers
+        int apart = (int)apart_on(np, p, q) | (int)apart_on(nq, p, q);
+#pragma unroll 1
+        for (int k = 0; k < 15; ++k) {
+            const int i = k / 5, j = k % 5;
+            float u[3], v[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const float epi = i == 0 ? ep[0][c] : i == 1 ? ep[1][c] : ep[2][c];
+                const float eqi = i == 0 ? eq[0][c] : i == 1 ? eq[1][c] : eq[2][c];
+                const float eqj = j == 0 ? eq[0][c] : j == 1 ? eq[1][c] : eq[2][c];
+                u[c] = j < 3 ? epi : j == 3 ? np[c] : nq[c];
+                v[c] = j < 3 ? eqj : j == 3 ? epi : eqi;
+            }
+            cross3(u, v, ax);
+            apart |= (int)apart_on(ax, p, q);
+        }
+        return !apart;
+    }
+    int apart = apart_on_tame(np, p, q) | apart_on_tame(nq, p, q);
+    if (__ballot(!apart) == 0) return false;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            cross3(ep[i], eq[j], ax);
+            apart |= apart_on_tame(ax, p, q);
+        }
+        cross3(np, ep[i], ax);
+        apart |= apart_on_tame(ax, p, q);
+        cross3(nq, eq[i], ax);
+        apart |= apart_on_tame(ax, p, q);
+    }
+    return !apart;
 }
 
 // Does the robot at `pose` collide with the environment?  Whole wave; the
-// pose is the same on every lane.  stack: this wave's kStackSlots LDS slots.
+// pose is the same on every lane.
 //
-// Per 256-triangle chunk, lane l poses robot triangles [4l, 4l + 4) and takes
-// their box; the wave walks the environment BVH depth-first once, visiting a
-// node when any lane's box overlaps it (a ballot), so node and triangle loads
-// are wave-uniform and no lane diverges in the walk.  At a leaf each lane
-// whose box overlaps it tests its triangles against the leaf's: a pair is
-// tested only when the boxes overlap, as the predicate requires, and a lane
-// whose box overlaps a leaf overlaps every ancestor of it, so the pairs
-// tested are those a per-lane walk would test.
-__device__ bool mesh_collides(const MeshArgs& m, const Pose32& pose, int32_t* stack) {
+// A lane owns a group of 2^shift robot triangles and takes a box around it:
+// the group's own box moved by the pose (centre R c + t, half-sides |R| h),
+// wide enough for every rounding here and in the posed vertices.  Per chunk of
+// 64 groups the wave opens BVH nodes that meet the box of them all, four nodes
+// at a time, a slot a lane; keeps the environment triangles of the
+// leaves that meet it, a triangle a lane; pairs each of those with the groups
+// whose boxes it meets; tests the boxes of the pairs' triangles, a triangle a
+// lane, which is the predicate's own test; and gives the pairs left to the
+// separating-axis test, 64 at a time.  Each of the lists passes its entries on
+// when it holds a wave's worth, and in the end.
+//
+// Bounds: instruction issue (1 600 vector and 1 050 scalar instructions per
+// counted check, 500 robot triangles among 50 000) and, for half of a wave's
+// time, the latency of dependent loads; sixteen-wide nodes make four or five
+// of them on the way to a leaf, four-wide ones took nine (142 -> 126 us for
+// the 4096 edges of mesh_link).  One four-wide node at a time, depth first,
+// with scalar loads and a ballot per slot over the lanes' boxes, took 75 nodes,
+// 3 300 vector and 2 400 scalar instructions per check (197 us), where 13
+// environment triangles lie in the robot's box.
+__device__ bool mesh_collides(const MeshArgs& m, const Pose32& pose, MeshLists& w) {
     const int lane = threadIdx.x & 63;
     if (m.nnodes == 0 || m.nrobot == 0) return false;
-    for (int c0 = 0; c0 < m.nrobot; c0 += kChunkTris) {
-        const int first = c0 + lane * kLaneTris;
-        const int cnt = max(0, min(kLaneTris, m.nrobot - first));
-        // box of this lane's posed triangles; the triangles themselves are
-        // posed again only for environment triangles inside this box
+    const int sh = m.shift;
+    const int per = 64 >> sh;  // pairs whose triangles fill the wave
+    for (int c0 = 0; c0 < m.nrobot; c0 += 64 << sh) {
+        const int first = c0 + (lane << sh);
+        const int cnt = max(0, min(1 << sh, m.nrobot - first));
         float llo[3] = {INFINITY, INFINITY, INFINITY}, lhi[3] = {-INFINITY, -INFINITY, -INFINITY};
-#pragma unroll 1
-        for (int t = 0; t < cnt; ++t) {
-            const float* src = m.robot + (size_t)(first + t) * 9;
-            float tri[9];
-#pragma unroll
-            for (int v = 0; v < 3; ++v) xform(pose, src + 3 * v, tri + 3 * v);
-            float tlo[3], thi[3];
-            tri_box(tri, tlo, thi);
+        bool odd = false;
+        if (cnt > 0) {
+            const float4 c = m.groups[2 * (first >> sh)], h = m.groups[2 * (first >> sh) + 1];
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
-                llo[i] = tlo[i] < llo[i] ? tlo[i] : llo[i];
-                lhi[i] = thi[i] > lhi[i] ? thi[i] : lhi[i];
+                const float r0 = pose.r[3 * i], r1 = pose.r[3 * i + 1], r2 = pose.r[3 * i + 2], t = pose.t[i];
+                const float a0 = __builtin_fabsf(r0), a1 = __builtin_fabsf(r1), a2 = __builtin_fabsf(r2);
+                const float mid = __builtin_fmaf(r0, c.x, __builtin_fmaf(r1, c.y, __builtin_fmaf(r2, c.z, t)));
+                // 32 roundings of the largest magnitude on the way: the sums
+                // here and in a posed vertex take 15 between them
+                const float slop = 0x1p-19f * (__builtin_fmaf(a0 + a1 + a2, m.reach, __builtin_fabsf(t)) + 0x1p-100f);
+                const float half =
+                    __builtin_fmaf(a0, h.x, __builtin_fmaf(a1, h.y, __builtin_fmaf(a2, h.z, slop)));
+                llo[i] = mid - half;
+                lhi[i] = mid + half;
+                odd |= !(__builtin_isfinite(llo[i]) && __builtin_isfinite(lhi[i]));
             }
         }
-        const bool live = cnt > 0;
-        // Current entry (ca, cb): a four-wide node (cb > 0) or a leaf's
-        // triangles [ca, ca - cb); an entry is entered only when some lane's
-        // box overlaps its box.  The four slot boxes of a node arrive in one
-        // uniform load; the wave descends into the first slot that some lane
-        // overlaps and keeps the other such slots on the stack.
-        int ca = 0, cb = 1;
-        int sp = 0;  // wave-uniform; at most 3 entries per four-wide level
+        if (__ballot(odd)) posed_box(m, pose, first, cnt, llo, lhi);  // a pose without finite bounds
+        float blo[3], bhi[3];
+        bool tame = m.env_reach < kTameReach;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            blo[i] = wave_min_f32(llo[i]);
+            bhi[i] = -wave_min_f32(-lhi[i]);
+            tame = tame && blo[i] > -kTameReach && bhi[i] < kTameReach;
+        }
+        int nopen = 1, nleaf = 0, npair = 0, nsat = 0;  // wave-uniform
+        if (lane == 0) w.stack[0] = 0;
+        int et = 0;  // this lane's environment triangle and its box; `tris`: the lanes that have one
+        float elo[3] = {}, ehi[3] = {};
+        uint64_t tris = 0;
         for (;;) {
-            if (cb > 0) {
-                const MeshNode4 N = load_node4(m.nodes, ca);
-                uint32_t take = 0;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float blo[3] = {N.lo[0][k], N.lo[1][k], N.lo[2][k]};
-                    const float bhi[3] = {N.hi[0][k], N.hi[1][k], N.hi[2][k]};
-                    take |= __ballot(live && boxes_overlap(blo, bhi, llo, lhi)) != 0 ? 1u << k : 0u;
-                }
-                if (take != 0) {
-#pragma unroll
-                    for (int k = 3; k >= 1; --k) {
-                        // every slot taken but the first goes on the stack
-                        if (((take >> k) & 1u) && (take & ((1u << k) - 1u))) {
-                            stack[2 * sp] = N.a[k];
-                            stack[2 * sp + 1] = N.b[k];
-                            ++sp;
-                        }
-                    }
-                    const int f = __builtin_ctz(take);
-                    ca = f == 0 ? N.a[0] : f == 1 ? N.a[1] : f == 2 ? N.a[2] : N.a[3];
-                    cb = f == 0 ? N.b[0] : f == 1 ? N.b[1] : f == 2 ? N.b[2] : N.b[3];
-                    continue;
-                }
-            } else {
-                // a lane meets a triangle's box only if it meets the leaf's
-                // and every ancestor's, so these pairs are the per-lane walk's
+            __syncthreads();
+            const bool found = nopen == 0 && nleaf == 0 && tris == 0;  // no more pairs to come
+            if (nsat >= 64 || (nsat > 0 && found && npair == 0)) {
+                const int n = min(nsat, 64);
                 bool hit = false;
-#pragma unroll 1
-                for (int i = ca; i < ca - cb; ++i) {  // wave-uniform bounds
-                    float ev[9], elo[3], ehi[3];
-                    load_env_tri(m.tris, i, ev, elo, ehi);
-                    if (!live || hit || !boxes_overlap(elo, ehi, llo, lhi)) continue;
-#pragma unroll 1
-                    for (int t = 0; t < cnt && !hit; ++t) {
-                        const float* src = m.robot + (size_t)(first + t) * 9;
-                        float tri[9], tlo[3], thi[3];
-#pragma unroll
-                        for (int v = 0; v < 3; ++v) xform(pose, src + 3 * v, tri + 3 * v);
-                        tri_box(tri, tlo, thi);
-                        hit = pair_collides(tri, tlo, thi, ev, elo, ehi);
-                    }
+                if (lane < n) {
+                    const uint32_t e = w.sat[nsat - 1 - lane];
+                    float tri[9], ev[9];
+                    load_posed(m, pose, c0 + (int)(e & 511u), tri);
+                    const float4* src = m.tris + 4 * (size_t)(e >> 9);
+                    const float4 a = src[0], b = src[1];
+                    ev[0] = a.x; ev[1] = a.y; ev[2] = a.z; ev[3] = a.w;
+                    ev[4] = b.x; ev[5] = b.y; ev[6] = b.z; ev[7] = b.w;
+                    ev[8] = src[2].x;
+                    hit = tri_tri_overlap_wave(tri, ev, tame);
                 }
                 if (__ballot(hit)) return true;
+                nsat -= n;
+            } else if (npair >= per || (npair > 0 && found)) {
+                const int n = min(npair, per);
+                const int p = lane >> sh;
+                bool meet = false;
+                uint32_t e = 0;
+                int t = 0;
+                if (p < n) {
+                    e = w.pair[npair - 1 - p];
+                    t = (int)((e & 63u) << sh) + (lane & ((1 << sh) - 1));
+                    if (c0 + t < m.nrobot) {
+                        float tri[9], tlo[3], thi[3];
+                        load_posed(m, pose, c0 + t, tri);
+                        tri_box(tri, tlo, thi);
+                        const float4* src = m.tris + 4 * (size_t)(e >> 6);
+                        const float4 c = src[2], d = src[3];
+                        const float blo_e[3] = {c.y, c.z, c.w}, bhi_e[3] = {d.x, d.y, d.z};
+                        meet = boxes_overlap(tlo, thi, blo_e, bhi_e);
+                    }
+                }
+                npair -= n;
+                const int at = take_slot(meet, nsat);
+                if (meet) w.sat[at] = (uint32_t)t | (e >> 6) << 9;
+            } else if (tris) {
+                do {
+                    const int src = __builtin_ctzll(tris);
+                    tris &= tris - 1;
+                    const float tlo[3] = {lane_f32(elo[0], src), lane_f32(elo[1], src), lane_f32(elo[2], src)};
+                    const float thi[3] = {lane_f32(ehi[0], src), lane_f32(ehi[1], src), lane_f32(ehi[2], src)};
+                    const bool meet = boxes_overlap(tlo, thi, llo, lhi);
+                    const uint32_t tri = (uint32_t)__builtin_amdgcn_readlane(et, src);
+                    const int at = take_slot(meet, npair);
+                    if (meet) w.pair[at] = (uint32_t)lane | tri << 6;
+                } while (tris && npair < per);
+            } else if (nleaf > 64 || (nleaf > 0 && nopen == 0)) {
+                const int n = min(nleaf, 16);
+                bool meet = false;
+                if ((lane >> 2) < n) {
+                    const uint32_t e = w.leaf[nleaf - 1 - (lane >> 2)];
+                    if ((uint32_t)(lane & 3) <= e >> 20) {
+                        et = (int)(e & 0xfffffu) + (lane & 3);
+                        const float4 c = m.tris[4 * (size_t)et + 2], d = m.tris[4 * (size_t)et + 3];
+                        elo[0] = c.y; elo[1] = c.z; elo[2] = c.w;
+                        ehi[0] = d.x; ehi[1] = d.y; ehi[2] = d.z;
+                        meet = boxes_overlap(elo, ehi, blo, bhi);
+                    }
+                }
+                nleaf -= n;
+                tris = __ballot(meet);
+            } else if (nopen > 0) {
+                do {
+                    const int n = nopen > kStackSoft ? 1 : min(nopen, kOpenNodes);
+                    bool inner = false, leaf = false;
+                    int a = 0, b = 0;
+                    const int o = lane / kWide;
+                    if (o < n) {
+                        const float4* src =
+                            m.slots + 2 * (kWide * (size_t)w.stack[nopen - 1 - o] + (lane & (kWide - 1)));
+                        const float4 lo = src[0], hi = src[1];
+                        a = (int)__float_as_uint(lo.w);
+                        b = (int)__float_as_uint(hi.w);
+                        const float slo[3] = {lo.x, lo.y, lo.z}, shi[3] = {hi.x, hi.y, hi.z};
+                        const bool meet = boxes_overlap(slo, shi, blo, bhi);
+                        inner = meet && b > 0;
+                        leaf = meet && b < 0;
+                    }
+                    __syncthreads();  // the entries are read before new ones take their places
+                    nopen -= n;
+                    const int at = take_slot(inner, nopen);
+                    if (inner) w.stack[at] = a;
+                    const int al = take_slot(leaf, nleaf);
+                    if (leaf) w.leaf[al] = (uint32_t)a | (uint32_t)(-b - 1) << 20;
+                    __syncthreads();
+                } while (nopen > 0 && nleaf <= 64);
+            } else {
+                break;
             }
-            if (sp == 0) break;
-            --sp;
-            ca = __builtin_amdgcn_readfirstlane(stack[2 * sp]);
-            cb = __builtin_amdgcn_readfirstlane(stack[2 * sp + 1]);
         }
     }
     return false;
@@ -391,12 +524,12 @@ __device__ bool mesh_collides(const MeshArgs& m, const Pose32& pose, int32_t* st
 
 __global__ __launch_bounds__(64) void mesh_valid(MeshArgs m, const double* __restrict__ q, int64_t n,
                                                  uint8_t* __restrict__ ok) {
-    __shared__ int32_t stack[kStackSlots];
+    __shared__ MeshLists lists;
     for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
         double s[7];
 #pragma unroll
         for (int j = 0; j < 7; ++j) s[j] = q[i * 7 + j];
-        const bool hit = mesh_collides(m, pose_from_state(s), stack);
+        const bool hit = mesh_collides(m, pose_from_state(s), lists);
         if (threadIdx.x == 0) ok[i] = hit ? 0 : 1;
     }
 }
@@ -404,13 +537,13 @@ __global__ __launch_bounds__(64) void mesh_valid(MeshArgs m, const double* __res
 __global__ __launch_bounds__(64) void mesh_filter(MeshArgs m, const double* __restrict__ q, int64_t n,
                                                   uint8_t* __restrict__ mask, uint8_t* __restrict__ status,
                                                   int invalid_code) {
-    __shared__ int32_t stack[kStackSlots];
+    __shared__ MeshLists lists;
     for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
         if (!mask[i]) continue;
         double s[7];
 #pragma unroll
         for (int j = 0; j < 7; ++j) s[j] = q[i * 7 + j];
-        const bool hit = mesh_collides(m, pose_from_state(s), stack);
+        const bool hit = mesh_collides(m, pose_from_state(s), lists);
         if (threadIdx.x == 0 && hit) {
             mask[i] = 0;
             status[i] = (uint8_t)invalid_code;
@@ -439,8 +572,11 @@ __global__ __launch_bounds__(64) void mesh_filter(MeshArgs m, const double* __re
 // the few long free edges checked up to a dozen waypoints in series while the
 // other waves had ended, and a larger P checked waypoints past failures; and
 // every lane of a wave computed the one pose, which was half of the registers.
-// 4096 edges, 15 600 waypoint checks against 50 000 triangles: 315 us before,
-// 197 now (312 with 32 waves dealt to each CU, 217 with 64).
+// 4096 edges, 19 700 counted checks against 50 000 triangles: 315 us that way,
+// 197 dealt out, 111 with the present mesh_collides (64 waves dealt to each CU:
+// 128, 111 and 123 us for 32, 64 and 128).  Storing the poses in the prepare
+// kernel instead took no less (its atomics, one wave per four edges, were as
+// long as the interpolation).
 //
 // Edges beyond 255 waypoints replay the 256-slot ring on one wave, 64 indices
 // at a time.
@@ -542,21 +678,19 @@ struct MeshRing {
 
 __device__ __forceinline__ Pose32 lane_pose(const Pose32& p, int src) {
     Pose32 o;
-    auto rl = [&](float v) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), src)); };
 #pragma unroll
-    for (int i = 0; i < 9; ++i) o.r[i] = rl(p.r[i]);
+    for (int i = 0; i < 9; ++i) o.r[i] = lane_f32(p.r[i], src);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) o.t[i] = rl(p.t[i]);
+    for (int i = 0; i < 3; ++i) o.t[i] = lane_f32(p.t[i], src);
     return o;
 }
 
-// Four waves per SIMD: 128 registers, none spilled (133 and three waves left
-// to itself; five spill 48 values).
+// Four waves per SIMD: 127 registers, none spilled (five waves spill 32).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void mesh_link(
     SpaceArgs sp, MeshArgs m, const uint8_t* __restrict__ table, const double* __restrict__ from,
     const double* __restrict__ to, int known_valid, const MeshWork* __restrict__ work,
     const uint2* __restrict__ live, uint32_t* __restrict__ slot) {
-    __shared__ int32_t stack[kStackSlots];
+    __shared__ MeshLists lists;
     __shared__ MeshRing ring;
     const int lane = threadIdx.x;
     const uint32_t pos0 = known_valid ? 1u : 0u;  // the first position checked
@@ -643,7 +777,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void me
             if ((uint32_t)__builtin_amdgcn_readfirstlane(
                     (int)__hip_atomic_load(&slot[ee], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < pp)
                 continue;
-            if (mesh_collides(m, lane_pose(pose, src), stack)) {
+            if (mesh_collides(m, lane_pose(pose, src), lists)) {
                 if (lane == 0) atomicMin(&slot[ee], pp);
                 if (in_ring) {
                     in_ring = false;
@@ -687,10 +821,21 @@ __global__ __launch_bounds__(256) void mesh_link_finish(SpaceArgs sp, double inv
 
 }  // namespace
 
+// Triangles of a lane's group: as few as give every lane a group, and at most
+// eight (their box is then that of the best part of a box of the robot's).
+static int group_shift(int nrobot) {
+    int sh = 0;
+    while (sh < kGroupShift && (64 << sh) < nrobot) ++sh;
+    return sh;
+}
+// The groups' boxes follow the robot's triangles, 16-byte aligned (floats).
+static size_t group_offset(int nrobot) { return ((size_t)nrobot * 9 + 3) / 4 * 4; }
+
 MeshArgs mesh_args(const mptg_ctx* ctx) {
     const SceneDev& s = ctx->scene;
-    return MeshArgs{(const MeshNode4*)s.mesh_nodes.p, (const float4*)s.mesh_tris.p, (const float*)s.mesh_robot.p,
-                    s.mesh_nnodes, s.mesh_nrobot};
+    return MeshArgs{(const float4*)s.mesh_nodes.p, (const float4*)s.mesh_tris.p,
+                    (const float*)s.mesh_robot.p,  (const float4*)((const float*)s.mesh_robot.p + group_offset(s.mesh_nrobot)),
+                    s.mesh_nnodes, s.mesh_nrobot, group_shift(s.mesh_nrobot), s.mesh_reach, s.mesh_env_reach};
 }
 
 int launch_mesh_valid(mptg_ctx* ctx, const double* d_q, int64_t n, uint8_t* d_ok) {
@@ -804,21 +949,46 @@ extern "C" int mptg_scene_mesh(mptg_ctx* ctx, const float* h_robot, int nrobot, 
         for (int t = 0; t < nrobot; ++t)
             std::memcpy(&robot[(size_t)t * 9], h_robot + (size_t)key[(size_t)t].second * 9, 9 * sizeof(float));
     }
+    // the groups' boxes, 8 floats each
+    const int sh = group_shift(nrobot);
+    const int ngroup = (nrobot + (1 << sh) - 1) >> sh;
+    robot.resize(group_offset(nrobot) + 8 * (size_t)ngroup, 0.0f);
+    float reach = 0.0f;
+    for (int g = 0; g < ngroup; ++g) {
+        const int t1 = std::min(nrobot, (g + 1) << sh);
+        float* o = &robot[group_offset(nrobot) + 8 * (size_t)g];
+        for (int i = 0; i < 3; ++i) {
+            float lo = INFINITY, hi = -INFINITY;
+            for (int v = 3 * (g << sh); v < 3 * t1; ++v) {
+                const float x = robot[(size_t)v * 3 + i];
+                lo = std::min(lo, x);
+                hi = std::max(hi, x);
+                reach = std::max(reach, std::fabs(x));
+            }
+            const float c = 0.5f * lo + 0.5f * hi;
+            o[i] = c;
+            o[4 + i] = std::nextafter(std::max(hi - c, c - lo), INFINITY);
+        }
+    }
     SceneDev& s = ctx->scene;
     MPTG_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    const std::vector<MeshNode4> nodes4 = collapse_bvh(bb.nodes);
-    if ((rc = ensure(ctx, s.mesh_nodes, sizeof(MeshNode4) * std::max<size_t>(1, nodes4.size())))) return rc;
+    std::vector<MeshNode16> wide;
+    if (!bb.nodes.empty()) collapse16(bb.nodes, 0, wide);
+    if ((rc = ensure(ctx, s.mesh_nodes, sizeof(MeshNode16) * std::max<size_t>(1, wide.size())))) return rc;
     if ((rc = ensure(ctx, s.mesh_tris, sizeof(float) * std::max<size_t>(16, tris.size())))) return rc;
     if ((rc = ensure(ctx, s.mesh_robot, sizeof(float) * std::max<size_t>(9, robot.size())))) return rc;
-    if (!nodes4.empty())
-        MPTG_HIP(ctx, hipMemcpy(s.mesh_nodes.p, nodes4.data(), sizeof(MeshNode4) * nodes4.size(),
+    if (!wide.empty())
+        MPTG_HIP(ctx, hipMemcpy(s.mesh_nodes.p, wide.data(), sizeof(MeshNode16) * wide.size(),
                                 hipMemcpyHostToDevice));
     if (!tris.empty())
         MPTG_HIP(ctx, hipMemcpy(s.mesh_tris.p, tris.data(), sizeof(float) * tris.size(), hipMemcpyHostToDevice));
     if (!robot.empty())
         MPTG_HIP(ctx, hipMemcpy(s.mesh_robot.p, robot.data(), sizeof(float) * robot.size(), hipMemcpyHostToDevice));
-    s.mesh_nnodes = (int)nodes4.size();
+    s.mesh_nnodes = (int)wide.size();
     s.mesh_nrobot = nrobot;
+    s.mesh_reach = reach;
+    s.mesh_env_reach = 0;
+    for (int64_t i = 0; i < (int64_t)nenv * 9; ++i) s.mesh_env_reach = std::max(s.mesh_env_reach, std::fabs(h_env[i]));
     s.kind = MPTG_SCENE_MESH;
     ctx->valid_upto = 0;  // valid() changed: every node is checked again
     ctx->some_invalid = false;

@@ -42,6 +42,31 @@ def test_mesh_valid_parity(ctx_factory, se3):
     assert 0.2 < want.mean() < 0.8
 
 
+@pytest.mark.parametrize("scale", [1.0, 2.0**40], ids=["plain", "huge"])
+@pytest.mark.parametrize("nrobot", [1, 64, 65, 129, 513, 1100])
+def test_mesh_valid_robot_sizes(ctx_factory, nrobot, scale):
+    """Robots around the sizes where a lane's group of triangles doubles and
+    where a second pass begins, at coordinates whose products fit FP32 and at
+    some whose do not, and poses without finite bounds: the oracle's verdicts."""
+    import dataclasses
+    _say("mesh valid", nrobot, scale)
+    sc = scenes.se3_scene(n_env_tris=3000, n_robot_tris=1200, seed_env=9, size=40.0)
+    sc = dataclasses.replace(sc, robot_tris=sc.robot_tris[:nrobot] * np.float32(scale),
+                             env_tris=sc.env_tris * np.float32(scale))
+    q = _states(np.random.default_rng(44), 508, 40.0)
+    q[:, 4:] *= scale
+    q[500:, 4] = [np.inf, -np.inf, np.nan, 3e38, 0, 0, 0, 0]
+    q[504, :4] = 0
+    q[505, 0] = np.nan
+    q[506, :4] *= 1e25
+    q[507, :4] *= 1e30
+    ctx = ctx_factory()
+    ctx.scene(sc)
+    want = oracle.Oracle(sc).valid(q)
+    assert np.array_equal(ctx.valid(q), want)
+    assert nrobot < 64 or 0.2 < want.mean() < 0.9
+
+
 def test_mesh_link_parity(ctx_factory, se3):
     _say("mesh link")
     ctx = ctx_factory()
@@ -77,12 +102,14 @@ def test_mesh_link_parity(ctx_factory, se3):
     assert (oc > 256).sum() >= 20 and gv.sum() >= 10
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 700])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 700, 2500])
 @pytest.mark.parametrize("waves", [1, 128])
 def test_mesh_link_mixed_lengths_in_one_batch(ctx_factory, se3, n, waves):
     """Zero-length, short, table-long and ring-long edges side by side in the
-    64-position batches of the link waves, for grids of few and many waves:
-    verdicts and first-failure check counts equal the oracle's."""
+    64-position batches of the link waves, for grids of few and many waves;
+    the largest batch has more table-long waypoints (some 150 an edge) than
+    the link call stores poses for.  Verdicts and first-failure check counts
+    equal the oracle's."""
     import dataclasses
     _say("mesh link mixed", n, waves)
     sparse = scenes.se3_scene(n_env_tris=1200, seed_env=7)
@@ -95,8 +122,10 @@ def test_mesh_link_mixed_lengths_in_one_batch(ctx_factory, se3, n, waves):
     near[:, 4:] += rng.normal(0, 1.0, (n, 3))
     b[0::4] = a[0::4]
     b[1::4] = near[1::4]
+    if n >= 1000:
+        b[1::4, 4:] += rng.normal(0, 35.0, (len(b[1::4]), 3))
     b[2::4, :4] = a[2::4, :4]
-    b[2::4, 4:] = a[2::4, 4:] + rng.normal(0, 6.0, (len(b[2::4]), 3))
+    b[2::4, 4:] = a[2::4, 4:] + rng.normal(0, 6.0 if n < 1000 else 35.0, (len(b[2::4]), 3))
     ctx = ctx_factory()
     ctx.scene(fine)
     ctx.tune_set(mesh_waves_per_cu=waves)
