@@ -60,6 +60,17 @@ def test_prrt_star_parity_boxes(ctx_factory, batch, target, range_):
     _say(" ", {k: st[k] for k in ("iterations", "rewires", "parent_changes", "cp_links", "rw_links", "deferred")})
 
 
+@pytest.mark.parametrize("batch", [63, 1000])
+@pytest.mark.parametrize("k", [1, 20])
+def test_prrt_star_tree_outgrows_lds(ctx_factory, batch, k):
+    """Trees that grow from one node past the 9 000 or so that the rewire pass
+    holds in LDS, in batches that are no multiple of a wave."""
+    _say("prrt* outgrows lds", batch, k)
+    sc = dataclasses.replace(scenes.boxes_scene(), range=10.0)
+    st, _ = _star_parity(ctx_factory(), sc, seed=22, batch=batch, target=10000, k=k)
+    assert st["rewires"] > 0 or k == 1
+
+
 def test_prrt_star_parity_reference_k(ctx_factory):
     _say("prrt* boxes, k = ceil(kRRG ln(n+1))")
     _star_parity(ctx_factory(), scenes.boxes_scene(), seed=22, batch=16, target=700, k=0)
