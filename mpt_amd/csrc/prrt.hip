@@ -286,6 +286,13 @@ double planner_coord_bound(const mptg_ctx* ctx) {
     return bound * (1.0 + 1e-12);
 }
 
+// A tree node's cost and links as a root has them.
+__global__ void root_init(double* __restrict__ cost, int32_t* __restrict__ child, int32_t* __restrict__ next,
+                          int32_t* __restrict__ prev) {
+    *cost = 0.0;
+    *child = *next = *prev = -1;
+}
+
 // Writes the stop condition of one run into the device counters: the next
 // iteration index, the size target and the iteration bound; clears `done`.
 int counters_arm(mptg_ctx* ctx, void* dcnt, int64_t iteration, int64_t target, int64_t max_iters) {
@@ -310,8 +317,11 @@ int counters_arm(mptg_ctx* ctx, void* dcnt, int64_t iteration, int64_t target, i
 
 namespace {
 
+// iterations enqueued ahead, at most, and the tree room reserved for them
+constexpr int64_t kSureIterations = 32, kSureNodes = 1 << 20;
+
 // Enqueues one PRRT iteration.  it >= 0: eager (host-known iteration index
-// and tree size); it < 0: graph body (both read from the device counters,
+// and tree size); it < 0: graph body or one enqueued ahead (both read from the device counters,
 // the kNN split planned for plan_n nodes).  pre: valid() before nearest
 // (no range limit, every tree node valid; see prrt_prevalid) -- the eager
 // grid search keeps its own order, so trees it serves are searched after.
@@ -486,13 +496,9 @@ int mptg_prrt_add_start(mptg_ctx* ctx, const double* h_q) {
     if (rc) return rc;
     // a start is a root: path cost 0 (Edge() at prrt_star.hpp:264-272), no children
     const int64_t id = ctx->size - 1;
-    const double zero = 0.0;
-    const int32_t none[3] = {-1, -1, -1};
-    MPTG_HIP(ctx, hipMemcpyAsync(ctx->cost + id, &zero, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    MPTG_HIP(ctx, hipMemcpyAsync(ctx->child + id, &none[0], sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    MPTG_HIP(ctx, hipMemcpyAsync(ctx->next + id, &none[1], sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    MPTG_HIP(ctx, hipMemcpyAsync(ctx->prev + id, &none[2], sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
-    MPTG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    hipLaunchKernelGGL(root_init, dim3(1), dim3(1), 0, ctx->stream, ctx->cost + id, ctx->child + id, ctx->next + id,
+                       ctx->prev + id);
+    MPTG_HIP(ctx, hipGetLastError());
     ctx->star_ok = star_ok;
     ctx->prrt.counters_valid = false;
     return MPTG_OK;
@@ -556,13 +562,27 @@ int mptg_prrt_run(mptg_ctx* ctx, int64_t target_size, int64_t max_iters, mptg_pr
     int64_t k = 0;
     bool warm = false;
     while (k < max_iters && ctx->size < target_size) {
-        int64_t ran = 1;
         const int64_t span = (int64_t)G * B;
         bool replay = G > 0 && (warm || (s.g_exec && s.g_epoch == ctx->epoch && s.g_iters == G));
         if (replay && (rc = tree_reserve(ctx, ctx->size + span))) break;
         if (!replay) {
-            if ((rc = tree_reserve(ctx, ctx->size + B))) break;
+            // An iteration adds at most B nodes, so these many are sure to
+            // run: they are enqueued with one read-back, the later ones taking
+            // the tree size from the device (a read-back is some 20 us of
+            // waiting, a third of a small iteration).  Not where the host
+            // takes part in an iteration, or where the size decides for the
+            // grid search.
+            int64_t sure = G > 0 || ctx->scene.kind == MPTG_SCENE_HOST || s.sampler
+                               ? 1
+                               : std::min({(target_size - ctx->size + B - 1) / B, max_iters - k, kSureIterations,
+                                           std::max<int64_t>(1, kSureNodes / B)});
+            while (sure > 1 && knn_grid_applies(ctx, ctx->size + (sure - 1) * B)) --sure;
+            if ((rc = tree_reserve(ctx, ctx->size + sure * B))) break;
+            if (sure > 1 && (rc = knn_reserve(ctx, B, ctx->size + sure * B))) break;
             if ((rc = enqueue_iteration(ctx, pd, s.iteration, 0, pre))) break;
+            for (int64_t i = 1; i < sure && rc == MPTG_OK; ++i)
+                rc = enqueue_iteration(ctx, pd, -1, ctx->size + i * B, pre);
+            if (rc) break;
             warm = G > 0;
         } else {
             if (!s.g_exec || s.g_epoch != ctx->epoch || s.g_iters != G || s.g_cap != ctx->cap ||
@@ -582,16 +602,15 @@ int mptg_prrt_run(mptg_ctx* ctx, int64_t target_size, int64_t max_iters, mptg_pr
                 break;
             }
             s.stats.graph_launches++;
-            ran = -1;  // read back below
         }
         if (hipMemcpyAsync(hc, dcnt, sizeof(Counters), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
             hipStreamSynchronize(ctx->stream) != hipSuccess) {
             rc = fail(ctx, MPTG_E_HIP, "reading the planner counters failed");
             break;
         }
-        if (ran < 0) ran = hc->iteration - s.iteration;
+        const int64_t ran = hc->iteration - s.iteration;
         if (ran <= 0) {
-            rc = fail(ctx, MPTG_E_STATE, "a graph launch ran no iteration");
+            rc = fail(ctx, MPTG_E_STATE, "a launch ran no iteration");
             break;
         }
         ctx->size = hc->size;
