@@ -218,6 +218,12 @@ int check_device(mptg_ctx* ctx);
 // (0 without a planner), with a 1e-12 relative margin.
 double planner_coord_bound(const mptg_ctx* ctx);
 
+// Nearest neighbour (k = 1) of a batch in up to 8 dimensions (knn_one.hip);
+// n_dev, skip and nq_dev as for launch_knn.
+bool knn_one_applies(const mptg_ctx* ctx, int64_t nq, int64_t n);
+int knn_one_path(mptg_ctx* ctx, const double* d_q, int64_t nq, double radius, int32_t* d_idx, double* d_dist,
+                 int64_t n, const int64_t* n_dev, const int32_t* skip, const uint32_t* nq_dev);
+
 // kernels launched from other translation units
 // n_dev: tree size read on the device (tree_n then only plans the split);
 // skip: device flag that turns the launch into a no-op

@@ -938,6 +938,8 @@ int knn_reserve(mptg_ctx* ctx, int64_t nq, int64_t tree_n) {
 static int knn_scan_path(mptg_ctx* ctx, const double* d_q, int64_t nq, double radius, int32_t* d_idx, double* d_dist,
                          int64_t tree_n, const int64_t* n_dev, const int32_t* skip,
                          const uint32_t* nq_dev = nullptr) {
+    if (knn_one_applies(ctx, nq, tree_n))
+        return knn_one_path(ctx, d_q, nq, radius, d_idx, d_dist, tree_n, n_dev, skip, nq_dev);
     // with n_dev, tree_n is only the size the split count is planned for;
     // with nq_dev (live queries on the device) the split is planned for half
     // of the nq slots

@@ -171,6 +171,33 @@ def test_default_prrt_star_grows_1e5_nodes_in_se3(ctx_factory):
 # wave lists (knn_wave.hip): rows shorter than a wave, one row either side of
 # a wave's 64 nodes, the tree sizes where a query gets 4 and 16 waves, and
 # enough queries (an odd count) for four per wave
+@pytest.mark.parametrize("scale", [1.0, 1e25], ids=["plain", "beyond-fp32-squares"])
+@pytest.mark.parametrize("metric,dim,n,nq", [
+    (scenes.METRIC_L2, 1, 1, 1), (scenes.METRIC_L1, 2, 255, 7), (scenes.METRIC_L2, 2, 256, 1023),
+    (scenes.METRIC_L2, 2, 1025, 1025), (scenes.METRIC_L2, 2, 5000, 4097), (scenes.METRIC_L1, 3, 2049, 2049),
+    (scenes.METRIC_L2, 4, 511, 1024), (scenes.METRIC_L1, 5, 513, 2050), (scenes.METRIC_L2, 6, 3000, 40),
+    (scenes.METRIC_L2, 7, 65535, 65), (scenes.METRIC_L1, 8, 4100, 2055), (scenes.METRIC_L2, 3, 65537, 3),
+])
+def test_knn_nearest_equals_oracle(ctx_factory, metric, dim, n, nq, scale):
+    _say("knn nearest", metric, dim, n, nq, scale)
+    ctx = ctx_factory()
+    ctx.tune_set(knn_grid=0)
+    rng = np.random.default_rng(dim * 1000 + n)
+    pts = rng.uniform(-2, 2, (n, dim)) * scale
+    pts[n // 2:n // 2 + 3] = pts[0]  # equal distances: the lowest id
+    pts[256::256][:3] = pts[0]  # and some that fall to the same lane
+    q = rng.uniform(-2.5, 2.5, (nq, dim)) * scale
+    q[0] = pts[0]
+    ctx.space(metric, dim)
+    ctx.tree_insert(pts)
+    o = oracle.Oracle(_plain(metric, dim))
+    some = np.unique(np.concatenate([[0, nq - 1], rng.integers(0, nq, 400)]))
+    for radius in (math.inf, 0.1 * scale):
+        gi, gd = ctx.knn(q, 1, radius=radius)
+        oi, od = o.knn(pts, q[some], 1, radius=radius, threads=8)
+        assert np.array_equal(gi[some], oi) and np.array_equal(gd[some], od), radius
+
+
 @pytest.mark.parametrize("metric,dim,k,n,nq", [
     (scenes.METRIC_L2, 2, 2, 1, 3), (scenes.METRIC_L2, 2, 20, 63, 100), (scenes.METRIC_L1, 3, 64, 64, 70),
     (scenes.METRIC_L2, 7, 64, 65, 70), (scenes.METRIC_L1, 1, 5, 1023, 64), (scenes.METRIC_L2, 12, 33, 1024, 1),
