@@ -589,6 +589,7 @@ int launch_arm_link(mptg_ctx* ctx, const double* from, const double* to, int64_t
     A.irregular = A.open + n;
     A.doubt = (uint64_t*)(A.irregular + n);
     if (!ctx->link_lists_clean && (rc = launch_zero_u32(ctx, (uint32_t*)A.lists, kArmListsBytes / 4))) return rc;
+    const bool was_clean = ctx->link_lists_clean;
     ctx->link_lists_clean = false;  // until both kernels are enqueued
     phase_mark(ctx, 0);
     switch (ctx->dim) {
@@ -598,7 +599,7 @@ int launch_arm_link(mptg_ctx* ctx, const double* from, const double* to, int64_t
     }
     if (rc) return rc;
     MPTG_HIP(ctx, hipGetLastError());
-    ctx->link_lists_clean = true;
+    ctx->link_lists_clean = was_clean || !stream_capturing(ctx);
     return MPTG_OK;
 }
 

@@ -43,6 +43,12 @@ int ensure(mptg_ctx* ctx, DevBuf& b, size_t bytes) {
     return MPTG_OK;
 }
 
+bool stream_capturing(const mptg_ctx* ctx) {
+    if (ctx->capturing) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 int ensure_pinned(mptg_ctx* ctx, size_t bytes) {
     if (ctx->pinned_bytes >= bytes) return MPTG_OK;
     if (ctx->pinned) {

@@ -155,6 +155,10 @@ struct mptg_ctx {
     // the arm or mesh link's list counters are zero (its last kernel clears them);
     // false after an allocation or a failed launch
     bool link_lists_clean = false;
+    // DMV link: which of scratch[7]'s two long-edge counts is next, and whether
+    // it is zero
+    int dmv_turn = 0;
+    bool dmv_counts_clean = false;
     // pinned host staging
     void* pinned = nullptr;
     size_t pinned_bytes = 0;
@@ -208,6 +212,9 @@ inline int pitch32(int dim) { return dim <= 2 ? 2 : (dim <= 4 ? 4 : (dim <= 8 ? 
 
 int ensure(mptg_ctx* ctx, DevBuf& b, size_t bytes);
 int ensure_pinned(mptg_ctx* ctx, size_t bytes);
+// Whether launches on the context's stream are being captured, by a planner or
+// by the owner of the stream: they run on every replay, or never.
+bool stream_capturing(const mptg_ctx* ctx);
 // Entry-point prologue: selects the context's device and retires captured
 // graphs (the call may change state they hold).
 int check_device_ready(mptg_ctx* ctx);

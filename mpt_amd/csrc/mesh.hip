@@ -848,6 +848,7 @@ int launch_mesh_link(mptg_ctx* ctx, const uint8_t* d_table, const double* d_from
     MeshWork* work = (MeshWork*)buf.p;
     uint2* live = (uint2*)((char*)buf.p + kMeshWorkBytes);
     if (!ctx->link_lists_clean && (rc = launch_zero_u32(ctx, (uint32_t*)work, kMeshWorkBytes / 4))) return rc;
+    const bool was_clean = ctx->link_lists_clean;
     ctx->link_lists_clean = false;  // until every kernel is enqueued
     const unsigned g1 = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(mesh_link_prepare, dim3(g1), dim3(256), 0, ctx->stream, space_args(ctx), 1.0 / ctx->link_param,
@@ -861,7 +862,7 @@ int launch_mesh_link(mptg_ctx* ctx, const uint8_t* d_table, const double* d_from
     hipLaunchKernelGGL(mesh_link_finish, dim3(g1), dim3(256), 0, ctx->stream, space_args(ctx), 1.0 / ctx->link_param,
                        d_from, d_to, n, d_mask, d_verdict, d_checks, work);
     MPTG_HIP(ctx, hipGetLastError());
-    ctx->link_lists_clean = true;
+    ctx->link_lists_clean = was_clean || !stream_capturing(ctx);
     return MPTG_OK;
 }
 

@@ -139,7 +139,9 @@ __global__ __launch_bounds__(kBlock) void link_dmv_lanes(SpaceArgs sp, SceneArgs
                                                          const uint8_t* __restrict__ mask,
                                                          uint8_t* __restrict__ verdict, uint32_t* __restrict__ checks,
                                                          int64_t* __restrict__ long_list,
-                                                         uint32_t* __restrict__ long_count) {
+                                                         uint32_t* __restrict__ long_count,
+                                                         uint32_t* __restrict__ next_count) {
+    if (next_count && blockIdx.x == 0 && threadIdx.x == 0) *next_count = 0u;
     constexpr int DA = D > 0 ? D : kMaxDim;
     constexpr int U = dmv_unroll<D>();
     const int dd = D > 0 ? D : sp.dim;
@@ -646,8 +648,8 @@ int launch_valid(mptg_ctx* ctx, const double* d_q, int64_t n, uint8_t* d_ok) {
 }
 
 static int launch_dmv(mptg_ctx* ctx, const uint8_t* table8, const uint16_t* table16, int64_t* long_list,
-                      uint32_t* long_count, const double* d_from, const double* d_to, int64_t n, int known_valid,
-                      const uint8_t* d_mask, uint8_t* d_verdict, uint32_t* d_checks);
+                      uint32_t* long_count, uint32_t* next_count, const double* d_from, const double* d_to,
+                      int64_t n, int known_valid, const uint8_t* d_mask, uint8_t* d_verdict, uint32_t* d_checks);
 
 int launch_link(mptg_ctx* ctx, const double* d_from, const double* d_to, int64_t n, int order, int known_valid,
                 uint8_t* d_verdict, uint32_t* d_checks) {
@@ -692,20 +694,38 @@ int launch_link_masked(mptg_ctx* ctx, const double* d_from, const double* d_to, 
     if (ctx->scene.kind == MPTG_SCENE_MESH)
         return launch_mesh_link(ctx, (const uint8_t*)ctx->scratch[6].p, d_from, d_to, n, known_valid, d_mask,
                                 d_verdict, d_checks);
+    if (!ctx->scratch[7].p || ctx->scratch[7].bytes < sizeof(int64_t) * n + 256) ctx->dmv_counts_clean = false;
     if ((rc = ensure(ctx, ctx->scratch[7], sizeof(int64_t) * n + 256))) return rc;
-    uint32_t* long_count = (uint32_t*)ctx->scratch[7].p;
+    // Two counts in turn: a call zeroes the one of the call after it, which
+    // the call before is done with (a launch, 4.5 us of a planner's iteration,
+    // less).  A captured call is replayed with what it captured, so it has a
+    // third count and zeroes it first.
+    uint32_t* counts = (uint32_t*)ctx->scratch[7].p;
     int64_t* long_list = (int64_t*)((char*)ctx->scratch[7].p + 256);
-    return launch_dmv(ctx, (const uint8_t*)ctx->scratch[6].p, (const uint16_t*)ctx->dmv_table16.p, long_list,
-                      long_count, d_from, d_to, n, known_valid, d_mask, d_verdict, d_checks);
+    const uint8_t* table8 = (const uint8_t*)ctx->scratch[6].p;
+    const uint16_t* table16 = (const uint16_t*)ctx->dmv_table16.p;
+    if (stream_capturing(ctx))
+        return launch_dmv(ctx, table8, table16, long_list, counts + 2, nullptr, d_from, d_to, n, known_valid, d_mask,
+                          d_verdict, d_checks);
+    if (!ctx->dmv_counts_clean && (rc = launch_zero_u32(ctx, counts, 2))) return rc;
+    ctx->dmv_counts_clean = false;  // until both kernels are enqueued
+    const int turn = ctx->dmv_turn;
+    rc = launch_dmv(ctx, table8, table16, long_list, counts + turn, counts + (turn ^ 1), d_from, d_to, n, known_valid,
+                    d_mask, d_verdict, d_checks);
+    if (rc) return rc;
+    ctx->dmv_turn = turn ^ 1;
+    ctx->dmv_counts_clean = true;
+    return MPTG_OK;
 }
 
 // The DMV link kernels over n edges, with the order tables and the long-edge
-// list (n entries) and count given by the caller.
+// list (n entries) and count given by the caller; the count is zeroed by a
+// launch, or is zero already and *next_count is zeroed on the way.
 static int launch_dmv(mptg_ctx* ctx, const uint8_t* table8, const uint16_t* table16, int64_t* long_list,
-                      uint32_t* long_count, const double* d_from, const double* d_to, int64_t n, int known_valid,
-                      const uint8_t* d_mask, uint8_t* d_verdict, uint32_t* d_checks) {
+                      uint32_t* long_count, uint32_t* next_count, const double* d_from, const double* d_to,
+                      int64_t n, int known_valid, const uint8_t* d_mask, uint8_t* d_verdict, uint32_t* d_checks) {
     int rc;
-    if ((rc = launch_zero_u32(ctx, long_count, 1))) return rc;
+    if (!next_count && (rc = launch_zero_u32(ctx, long_count, 1))) return rc;
     double inv = 1.0 / ctx->link_param;
     unsigned lg = (unsigned)std::min<int64_t>(n, (int64_t)ctx->cus * ctx->tune.dmv_long_waves_per_cu);
     // lanes per edge, fewer where n edges at the tuned count would pass 2^31 threads
@@ -715,7 +735,7 @@ static int launch_dmv(mptg_ctx* ctx, const uint8_t* table8, const uint16_t* tabl
     auto launch = [&]<int D, int K>() {
         hipLaunchKernelGGL((link_dmv_lanes<D, K>), dim3(sblocks), dim3(kBlock), 0, ctx->stream, space_args(ctx),
                            scene_args(ctx), inv, lanes_log2, table8, d_from, d_to, n, known_valid, d_mask, d_verdict,
-                           d_checks, long_list, long_count);
+                           d_checks, long_list, long_count, next_count);
         hipLaunchKernelGGL((link_dmv_long<D, K>), dim3(lg), dim3(64), 0, ctx->stream, space_args(ctx),
                            scene_args(ctx), inv, table16, d_from, d_to, long_list, long_count, d_verdict, d_checks);
     };
@@ -826,7 +846,7 @@ int link_dev_noalloc(mptg_ctx* ctx, const double* d_from, const double* d_to, in
     if (rc) return rc;
     return launch_dmv(ctx, base + kNaTableOff, reinterpret_cast<const uint16_t*>(base + kNaTable16Off),
                       reinterpret_cast<int64_t*>(base + kNaListOff), reinterpret_cast<uint32_t*>(base + kNaCountOff),
-                      d_from, d_to, n, known_valid, nullptr, d_verdict, d_checks);
+                      nullptr, d_from, d_to, n, known_valid, nullptr, d_verdict, d_checks);
 }
 
 }  // namespace mptg
