@@ -354,7 +354,7 @@ __device__ __forceinline__ bool tri_tri_overlap_wave(const float* p, const float
 // separating-axis test, 64 at a time.  Each of the lists passes its entries on
 // when it holds a wave's worth, and in the end.
 //
-// Bounds: instruction issue (1 600 vector and 1 050 scalar instructions per
+// Bounds: instruction issue (1 370 vector and 920 scalar instructions per
 // counted check, 500 robot triangles among 50 000) and, for half of a wave's
 // time, the latency of dependent loads; sixteen-wide nodes make four or five
 // of them on the way to a leaf, four-wide ones took nine (142 -> 126 us for
