@@ -293,7 +293,7 @@ __device__ __forceinline__ void arm_block(const ArmLinkArgs& A, ArmEdge<D>* edge
 
     // One call site for every round (inlined once).  Stage 0: the end states
     // of the wave's own edge; 1: its own first round; 2: the open edges.
-    const bool own = w < E && edges[w].status == kEdgeLive;
+    const bool own = w < E && edges[w].status != kEdgeNone;  // (over the limit: W = 0, the end states alone)
     int stage = A.known_valid ? 1 : 0, i = w;
     uint32_t key = 0;
     const uint32_t key0 = 2u + (uint32_t)R * (uint32_t)((E == P ? 1 : 0) + w);
@@ -327,15 +327,15 @@ __device__ __forceinline__ void arm_block(const ArmLinkArgs& A, ArmEdge<D>* edge
     if (threadIdx.x < E) {
         const ArmEdge<D>& ed = edges[threadIdx.x];
         const int64_t e = ed.e;
-        if (ed.status == kEdgeOverLimit) {
-            A.verdict[e] = 0;
-            A.checks[e] = MPTG_CHECKS_OVER_LIMIT;
-        } else if (ed.status == kEdgeLive) {
+        if (ed.status != kEdgeNone) {
             if (!EXACT && ed.open < ed.first) {
                 A.open[atomicAdd(&A.lists->n_open, 1u)] = e;
+            } else if (ed.first != kNoKey) {
+                A.verdict[e] = 0;
+                A.checks[e] = ed.first + 1u;
             } else {
-                A.verdict[e] = ed.first == kNoKey;
-                A.checks[e] = ed.first == kNoKey ? 2u + ed.W : ed.first + 1u;
+                A.verdict[e] = ed.status == kEdgeLive;
+                A.checks[e] = ed.status == kEdgeLive ? 2u + ed.W : MPTG_CHECKS_OVER_LIMIT;
             }
         }
     }

@@ -9,6 +9,7 @@ import sys
 import numpy as np
 import pytest
 
+import mpt_amd
 import oracle
 from conftest import GPU_ITER_CAP
 from mpt_amd import scenes
@@ -289,6 +290,38 @@ def test_arm_checks_at_the_bounds_are_exact(ctx_factory, links, n, span):
     gv, gc = ctx.link(q[:250], q[:250] + 0.3)
     ov, oc = o.link(q[:250], q[:250] + 0.3, threads=16)
     assert np.array_equal(gv, ov) and np.array_equal(gc, oc)
+
+
+@pytest.mark.parametrize("links,n", [(5, 1), (5, 2500), (10, 70), (20, 300), (20, 2100)])
+def test_arm_over_limit_edges_check_their_ends_first(ctx_factory, links, n):
+    """An edge of more than 30 bisection levels still answers for its end
+    states: one check where valid(from) fails, two where valid(to) does, and
+    the limit only where both hold or are vouched for."""
+    _say("arm over the limit", links, n)
+    sc = dataclasses.replace(scenes.arm_scene(links=links, ndisks=20), link_param=1e-13)
+    ctx = ctx_factory()
+    ctx.scene(sc)
+    rng = np.random.default_rng(52)
+    a, b = rng.uniform(-math.pi, math.pi, (2, n, links))
+    o = oracle.Oracle(sc)
+    va, vb = o.valid(a), o.valid(b)
+    over = np.uint32(0xffffffff)
+    want = np.where(~va, np.uint32(1), np.where(~vb, np.uint32(2), over))
+    if n > 1:
+        assert (want == 1).any() and (want == 2).any() and (want == over).any()
+    da, db = ctx.to_device(a), ctx.to_device(b)
+    v, c = ctx.array(n, np.uint8), ctx.array(n, np.uint32)
+    ctx.surrogate_init(3)
+    for order in (mpt_amd.ORDER_REFERENCE, mpt_amd.ORDER_SURROGATE):
+        for kv in (False, True):
+            ctx.link_dev(da.ptr, db.ptr, n, order, kv, v.ptr, c.ptr)
+            ctx.sync()
+            assert not v.numpy().any()
+            assert np.array_equal(c.numpy(), np.full(n, over) if kv else want), (order, kv)
+    bad = ~(va & vb)
+    if bad.any():  # host arrays: no edge of these exceeds the limit's report
+        gv, gc = ctx.link(a[bad], b[bad])
+        assert not gv.any() and np.array_equal(gc, want[bad])
 
 
 # ---- whole trees -------------------------------------------------------------
