@@ -575,8 +575,8 @@ __device__ __forceinline__ int64_t mesh_waypoints(const SpaceArgs& sp, const dou
 
 __global__ __launch_bounds__(256) void mesh_link_prepare(SpaceArgs sp, double inv, const double* __restrict__ from,
                                                          const double* __restrict__ to, int64_t n,
-                                                         const uint8_t* __restrict__ mask, uint32_t* __restrict__ slot,
-                                                         MeshWork* __restrict__ work, uint2* __restrict__ live) {
+                                                         int known_valid, const uint8_t* __restrict__ mask,
+                                                         uint32_t* __restrict__ slot, MeshWork* __restrict__ work, uint2* __restrict__ live) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int lane = threadIdx.x & 63;
     int mw = -1;
@@ -590,7 +590,10 @@ __global__ __launch_bounds__(256) void mesh_link_prepare(SpaceArgs sp, double in
                 b[j] = to[e * 7 + j];
             }
             const int64_t w = mesh_waypoints(sp, a, b, inv);
-            if (w <= kMaxDmvWaypointsMesh) mw = (int)w;  // beyond: not checked, the finish kernel reports it
+            // over the limit: valid(to) alone is checked; if it holds, the
+            // finish kernel reports the edge
+            if (w <= kMaxDmvWaypointsMesh) mw = (int)w;
+            else if (!known_valid) mw = 0;
         }
     }
     const uint64_t m = __ballot(mw >= 0);
@@ -852,7 +855,7 @@ int launch_mesh_link(mptg_ctx* ctx, const uint8_t* d_table, const double* d_from
     ctx->link_lists_clean = false;  // until every kernel is enqueued
     const unsigned g1 = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(mesh_link_prepare, dim3(g1), dim3(256), 0, ctx->stream, space_args(ctx), 1.0 / ctx->link_param,
-                       d_from, d_to, n, d_mask, d_checks, work, live);
+                       d_from, d_to, n, known_valid, d_mask, d_checks, work, live);
     // waves: as many as the device holds, or 256 per edge (every waypoint of
     // a short edge at once) in a batch too small for that (the rewire pass's
     // late batches hold a few edges)

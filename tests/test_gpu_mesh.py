@@ -135,6 +135,35 @@ def test_mesh_link_mixed_lengths_in_one_batch(ctx_factory, se3, n, waves):
         assert np.array_equal(gv, ov) and np.array_equal(gc, oc), kv
 
 
+@pytest.mark.parametrize("n", [1, 65, 700])
+def test_mesh_over_limit_edges_check_valid_to_first(ctx_factory, se3, n):
+    """An edge of more than 2^24 waypoints whose end state collides fails
+    there, after one check; the limit is reported only where valid(to) holds
+    or is vouched for."""
+    import dataclasses
+    _say("mesh over the limit", n)
+    sc = dataclasses.replace(se3, link_param=1e-9)
+    rng = np.random.default_rng(47)
+    a, b = _states(rng, n), _states(rng, n)
+    ok = oracle.Oracle(sc).valid(b)
+    over = np.uint32(0xffffffff)
+    want = np.where(ok, over, np.uint32(1))
+    if n > 1:
+        assert ok.any() and not ok.all()
+    ctx = ctx_factory()
+    ctx.scene(sc)
+    da, db = ctx.to_device(a), ctx.to_device(b)
+    v, c = ctx.array(n, np.uint8), ctx.array(n, np.uint32)
+    for kv in (False, True):
+        ctx.link_dev(da.ptr, db.ptr, n, 0, kv, v.ptr, c.ptr)
+        ctx.sync()
+        assert not v.numpy().any()
+        assert np.array_equal(c.numpy(), np.full(n, over) if kv else want), kv
+    if not ok.all():
+        gv, gc = ctx.link(a[~ok], b[~ok])
+        assert not gv.any() and (gc == 1).all()
+
+
 def test_mesh_prrt_tree_parity(ctx_factory, se3):
     _say("mesh prrt")
     ctx = ctx_factory()
