@@ -451,6 +451,7 @@ __device__ __forceinline__ bool arm_exact_wave(const SceneArgs& sc, const double
         fy = i < lane ? fy + vy : fy;
     }
     const double tx = fx + lx, ty = fy + ly;
+    if (__ballot(mine && joint_lost(tx, ty))) return sc.ndisks == 0;
     const float inv = sc.near_inv, mid = sc.near_extent * inv;
     const int nc = sc.near_n;
     int ix = (int)__builtin_fmaf(0.5f * ((float)fx + (float)tx), inv, mid);

@@ -335,6 +335,10 @@ __device__ __forceinline__ bool disk_clear(const ArmDisk& dk, double fx, double 
 // cross-lane operation: lanes may call it divergently.
 constexpr int kArmGroup = 5;
 
+// A joint past an angle that sincos does not take (from 2^20 pi/2 on) is no
+// number: no distance to it exceeds any radius, so the state hits every disk.
+__device__ __forceinline__ bool joint_lost(double x, double y) { return x != x || y != y; }
+
 template <int D, typename Coord>
 __device__ __forceinline__ bool arm_ok_lane(const SceneArgs& sc, Coord&& coord) {
     constexpr int G = (D + kArmGroup - 1) / kArmGroup;
@@ -367,6 +371,7 @@ __device__ __forceinline__ bool arm_ok_lane(const SceneArgs& sc, Coord&& coord) 
                 last_y = jy[k];
             }
         const double mx = (jx[0] + last_x) / 2, my = (jy[0] + last_y) / 2;
+        if (joint_lost(mx, my)) return sc.ndisks == 0;
         const double rho = sc.arm_lim[D + g];
         const double Rmax = (rho + ag.rtmax) * (1.0 + 0x1.0p-40) + 1e-12;
         const int gx0 = arm_cell(mx - Rmax, ag.x0, ag.ix, ag.nx), gx1 = arm_cell(mx + Rmax, ag.x0, ag.ix, ag.nx);
@@ -438,13 +443,15 @@ __device__ __forceinline__ bool arm_ok_split(const SceneArgs& sc, Coord&& coord,
         const double rho = sc.arm_lim[D + g];
         const double Rmax = (rho + ag.rtmax) * (1.0 + 0x1.0p-40) + 1e-12;
         int gx0 = 0, gx1 = -1, gy0 = 0, gy1 = -1;
-        if (active && ok) {
+        bool hit = false;
+        if (active && ok && joint_lost(mx, my)) {
+            hit = sc.ndisks > 0;
+        } else if (active && ok) {
             gx0 = arm_cell(mx - Rmax, ag.x0, ag.ix, ag.nx);
             gx1 = arm_cell(mx + Rmax, ag.x0, ag.ix, ag.nx);
             gy0 = arm_cell(my - Rmax, ag.y0, ag.iy, ag.ny);
             gy1 = arm_cell(my + Rmax, ag.y0, ag.iy, ag.ny);
         }
-        bool hit = false;
         // the group's disk runs, row after row, dealt to its L lanes in turn
         for (int gy = gy0; gy <= gy1 && !hit; ++gy) {
         const int j0 = ag.starts[gy * ag.nx + gx0], j1 = ag.starts[gy * ag.nx + gx1 + 1];

@@ -324,6 +324,32 @@ def test_arm_over_limit_edges_check_their_ends_first(ctx_factory, links, n):
         assert not gv.any() and np.array_equal(gc, want[bad])
 
 
+@pytest.mark.parametrize("links", [5, 10, 20])
+@pytest.mark.parametrize("ndisks", [0, 1, 40])
+def test_arm_angles_past_sincos(ctx_factory, links, ndisks):
+    """Angles of 2^20 pi/2 and more have no sine: such a state hits every
+    disk there is.  Angles on both sides of that line, coordinates whose sum
+    passes it, few edges and many; verdicts and counts equal the oracle's."""
+    _say("arm angles past sincos", links, ndisks)
+    sc = scenes.arm_scene(links=links, ndisks=ndisks)
+    sc = dataclasses.replace(sc, disks=np.asarray(sc.disks).reshape(-1, 3))
+    ctx = ctx_factory()
+    ctx.scene(sc)
+    o = oracle.Oracle(sc)
+    rng = np.random.default_rng(53)
+    line = 2.0 ** 20 * math.pi / 2
+    for n in (60, 2100):
+        a = rng.uniform(-math.pi, math.pi, (n, links))
+        a[0::3, rng.integers(0, links)] += line
+        a[1::3] += line / links  # the sum reaches the line near the last link
+        b = a + rng.uniform(-0.4, 0.4, (n, links))
+        assert np.array_equal(ctx.valid(a), o.valid(a))
+        for kv in (False, True):
+            gv, gc = ctx.link(a, b, endpoints_known_valid=kv)
+            ov, oc = o.link(a, b, known_valid=kv, threads=16)
+            assert np.array_equal(gv, ov) and np.array_equal(gc, oc), (n, kv)
+
+
 # ---- whole trees -------------------------------------------------------------
 def _planner_parity(ctx, sc, seed, batch, target, max_iters=1 << 30):
     ctx.scene(sc)
