@@ -170,7 +170,8 @@ static void near_lists(const double* len, int nlinks, const std::vector<double>&
             const double* d = &disks[4 * (size_t)i];
             const double reach = longest / 2 + d[3] + slack;
             if (std::fabs(d[0]) > T + reach || std::fabs(d[1]) > T + reach) continue;
-            auto cell = [&](double v) { return std::max(0, std::min(n - 1, (int)std::floor((v + T) / size))); };
+            // (clamped before the cast: a disk may reach any number of cells past the square)
+            auto cell = [&](double v) { return (int)std::min(n - 1.0, std::max(0.0, std::floor((v + T) / size))); };
             const int x0 = cell(d[0] - reach) - 1, x1 = cell(d[0] + reach) + 1;
             const int y0 = cell(d[1] - reach) - 1, y1 = cell(d[1] + reach) + 1;
             for (int y = std::max(0, y0); y <= std::min(n - 1, y1); ++y)

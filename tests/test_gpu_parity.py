@@ -350,6 +350,31 @@ def test_arm_angles_past_sincos(ctx_factory, links, ndisks):
             assert np.array_equal(gv, ov) and np.array_equal(gc, oc), (n, kv)
 
 
+@pytest.mark.parametrize("scale", [2e-4, 1e-6])
+def test_small_arm_among_huge_disks(ctx_factory, scale):
+    """A disk some 10^9 times the arm's cells: one that covers everything, one
+    whose edge passes through the arm's reach, one out of reach; alone and
+    beside small disks, few edges and many."""
+    _say("small arm, huge disks", scale)
+    base = scenes.arm_scene(links=20, ndisks=30)
+    total = float(base.lengths.sum()) * scale
+    small = np.asarray(base.disks) * scale
+    rng = np.random.default_rng(54)
+    for cx, r in ((4e5, 5e5), (4e5, 4e5 - 0.3 * total), (-2e5, 2e5 - 0.5 * total), (4e5, 1e5)):
+        for others, n in ((small, 2100), (small[:0], 2100), (small[:0], 40)):
+            sc = dataclasses.replace(base, lengths=base.lengths * scale, robot_radius=0.0,
+                                     disks=np.concatenate([others, [[cx, 0.0, r]]]))
+            ctx = ctx_factory()
+            ctx.scene(sc)
+            o = oracle.Oracle(sc)
+            a = rng.uniform(-math.pi, math.pi, (n, 20))
+            b = a + rng.uniform(-0.4, 0.4, a.shape)
+            assert np.array_equal(ctx.valid(a), o.valid(a)), (cx, r, n)
+            gv, gc = ctx.link(a, b)
+            ov, oc = o.link(a, b, threads=16)
+            assert np.array_equal(gv, ov) and np.array_equal(gc, oc), (cx, r, n)
+
+
 # ---- whole trees -------------------------------------------------------------
 def _planner_parity(ctx, sc, seed, batch, target, max_iters=1 << 30):
     ctx.scene(sc)
