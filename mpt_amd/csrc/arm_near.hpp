@@ -21,12 +21,13 @@
 // 20 000 is left to the exact one.
 //
 // Margin.  With T = the sum of the link lengths, Lm the longest link and rm
-// the largest r + R, the FP32 distance differs from the exact expression's by
+// the disk's r + R, the FP32 distance differs from the exact expression's by
 // less than the sum of
 //   directions: the angle's rounding 2^-26 turns = 9.4e-8 rad and the
 //     instructions' error, at most 1.26e-7 each on gfx950 over every FP32
 //     argument in [-1/2, 1/2] (measured exhaustively): 2.8e-7 T over the
-//     chain; angles below kMaxTurns turns in FP64 add under 1e-10 T;
+//     chain; angles below kMaxTurns turns in FP64, and the exact test's own
+//     sums and midpoints of them, add under 1.5e-7 T;
 //   joints: lengths rounded to FP32, five links summed per lane, at most
 //     three prefix sums and one addition, each 2^-24 T, both axes: 8.3e-7 T;
 //   the centre's rounding, |centre| below T + Lm + 2 rm where it matters:
@@ -34,15 +35,18 @@
 //   the distance itself, a dozen FP32 operations on values below Lm + rm:
 //     8e-7 (Lm + rm);
 //   the exact expression's own FP64 rounding: below 1e-11 T.
-// The sum is below 1.2e-6 T + 9e-7 Lm + 1e-6 rm; the margin is kNearMargin
-// (T + Lm + 2 rm) with kNearMargin = 2^-18 = 3.8e-6, three times that.
+// The sum is below 1.35e-6 T + 9e-7 Lm + 1e-6 rm; the disk's margin is
+// kNearMargin (T + Lm + rm) with kNearMargin = 2^-18 = 3.8e-6, 2.8 times that.
+// (A margin from the scene's largest disk left the checks near every disk in
+// doubt: 8192 edges beside a wall of radius 1e5 took 700 us, 37 now.  Angles
+// above 1024 turns left to the exact test took 1 450 us, 31 now.)
 #pragma once
 #include "bisect_dev.hpp"
 
 namespace mptg {
 
 constexpr int kNearLinks = 5;  // links per lane
-constexpr double kMaxTurns = 1024.0;
+constexpr double kMaxTurns = 131072.0;  // half of what pm::sincos takes
 constexpr double kInv2Pi = 0.15915494309189533577;
 
 template <int D>

@@ -155,20 +155,20 @@ static void near_lists(const double* len, int nlinks, const std::vector<double>&
         rmax = std::max(rmax, d[3]);
     }
     // the FP32 squares stay clear of overflow and of denormals
-    if (!(T > 1e-6) || !(T + rmax < 1e6)) return;
-    const double margin = kNearMargin * (T + longest + 2.0 * rmax);
+    if (!(T > kNearLeast) || !(T + rmax < kNearMost)) return;
+    auto margin = [&](const double* d) { return kNearMargin * (T + longest + d[3]); };
     // cells half a link wide: the lists are then within a third of the
     // shortest possible, and 64 x 64 cells of the 20-link arm stay in L2
     const int n = std::max(1, std::min(kNearCells, (int)std::ceil(4.0 * T / longest)));
     const double size = 2.0 * T / n;
-    // the midpoint's error is a joint's; its cell coordinate's FP32 rounding
-    // is within 1e-6 T
-    const double slack = 2.0 * margin + 8e-6 * T;
     cells->assign((size_t)n * n, make_uint2(0, 0));
     auto visit = [&](auto&& take) {
         for (int i = 0; i < ndisks; ++i) {
             const double* d = &disks[4 * (size_t)i];
-            const double reach = longest / 2 + d[3] + slack;
+            // the midpoint's error is a joint's; its cell coordinate's FP32
+            // rounding is within 1e-6 T; rounding here and in the exact
+            // expression is below 1e-12 r
+            const double reach = longest / 2 + d[3] + 2.0 * margin(d) + 8e-6 * T;
             if (std::fabs(d[0]) > T + reach || std::fabs(d[1]) > T + reach) continue;
             // (clamped before the cast: a disk may reach any number of cells past the square)
             auto cell = [&](double v) { return (int)std::min(n - 1.0, std::max(0.0, std::floor((v + T) / size))); };
@@ -195,7 +195,7 @@ static void near_lists(const double* len, int nlinks, const std::vector<double>&
     ids->assign(out->size(), 0);
     visit([&](size_t c, int i) {
         const double* d = &disks[4 * (size_t)i];
-        const double lo = std::max(d[3] - margin, 0.0), hi = d[3] + margin;
+        const double lo = std::max(d[3] - margin(d), 0.0), hi = d[3] + margin(d);
         const size_t at = (*cells)[c].x + (*cells)[c].y++;
         (*ids)[at] = i;
         (*out)[at] = make_float4((float)d[0], (float)d[1], std::nextafterf((float)(lo * lo), 0.0f),

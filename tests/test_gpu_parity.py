@@ -375,6 +375,41 @@ def test_small_arm_among_huge_disks(ctx_factory, scale):
             assert np.array_equal(gv, ov) and np.array_equal(gc, oc), (cx, r, n)
 
 
+@pytest.mark.parametrize("links", [5, 20])
+@pytest.mark.parametrize("scale", [1e-16, 1e-12, 1e-7, 1e7, 1e15, 1e18])
+def test_arm_in_any_unit(ctx_factory, links, scale):
+    """The same arm in units on both sides of those the FP32 bounds take, and
+    at the angles where they end; a wall (a disk of 10^4 arm lengths) beside
+    the small disks.  Verdicts and counts equal the oracle's, and the units
+    that the bounds take leave no walk to the exact checks."""
+    _say("arm in units", links, scale)
+    base = scenes.arm_scene(links=links, ndisks=20)
+    total = float(base.lengths.sum())
+    rng = np.random.default_rng(55)
+    for wall in (False, True):
+        disks = np.asarray(base.disks)
+        if wall:
+            disks = np.concatenate([disks, [[1e4 * total + 0.4 * total, 0.0, 1e4 * total]]])
+        sc = dataclasses.replace(base, lengths=base.lengths * scale, disks=disks * scale,
+                                 robot_radius=base.robot_radius * scale)
+        ctx = ctx_factory()
+        ctx.scene(sc)
+        o = oracle.Oracle(sc)
+        for n, turn in ((50, 0.0), (2100, 0.0), (300, 131072.0), (300, 5e4)):
+            a = rng.uniform(-math.pi, math.pi, (n, links))
+            a[:, 0] += turn * 2 * math.pi
+            b = a + rng.uniform(-0.4, 0.4, a.shape)
+            assert np.array_equal(ctx.valid(a), o.valid(a)), (wall, n, turn)
+            for kv in (False, True):
+                gv, gc = ctx.link(a, b, endpoints_known_valid=kv)
+                ov, oc = o.link(a, b, known_valid=kv, threads=16)
+                assert np.array_equal(gv, ov) and np.array_equal(gc, oc), (wall, n, turn, kv)
+            if 1e-12 <= scale <= 1e11 and turn < 1e5:
+                da, db = ctx.to_device(a), ctx.to_device(b)
+                w = ctx.link_work(da.ptr, db.ptr, n, known_valid=True)
+                assert w["group"] > 0 and w["exact"] == 0, (wall, n, turn, w)
+
+
 # ---- whole trees -------------------------------------------------------------
 def _planner_parity(ctx, sc, seed, batch, target, max_iters=1 << 30):
     ctx.scene(sc)
