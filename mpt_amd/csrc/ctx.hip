@@ -138,72 +138,148 @@ int tree_reserve(mptg_ctx* ctx, int64_t cap) {
 // Disk lists of the arm's FP32 clearance bounds (arm_near.hpp): per cell of an
 // n x n grid over the square the joints can reach, every disk a link whose
 // midpoint lies in the cell may touch, with the squared distances below and
-// above which the FP32 test is certain.  disks: [cx, cy, (r+R)^2, r+R].
-// near_n = 0 (no lists) for arms and disks outside the bounds' assumptions.
-static void near_lists(const double* len, int nlinks, const std::vector<double>& disks, int ndisks, SceneDev* sd,
-                       std::vector<uint2>* cells, std::vector<float4>* out, std::vector<int32_t>* ids) {
-    sd->near_n = 0;
+// above which the FP32 test is certain.  A cell inside a disk by more than the
+// margins needs that disk alone: every such link hits it.
+//
+// A wave per cell, sixteen to a block: one pass over the disks counts (or finds
+// a disk around the cell), an atomic add takes the block's place in the lists
+// (one per cell, on the one address, took 30 us), a second pass writes the
+// entries.  Built on the host and copied in three pieces the lists took two
+// thirds of a scene's upload (20 links, 200 disks: 60 us without them, 180
+// with; 5000 disks 0.62 and 2.2 ms; 3000 disks that each reach most cells 0.31
+// and 13 ms; now, with one copy for the rest and a counting sort, 41 us, 0.27
+// and 0.11 ms).
+struct NearBuild {
+    const ArmDisk* disks;
+    int ndisks, n;
+    double T, longest;  // all links, the longest
+    uint32_t cap;       // entries there is room for
+    uint32_t* total;    // entries there are
+    uint2* cells;
+    float4* out;
+    int32_t* ids;
+};
+
+constexpr int kNearWaves = 16;
+__global__ __launch_bounds__(64 * kNearWaves) void near_lists(NearBuild B) {
+    __shared__ uint32_t counts[kNearWaves], first;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int cell = (int)blockIdx.x * kNearWaves + w;
+    const bool have = cell < B.n * B.n;
+    const int ndisks = have ? B.ndisks : 0;
+    const double size = 2.0 * B.T / B.n;
+    const double lx = -B.T + (cell % B.n) * size, ly = -B.T + (cell / B.n) * size;
+    auto margin = [&](const ArmDisk& d) { return kNearMargin * (B.T + B.longest + d.rt); };
+    auto near = [&](const ArmDisk& d, bool* around) {
+        // the midpoint's error is a joint's; its cell coordinate's FP32
+        // rounding is within 1e-6 T; rounding here and in the exact
+        // expression is below 1e-12 r
+        const double slack = 2.0 * margin(d) + 8e-6 * B.T;
+        const double reach = B.longest / 2 + d.rt + slack, inside = d.rt - slack;
+        const double x0 = lx - d.cx, x1 = d.cx - (lx + size), y0 = ly - d.cy, y1 = d.cy - (ly + size);
+        const double gx = __builtin_fmax(__builtin_fmax(x0, x1), 0.0), gy = __builtin_fmax(__builtin_fmax(y0, y1), 0.0);
+        const double fx = __builtin_fmax(-x0, -x1), fy = __builtin_fmax(-y0, -y1);  // to the farthest corner
+        *around = inside > 0.0 && fx * fx + fy * fy < inside * inside;
+        return gx * gx + gy * gy <= reach * reach;
+    };
+    auto entry = [&](uint32_t at, int i, const ArmDisk& d) {
+        const double lo = __builtin_fmax(d.rt - margin(d), 0.0), hi = d.rt + margin(d);
+        B.ids[at] = i;
+        B.out[at] = make_float4((float)d.cx, (float)d.cy, __double2float_rd(lo * lo), __double2float_ru(hi * hi));
+    };
+    uint32_t count = 0;
+    int alone = -1;
+    for (int i0 = 0; i0 < ndisks && alone < 0; i0 += 64) {
+        const int i = i0 + lane;
+        bool around = false;
+        const bool take = i < ndisks && near(B.disks[i], &around);
+        const uint64_t a = __ballot(around);
+        if (a) alone = i0 + (int)__builtin_ctzll(a);
+        count += (uint32_t)__popcll(__ballot(take));
+    }
+    if (alone >= 0) count = 1;
+    if (lane == 0) counts[w] = count;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t sum = 0;
+        for (int v = 0; v < kNearWaves; ++v) sum += counts[v];
+        first = atomicAdd(B.total, sum);
+    }
+    __syncthreads();
+    uint32_t base = first;
+    for (int v = 0; v < w; ++v) base += counts[v];
+    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+    if (lane == 0 && have) B.cells[cell] = make_uint2(base, count);
+    if (base + count > B.cap) return;  // no room: the caller reads the total
+    if (alone >= 0) {
+        if (lane == 0) entry(base, alone, B.disks[alone]);
+        return;
+    }
+    for (int i0 = 0; i0 < ndisks; i0 += 64) {
+        const int i = i0 + lane;
+        bool around = false;
+        const ArmDisk d = B.disks[i < ndisks ? i : 0];
+        const bool take = i < ndisks && near(d, &around);
+        const uint64_t m = __ballot(take);
+        if (take) entry(base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)), i, d);
+        base += (uint32_t)__popcll(m);
+    }
+}
+
+// Builds the lists; *more: they did not fit, call again with the *entries there
+// are.  near_n = 0 (no lists) for arms and disks outside the bounds'
+// assumptions, and for lists past kNearMaxEntries.
+static int build_near(mptg_ctx* ctx, const double* len, int nlinks, const double* disks, int ndisks,
+                      uint32_t* entries, bool* more) {
+    SceneDev& s = ctx->scene;
+    *more = false;
+    s.near_n = 0;
     double T = 0.0, longest = 0.0, rmax = 0.0;
     for (int i = 0; i < nlinks; ++i) {
-        if (!(len[i] >= 0.0) || !std::isfinite(len[i])) return;
+        if (!(len[i] >= 0.0) || !std::isfinite(len[i])) return MPTG_OK;
         T += len[i];
         longest = std::max(longest, len[i]);
     }
     for (int i = 0; i < ndisks; ++i) {
         const double* d = &disks[4 * (size_t)i];
-        if (!std::isfinite(d[0]) || !std::isfinite(d[1]) || !(d[3] >= 0.0) || !std::isfinite(d[3])) return;
+        if (!std::isfinite(d[0]) || !std::isfinite(d[1]) || !(d[3] >= 0.0) || !std::isfinite(d[3])) return MPTG_OK;
         rmax = std::max(rmax, d[3]);
     }
     // the FP32 squares stay clear of overflow and of denormals
-    if (!(T > kNearLeast) || !(T + rmax < kNearMost)) return;
-    auto margin = [&](const double* d) { return kNearMargin * (T + longest + d[3]); };
+    if (!(T > kNearLeast) || !(T + rmax < kNearMost)) return MPTG_OK;
     // cells half a link wide: the lists are then within a third of the
     // shortest possible, and 64 x 64 cells of the 20-link arm stay in L2
     const int n = std::max(1, std::min(kNearCells, (int)std::ceil(4.0 * T / longest)));
-    const double size = 2.0 * T / n;
-    cells->assign((size_t)n * n, make_uint2(0, 0));
-    auto visit = [&](auto&& take) {
-        for (int i = 0; i < ndisks; ++i) {
-            const double* d = &disks[4 * (size_t)i];
-            // the midpoint's error is a joint's; its cell coordinate's FP32
-            // rounding is within 1e-6 T; rounding here and in the exact
-            // expression is below 1e-12 r
-            const double reach = longest / 2 + d[3] + 2.0 * margin(d) + 8e-6 * T;
-            if (std::fabs(d[0]) > T + reach || std::fabs(d[1]) > T + reach) continue;
-            // (clamped before the cast: a disk may reach any number of cells past the square)
-            auto cell = [&](double v) { return (int)std::min(n - 1.0, std::max(0.0, std::floor((v + T) / size))); };
-            const int x0 = cell(d[0] - reach) - 1, x1 = cell(d[0] + reach) + 1;
-            const int y0 = cell(d[1] - reach) - 1, y1 = cell(d[1] + reach) + 1;
-            for (int y = std::max(0, y0); y <= std::min(n - 1, y1); ++y)
-                for (int x = std::max(0, x0); x <= std::min(n - 1, x1); ++x) {
-                    const double lx = -T + x * size, ly = -T + y * size;
-                    const double gx = std::max({lx - d[0], d[0] - (lx + size), 0.0});
-                    const double gy = std::max({ly - d[1], d[1] - (ly + size), 0.0});
-                    if (gx * gx + gy * gy <= reach * reach) take((size_t)y * n + x, i);
-                }
-        }
-    };
-    visit([&](size_t c, int) { (*cells)[c].y++; });
-    uint64_t total = 0;
-    for (uint2& c : *cells) {
-        c.x = (uint32_t)total;
-        total += c.y;
-        c.y = 0;
+    // room for 64 cells a disk at first, then for the entries there are
+    constexpr size_t kEntry = sizeof(float4) + sizeof(int32_t);
+    const size_t cells = 256, out = cells + sizeof(uint2) * kNearCells * kNearCells;
+    if (*entries > (uint32_t)kNearMaxEntries) return MPTG_OK;
+    uint32_t cap = std::max<uint32_t>(*entries, (uint32_t)std::min<int64_t>(kNearMaxEntries, std::max<int64_t>(1 << 12, (int64_t)ndisks * 64)));
+    if (s.near.bytes > out + kEntry * cap)
+        cap = (uint32_t)std::min<size_t>((s.near.bytes - out) / kEntry, (size_t)kNearMaxEntries);
+    const size_t ids = out + sizeof(float4) * (size_t)cap;
+    int rc;
+    if ((rc = ensure(ctx, s.near, ids + sizeof(int32_t) * (size_t)cap))) return rc;
+    char* p = (char*)s.near.p;
+    if ((rc = launch_zero_u32(ctx, (uint32_t*)p, 1))) return rc;
+    NearBuild B{(const ArmDisk*)s.arm_disks, ndisks, n, T, longest, cap, (uint32_t*)p,
+                (uint2*)(p + cells), (float4*)(p + out), (int32_t*)(p + ids)};
+    hipLaunchKernelGGL(near_lists, dim3((unsigned)((n * n + kNearWaves - 1) / kNearWaves)), dim3(64 * kNearWaves), 0,
+                       ctx->stream, B);
+    MPTG_HIP(ctx, hipGetLastError());
+    MPTG_HIP(ctx, hipMemcpyAsync(entries, p, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    MPTG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (*entries > cap) {
+        *more = true;
+        return MPTG_OK;
     }
-    if (total > (uint64_t)kNearMaxEntries) return;
-    out->assign((size_t)std::max<uint64_t>(total, 1), make_float4(0, 0, 0, 0));
-    ids->assign(out->size(), 0);
-    visit([&](size_t c, int i) {
-        const double* d = &disks[4 * (size_t)i];
-        const double lo = std::max(d[3] - margin(d), 0.0), hi = d[3] + margin(d);
-        const size_t at = (*cells)[c].x + (*cells)[c].y++;
-        (*ids)[at] = i;
-        (*out)[at] = make_float4((float)d[0], (float)d[1], std::nextafterf((float)(lo * lo), 0.0f),
-                                 std::nextafterf((float)(hi * hi), INFINITY));
-    });
-    sd->near_n = n;
-    sd->near_extent = (float)T;
-    sd->near_inv = (float)(n / (2.0 * T));
+    s.near_n = n;
+    s.near_extent = (float)T;
+    s.near_inv = (float)(n / (2.0 * T));
+    s.near_cells = B.cells;
+    s.near_disks = B.out;
+    s.near_ids = B.ids;
+    return MPTG_OK;
 }
 
 }  // namespace mptg
@@ -245,15 +321,9 @@ void mptg_destroy(mptg_ctx* ctx) {
     free_tree(ctx);
     (void)hipFree(ctx->scene.boxes);
     (void)hipFree(ctx->scene.grid);
-    (void)hipFree(ctx->scene.lengths);
-    (void)hipFree(ctx->scene.disks);
     (void)hipFree(ctx->scene.circles);
-    (void)hipFree(ctx->scene.arm_disks.p);
-    (void)hipFree(ctx->scene.arm_lim.p);
-    (void)hipFree(ctx->scene.arm_index.p);
-    (void)hipFree(ctx->scene.near_cells.p);
-    (void)hipFree(ctx->scene.near_disks.p);
-    (void)hipFree(ctx->scene.near_ids.p);
+    (void)hipFree(ctx->scene.arm.p);
+    (void)hipFree(ctx->scene.near.p);
     (void)hipFree(ctx->scene.mesh_nodes.p);
     (void)hipFree(ctx->scene.mesh_tris.p);
     (void)hipFree(ctx->scene.mesh_robot.p);
@@ -550,10 +620,6 @@ int mptg_scene_arm(mptg_ctx* ctx, const double* h_lengths, int nlinks, double ro
         dk[4 * i + 2] = rr * rr;
         dk[4 * i + 3] = rr;
     }
-    rc = upload(ctx, (void**)&ctx->scene.lengths, h_lengths, sizeof(double) * nlinks);
-    if (rc) return rc;
-    rc = upload(ctx, (void**)&ctx->scene.disks, dk.data(), sizeof(double) * 4 * ndisks);
-    if (rc) return rc;
     // kernel layout: [cx, cy, (r+R)^2, r+R] and a per-link segment-length
     // bound L (1 + 2^-30) + 1e-12 for the far-disk skip
     // then per group of kArmGroup links a bound on its half-length,
@@ -591,65 +657,56 @@ int mptg_scene_arm(mptg_ctx* ctx, const double* h_lengths, int nlinks, double ro
         gix = xmax > xmin ? (double)gnx / (xmax - xmin) : 0.0;
         giy = ymax > ymin ? (double)gny / (ymax - ymin) : 0.0;
     }
-    auto key = [&](size_t i) {
-        return arm_cell(ad[4 * i + 1], gy0, giy, gny) * gnx + arm_cell(ad[4 * i], gx0, gix, gnx);
-    };
-    {
-        std::vector<int> ord((size_t)ndisks);
-        for (int i = 0; i < ndisks; ++i) ord[(size_t)i] = i;
-        std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return key((size_t)x) < key((size_t)y); });
-        std::vector<double> sorted(ad.size(), 0.0);
-        for (int i = 0; i < ndisks; ++i)
-            for (int k = 0; k < 4; ++k) sorted[4 * (size_t)i + k] = ad[4 * (size_t)ord[(size_t)i] + k];
-        ad.swap(sorted);
-    }
     const int ncells = gnx * gny;
     std::vector<double> index(8 + (ncells + 1 + 1) / 2, 0.0);
+    index[0] = gx0;
+    index[1] = gy0;
+    index[2] = gix;
+    index[3] = giy;
+    index[4] = rtmax;
+    index[5] = gnx;
+    index[6] = gny;
     {
-        index[0] = gx0;
-        index[1] = gy0;
-        index[2] = gix;
-        index[3] = giy;
-        index[4] = rtmax;
-        index[5] = gnx;
-        index[6] = gny;
+        // counting sort by cell; starts[c]: the disks in cells below c
         int32_t* starts = reinterpret_cast<int32_t*>(index.data() + 8);
-        int j = 0;
-        for (int c = 0; c <= ncells; ++c) {
-            while (j < ndisks && key((size_t)j) < c) ++j;
-            starts[c] = j;
+        std::vector<int> key((size_t)ndisks);
+        for (int i = 0; i < ndisks; ++i) {
+            key[(size_t)i] = arm_cell(ad[4 * (size_t)i + 1], gy0, giy, gny) * gnx + arm_cell(ad[4 * (size_t)i], gx0, gix, gnx);
+            starts[key[(size_t)i] + 1]++;
         }
+        for (int c = 0; c < ncells; ++c) starts[c + 1] += starts[c];
+        std::vector<int> next(starts, starts + ncells);
+        std::vector<double> sorted(ad.size(), 0.0);
+        for (int i = 0; i < ndisks; ++i)
+            std::memcpy(&sorted[4 * (size_t)next[(size_t)key[(size_t)i]]++], &ad[4 * (size_t)i], 4 * sizeof(double));
+        ad.swap(sorted);
     }
-    if ((rc = ensure(ctx, ctx->scene.arm_index, sizeof(double) * index.size()))) return rc;
-    MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.arm_index.p, index.data(), sizeof(double) * index.size(),
-                                 hipMemcpyHostToDevice, ctx->stream));
     for (int i = 0; i < nlinks; ++i) lim[i] = h_lengths[i] * (1.0 + 0x1.0p-30) + 1e-12;
     for (int g = 0; g < ngroups; ++g) {
         double S = 0.0;
         for (int i = g * kGroup; i < (g + 1) * kGroup && i < nlinks; ++i) S += h_lengths[i];
         lim[nlinks + g] = S / 2 * (1.0 + 0x1.0p-30) + 1e-12;
     }
-    if ((rc = ensure(ctx, ctx->scene.arm_disks, sizeof(double) * ad.size()))) return rc;
-    if ((rc = ensure(ctx, ctx->scene.arm_lim, sizeof(double) * lim.size()))) return rc;
-    MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.arm_disks.p, ad.data(), sizeof(double) * ad.size(),
-                                 hipMemcpyHostToDevice, ctx->stream));
-    MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.arm_lim.p, lim.data(), sizeof(double) * lim.size(),
-                                 hipMemcpyHostToDevice, ctx->stream));
-    std::vector<uint2> cells;
-    std::vector<float4> near;
-    std::vector<int32_t> near_ids;
-    near_lists(h_lengths, nlinks, ad, ndisks, &ctx->scene, &cells, &near, &near_ids);
-    if (ctx->scene.near_n > 0) {
-        if ((rc = ensure(ctx, ctx->scene.near_cells, sizeof(uint2) * cells.size()))) return rc;
-        if ((rc = ensure(ctx, ctx->scene.near_disks, sizeof(float4) * near.size()))) return rc;
-        if ((rc = ensure(ctx, ctx->scene.near_ids, sizeof(int32_t) * near_ids.size()))) return rc;
-        MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.near_ids.p, near_ids.data(), sizeof(int32_t) * near_ids.size(),
-                                     hipMemcpyHostToDevice, ctx->stream));
-        MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.near_cells.p, cells.data(), sizeof(uint2) * cells.size(),
-                                     hipMemcpyHostToDevice, ctx->stream));
-        MPTG_HIP(ctx, hipMemcpyAsync(ctx->scene.near_disks.p, near.data(), sizeof(float4) * near.size(),
-                                     hipMemcpyHostToDevice, ctx->stream));
+    // one block, one copy (16-byte aligned pieces first)
+    std::vector<double> len(h_lengths, h_lengths + nlinks);
+    std::vector<double> all;
+    size_t at[5], k = 0;
+    for (const std::vector<double>* v : {&ad, &dk, &index, &lim, &len}) {
+        at[k++] = all.size();
+        all.insert(all.end(), v->begin(), v->end());
     }
+    MPTG_HIP(ctx, hipStreamSynchronize(ctx->stream));  // nothing reads the old scene any more
+    if ((rc = ensure(ctx, ctx->scene.arm, sizeof(double) * all.size()))) return rc;
+    double* base = (double*)ctx->scene.arm.p;
+    MPTG_HIP(ctx, hipMemcpyAsync(base, all.data(), sizeof(double) * all.size(), hipMemcpyHostToDevice, ctx->stream));
+    ctx->scene.arm_disks = base + at[0];
+    ctx->scene.disks = base + at[1];
+    ctx->scene.arm_index = base + at[2];
+    ctx->scene.arm_lim = base + at[3];
+    ctx->scene.lengths = base + at[4];
+    uint32_t entries = 0;
+    for (bool more = true; more;)
+        if ((rc = build_near(ctx, h_lengths, nlinks, ad.data(), ndisks, &entries, &more))) return rc;
     MPTG_HIP(ctx, hipStreamSynchronize(ctx->stream));
     ctx->scene.kind = MPTG_SCENE_ARM;
     ctx->valid_upto = 0;  // valid() changed: every node is checked again

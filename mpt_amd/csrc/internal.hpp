@@ -33,17 +33,21 @@ struct SceneDev {
     uint64_t* grid = nullptr;
     int width = 0, height = 0, grid_tx = 0;
     // arm
+    DevBuf arm;  // what the pointers below point into
     double* lengths = nullptr;
     int nlinks = 0;
     double robot_radius = 0;
     double* disks = nullptr;  // [cx, cy, (r+R)^2, r+R] per disk, reference order
     int ndisks = 0;
-    DevBuf arm_disks, arm_lim;  // kernel layout of the disks (ascending cx), per-link bounds
-    DevBuf arm_index;           // [xmin, 1/bucket width, max (r+R), 0] + int32 bucket starts
-    double total_length = 0;    // sum of link lengths (feature scale)
+    double *arm_disks = nullptr, *arm_lim = nullptr;  // the disks by grid cell, per-link bounds
+    double* arm_index = nullptr;                      // see ArmGrid
+    double total_length = 0;                          // sum of link lengths (feature scale)
     // FP32 clearance bounds: cells and disk lists (arm_near.hpp); near_n = 0:
     // the scene has none (every check is exact)
-    DevBuf near_cells, near_disks, near_ids;
+    DevBuf near;  // the entries' count, then the cells, disks and ids
+    const uint2* near_cells = nullptr;
+    const float4* near_disks = nullptr;
+    const int32_t* near_ids = nullptr;
     float near_extent = 0, near_inv = 0;
     int near_n = 0;
     // mesh (SE(3) rigid body): env BVH nodes, env triangles, robot triangles

@@ -91,9 +91,8 @@ inline SceneArgs scene_args(const mptg_ctx* ctx) {
     const SceneDev& s = ctx->scene;
     return SceneArgs{s.kind,    s.boxes,  s.nboxes, s.grid,   s.width,
                      s.height,  s.grid_tx, s.lengths, s.nlinks, s.disks, s.ndisks,
-                     (const ArmDisk*)s.arm_disks.p, (const double*)s.arm_lim.p, (const double*)s.arm_index.p,
-                     s.circles, s.ncircles, (const uint2*)s.near_cells.p, (const float4*)s.near_disks.p,
-                     (const int32_t*)s.near_ids.p, s.near_extent, s.near_inv, s.near_n};
+                     (const ArmDisk*)s.arm_disks, s.arm_lim, s.arm_index, s.circles, s.ncircles, s.near_cells,
+                     s.near_disks, s.near_ids, s.near_extent, s.near_inv, s.near_n};
 }
 
 __device__ __forceinline__ double so3_dist(const double* a, const double* b) {

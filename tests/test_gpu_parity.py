@@ -410,6 +410,35 @@ def test_arm_in_any_unit(ctx_factory, links, scale):
                 assert w["group"] > 0 and w["exact"] == 0, (wall, n, turn, w)
 
 
+def test_arm_uploads_in_a_row(ctx_factory):
+    """Scenes of many and few disks one after another in one context: lists
+    that outgrow their room, disks that lie around whole cells, lists past the
+    most that are kept, none.  Verdicts and counts equal the oracle's."""
+    _say("arm uploads in a row")
+    base = scenes.arm_scene(links=20, ndisks=5)
+    total = float(base.lengths.sum())
+    rng = np.random.default_rng(56)
+    ang = rng.uniform(0, 2 * math.pi, 6000)
+    ring = np.stack([np.cos(ang), np.sin(ang)], 1)
+    tiny = np.concatenate([rng.uniform(-total, total, (30000, 2)), np.full((30000, 1), 1e-3)], axis=1)
+    rim = np.concatenate([1.5 * total * ring, np.full((6000, 1), 1.5 * total - 12.0)], axis=1)  # a free core
+    one = np.repeat([[1.5 * total, 0.0, 1.4 * total]], 40000, axis=0)  # edge cells of 40 000 entries each
+    ctx = ctx_factory()
+    for name, disks, r in (("few", base.disks, 0.1), ("rim", rim, 0.0), ("tiny", tiny, 0.0), ("none", tiny[:0], 0.0),
+                           ("one", one, 0.0), ("few", base.disks, 0.1)):
+        sc = dataclasses.replace(base, disks=disks, robot_radius=r)
+        ctx.scene(sc)
+        o = oracle.Oracle(sc)
+        a = rng.uniform(-math.pi, math.pi, (200, 20))
+        a[:100] = np.where(np.arange(20) % 2, 3.1, 0.0)  # folded: within the core
+        a[:100, 0] = rng.uniform(-math.pi, math.pi, 100)
+        b = a + rng.uniform(-0.05, 0.05, a.shape)
+        assert np.array_equal(ctx.valid(a), o.valid(a)), name
+        gv, gc = ctx.link(a, b)
+        ov, oc = o.link(a, b, threads=16)
+        assert np.array_equal(gv, ov) and np.array_equal(gc, oc), name
+
+
 # ---- whole trees -------------------------------------------------------------
 def _planner_parity(ctx, sc, seed, batch, target, max_iters=1 << 30):
     ctx.scene(sc)
