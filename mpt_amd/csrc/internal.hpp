@@ -230,8 +230,9 @@ int check_device(mptg_ctx* ctx);
 double planner_coord_bound(const mptg_ctx* ctx);
 
 // Nearest neighbour (k = 1) of a batch in up to 8 dimensions (knn_one.hip);
-// n_dev, skip and nq_dev as for launch_knn.
-bool knn_one_applies(const mptg_ctx* ctx, int64_t nq, int64_t n);
+// n_dev, skip and nq_dev as for launch_knn.  Whether nq queries over n nodes take
+// it rather than the scan (q8: with its byte prefilter).
+bool knn_one_applies(const mptg_ctx* ctx, int64_t nq, int64_t n, bool q8);
 int knn_one_path(mptg_ctx* ctx, const double* d_q, int64_t nq, double radius, int32_t* d_idx, double* d_dist,
                  int64_t n, const int64_t* n_dev, const int32_t* skip, const uint32_t* nq_dev);
 

@@ -938,26 +938,27 @@ int knn_reserve(mptg_ctx* ctx, int64_t nq, int64_t tree_n) {
 static int knn_scan_path(mptg_ctx* ctx, const double* d_q, int64_t nq, double radius, int32_t* d_idx, double* d_dist,
                          int64_t tree_n, const int64_t* n_dev, const int32_t* skip,
                          const uint32_t* nq_dev = nullptr) {
-    if (knn_one_applies(ctx, nq, tree_n))
-        return knn_one_path(ctx, d_q, nq, radius, d_idx, d_dist, tree_n, n_dev, skip, nq_dev);
     // with n_dev, tree_n is only the size the split count is planned for;
     // with nq_dev (live queries on the device) the split is planned for half
     // of the nq slots
     int64_t n = tree_n, chunk;
     const int64_t splits = plan_splits(ctx, nq_dev ? (nq + 1) / 2 : nq, n, &chunk);
+    // a seed bound pays off when the tree is split many ways: every chunk
+    // starts from it
+    const bool seeded = splits >= 8 && ctx->metric != MPTG_METRIC_SE3;
+    // L1 in 8 or more dimensions: the byte prefilter
+    const bool q8 = seeded && ctx->metric == MPTG_METRIC_L1 && ctx->dim >= 8 && ctx->tune.knn_q8 &&
+                    ctx->coord_bound > 0 && ctx->coord_bound < 1e300;
+    if (knn_one_applies(ctx, nq, n, q8))
+        return knn_one_path(ctx, d_q, nq, radius, d_idx, d_dist, tree_n, n_dev, skip, nq_dev);
     int rc;
     if ((rc = ensure(ctx, ctx->scratch[4], sizeof(double) * nq * splits))) return rc;
     if ((rc = ensure(ctx, ctx->scratch[5], sizeof(int32_t) * nq * splits))) return rc;
-    // a seed bound pays off when the tree is split many ways: every chunk
-    // starts from it
     double* seed = nullptr;
-    if (splits >= 8 && ctx->metric != MPTG_METRIC_SE3) {
+    if (seeded) {
         if ((rc = ensure(ctx, ctx->scratch[3], sizeof(double) * nq))) return rc;
         seed = (double*)ctx->scratch[3].p;
     }
-    // L1 in 8 or more dimensions: the byte prefilter
-    const bool q8 = seed && ctx->metric == MPTG_METRIC_L1 && ctx->dim >= 8 && ctx->tune.knn_q8 &&
-                    ctx->coord_bound > 0 && ctx->coord_bound < 1e300;
     // the byte prefilter's blocks (4 waves, 4 resident per CU) re-split on
     // the device to one full round for the live queries
     const int64_t q8_target = q8 ? (int64_t)ctx->cus * kQ8BlocksPerCu : 0;

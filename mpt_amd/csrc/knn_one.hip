@@ -316,11 +316,27 @@ constexpr int one_queries() {
 // A block goes through the whole tree (0.45 us per 1000 nodes in two
 // dimensions, 0.6 in seven), so few queries over a large tree take the scan,
 // which splits it: at 65 000 nodes one query takes 24 us here and 36 there, at
-// 10^6 450 and 101.  From 32 queries per CU on every block is resident and the
-// scan no faster at any size (8192 queries, 10^6 nodes: 1585 and 1711 us).
-bool knn_one_applies(const mptg_ctx* ctx, int64_t nq, int64_t n) {
-    return ctx->dim >= 1 && ctx->dim <= 8 && (ctx->metric == MPTG_METRIC_L1 || ctx->metric == MPTG_METRIC_L2) &&
-           nq > 0 && nq < ((int64_t)1 << 31) && (n <= (int64_t)1 << 16 || nq >= (int64_t)ctx->cus * 32);
+// 10^6 450 and 101.  From 32 queries per CU on every block is resident, and
+// the line depends on how much of a row it reads is padding, which the scan
+// does not compare: in 2 to 4, 7 and 8 dimensions the scan gains on it slowly
+// (8192 queries, L2: 0.24 ms there, 0.12 here in R^2 at 70 000, 1.72 and 1.57
+// at 10^6; L1: 0.49 and 0.45 at 300 000, 1.28 and 1.43 at 10^6), with 5 or 6
+// of 8 coordinates sooner (L2: 0.91 and 0.93 at 300 000; L1: 0.30 both at
+// 100 000, 0.37 and 0.41 at 131 072), on the line too (0.20 and 0.14 ms at
+// 100 000, 0.34 and 0.46 at 200 000).
+// The byte prefilter of L1 in 8 dimensions (q8: the scan would use it) tests a
+// pair in 2 instructions, not 20, behind two more launches: 8192 queries
+// over 16 000 nodes 49 us, here 63; 1024 over 65 000 47 and 61; 16 384 over 500
+// 21 and 26; but 4096 over 8000 27 and 20, 256 over 65 000 78 and 34.
+bool knn_one_applies(const mptg_ctx* ctx, int64_t nq, int64_t n, bool q8) {
+    const bool l2 = ctx->metric == MPTG_METRIC_L2;
+    if (ctx->dim < 1 || ctx->dim > 8 || (ctx->metric != MPTG_METRIC_L1 && !l2)) return false;
+    if (nq <= 0 || nq >= ((int64_t)1 << 31)) return false;
+    if (n <= (int64_t)1 << 16) return !(q8 && (nq >= (int64_t)ctx->cus * 64 || nq * n >= (int64_t)1 << 25));
+    if (q8 || nq < (int64_t)ctx->cus * 32) return false;
+    if (ctx->dim == 1) return n <= 100000;
+    if (ctx->dim == 5 || ctx->dim == 6) return n <= (l2 ? (int64_t)1 << 18 : 100000);
+    return n <= (l2 ? (int64_t)1 << 20 : (int64_t)1 << 19);
 }
 
 int knn_one_path(mptg_ctx* ctx, const double* d_q, int64_t nq, double radius, int32_t* d_idx, double* d_dist,

@@ -168,9 +168,9 @@ def test_default_prrt_star_grows_1e5_nodes_in_se3(ctx_factory):
     assert st["rewires"] > 0
 
 
-# wave lists (knn_wave.hip): rows shorter than a wave, one row either side of
-# a wave's 64 nodes, the tree sizes where a query gets 4 and 16 waves, and
-# enough queries (an odd count) for four per wave
+# k = 1 (knn_one.hip): trees of less than a block's rows and one row either
+# side of them, odd counts of queries for 1, 4, 8 and 16 per block, a larger
+# tree that few queries leave to the scan
 @pytest.mark.parametrize("scale", [1.0, 1e25], ids=["plain", "beyond-fp32-squares"])
 @pytest.mark.parametrize("metric,dim,n,nq", [
     (scenes.METRIC_L2, 1, 1, 1), (scenes.METRIC_L1, 2, 255, 7), (scenes.METRIC_L2, 2, 256, 1023),
@@ -198,6 +198,47 @@ def test_knn_nearest_equals_oracle(ctx_factory, metric, dim, n, nq, scale):
         assert np.array_equal(gi[some], oi) and np.array_equal(gd[some], od), radius
 
 
+@pytest.mark.parametrize("metric,dim,n,nq", [
+    (scenes.METRIC_L1, 8, 700, 16385), (scenes.METRIC_L1, 8, 2050, 16383), (scenes.METRIC_L1, 8, 40001, 841),
+    (scenes.METRIC_L1, 8, 65537, 8193), (scenes.METRIC_L2, 8, 65537, 8193), (scenes.METRIC_L2, 1, 100001, 8193),
+    (scenes.METRIC_L1, 5, 100001, 8193), (scenes.METRIC_L1, 3, 131073, 8193), (scenes.METRIC_L2, 6, 262145, 8193),
+    (scenes.METRIC_L1, 20, 30001, 1025),
+])
+@pytest.mark.parametrize("spread", [1.0, 1.3], ids=["inside", "beyond-the-tree"])
+def test_knn_nearest_routes_agree(ctx_factory, metric, dim, n, nq, spread):
+    """k = 1 on both sides of the lines between a block per query and the
+    scans (with and without the byte prefilter): the same ids and distances,
+    the oracle's.  Queries a little and far outside the tree's box, where the
+    byte rows are clamped, and past where they are used."""
+    _say("knn nearest routes", metric, dim, n, nq, spread)
+    ctx = ctx_factory()
+    rng = np.random.default_rng(dim * 1000 + n)
+    pts = rng.uniform(-2, 2, (n, dim))
+    pts[n // 2:n // 2 + 3] = pts[0]
+    q = rng.uniform(-1.9 * spread, 1.9 * spread, (nq, dim))
+    if spread > 1.0:
+        for i, far in enumerate((1.1, 3.0, 1e3, 2.0 ** 19, 2.0 ** 22, 1e17)):
+            q[1 + i] *= far
+            q[100 + i, dim - 1] *= far  # one coordinate alone
+    q[0] = pts[0]
+    ctx.space(metric, dim)
+    ctx.tree_insert(pts)
+    o = oracle.Oracle(_plain(metric, dim))
+    some = np.unique(np.concatenate([np.arange(7), np.arange(100, 106), [nq - 1], rng.integers(0, nq, 100)]))
+    oi, od = o.knn(pts, q[some], 1, radius=math.inf, threads=8)
+    got = []
+    for q8 in (1, 0):
+        ctx.tune_set(knn_grid=0, knn_q8=q8)
+        got.append(ctx.knn(q, 1))
+        assert np.array_equal(got[-1][0][some], oi) and np.array_equal(got[-1][1][some], od), q8
+    few = ctx.knn(q[:300], 1)
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    assert np.array_equal(got[0][0][:300], few[0]) and np.array_equal(got[0][1][:300], few[1])
+
+
+# wave lists (knn_wave.hip): rows shorter than a wave, one row either side of
+# a wave's 64 nodes, the tree sizes where a query gets 4 and 16 waves, and
+# enough queries (an odd count) for four per wave
 @pytest.mark.parametrize("metric,dim,k,n,nq", [
     (scenes.METRIC_L2, 2, 2, 1, 3), (scenes.METRIC_L2, 2, 20, 63, 100), (scenes.METRIC_L1, 3, 64, 64, 70),
     (scenes.METRIC_L2, 7, 64, 65, 70), (scenes.METRIC_L1, 1, 5, 1023, 64), (scenes.METRIC_L2, 12, 33, 1024, 1),
