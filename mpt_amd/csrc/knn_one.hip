@@ -10,7 +10,9 @@
 // node exactly.  Where a lane's second smallest is under it too (nodes on a
 // small circle seen from afar, as a tree of limited range begins, or a goal
 // sampled often), one more pass over the rows lists those queries' pairs, and
-// the block measures the list.  (A lane per query over broadcast rows, chunk by
+// the block measures the list; past the list's end each lane measures its rows'
+// pairs as it meets them (a query at a time over all rows, 8192 queries and
+// 3000 nodes at 8 points took 176 us, 72 now; 66 in the scan).  (A lane per query over broadcast rows, chunk by
 // chunk of the tree, took a list, a branch per four nodes, a seed bound and a
 // merge, three launches: 256 queries and 2000 nodes of R^2 19.7 us then, 5.2
 // now; 8192 and 16 000 93 and 39; 65 536 and 65 000 1050 and 800.)
@@ -170,6 +172,9 @@ __global__ __launch_bounds__(kOneBlock) void knn_one(const double* __restrict__ 
                          ? __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(thr_s[c])))
                          : -1.0f;
         for (int64_t j0 = 0; j0 < n; j0 += kOneBlock * U) {
+            if (__builtin_amdgcn_readfirstlane(
+                    __hip_atomic_load(&ncand, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) > kOneCand)
+                break;  // too many already
             OneRow<D> row[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -193,7 +198,7 @@ __global__ __launch_bounds__(kOneBlock) void knn_one(const double* __restrict__ 
         }
         __syncthreads();
         const int found = ncand;
-        listed = found <= kOneCand;  // (else lane by lane below)
+        listed = found <= kOneCand;
         if (listed) {
             auto exact = [&](int i) {
                 return exact_dist<D, METRIC>(q + (q0 + cand_c[i]) * D, x64 + (int64_t)cand_j[i] * D);
@@ -209,52 +214,79 @@ __global__ __launch_bounds__(kOneBlock) void knn_one(const double* __restrict__ 
                     const double d = exact(i);
                     if (d <= radius && bits_of(d) == near_d[cand_c[i]]) atomicMin(&near_i[cand_c[i]], (int)cand_j[i]);
                 }
-        }
-    }
+        } else {
+            // More pairs than the list holds (many nodes at one place): a
+            // lane measures the pairs of its rows as it meets them.  Its rows
+            // come by ascending id, so none past a node at the query itself.
+            double bd[Q];
+            int32_t bi[Q];
 #pragma unroll
-    for (int c = 0; c < Q; ++c) {
-        if (listed && ((crowd >> c) & 1u)) continue;
-        const float thr = thr_s[c];
-        const double* qc = q + (q0 + c < live ? q0 + c : live - 1) * D;
-        double bd = inf;
-        int32_t bi = INT_MAX;
-        // (a threshold of +inf: values that FP32 cannot hold, or no node)
-        if (second[c] <= thr) {
-            // Several nodes at one place, as a goal sampled often leaves
-            // them: rows and coordinates some at a time, and none past a node
-            // at the query itself (the lane's nodes come by ascending id).
-            constexpr int R = D <= 2 ? 8 : 4;
-            for (int64_t j0 = t; j0 < n && !(bd == 0.0); j0 += R * kOneBlock) {
-                float a[R];
-#pragma unroll
-                for (int u = 0; u < R; ++u) {
-                    const int64_t j = j0 + u * kOneBlock;
-                    OneRow<D> row;
-                    row.load(x32, j < n ? j : 0);
-                    a[u] = j < n ? one_value<D, METRIC>(qv[c], row.v) : finf;
-                }
+            for (int c = 0; c < Q; ++c) {
+                bd[c] = inf;
+                bi[c] = INT_MAX;
+            }
+            uint32_t open = crowd;
+            constexpr int R = Q == 1 ? 4 : Q == 4 ? 2 : 1;  // rows in flight
+            for (int64_t j0 = t; j0 < n && open; j0 += kOneBlock * R) {
+                OneRow<D> row[R];
                 double x[R][D];
+                uint32_t in[R];
+#pragma unroll
+                for (int u = 0; u < R; ++u) row[u].load(x32, j0 + u * kOneBlock < n ? j0 + u * kOneBlock : 0);
 #pragma unroll
                 for (int u = 0; u < R; ++u) {
-                    const int64_t j = j0 + u * kOneBlock;
-                    if (j < n && a[u] <= thr) {
+                    in[u] = 0;
 #pragma unroll
-                        for (int i = 0; i < D; ++i) x[u][i] = x64[j * D + i];
+                    for (int c = 0; c < Q; ++c) in[u] |= (one_value<D, METRIC>(qv[c], row[u].v) <= lim[c] ? 1u : 0u) << c;
+                    in[u] = j0 + u * kOneBlock < n ? in[u] & open : 0u;
+                    if (in[u]) {
+#pragma unroll
+                        for (int i = 0; i < D; ++i) x[u][i] = x64[(j0 + u * kOneBlock) * D + i];
                     }
                 }
 #pragma unroll
                 for (int u = 0; u < R; ++u) {
-                    const int64_t j = j0 + u * kOneBlock;
-                    if (j < n && a[u] <= thr) {
-                        const double d = exact_dist<D, METRIC>(qc, x[u]);
-                        if (d <= radius && one_better(d, (int32_t)j, bd, bi)) {
-                            bd = d;
-                            bi = (int32_t)j;
+#pragma unroll
+                    for (int c = 0; c < Q; ++c) {
+                        if (!((in[u] & open) >> c & 1u)) continue;
+                        const double d = exact_dist<D, METRIC>(q + (q0 + c < live ? q0 + c : live - 1) * D, x[u]);
+                        if (d <= radius && d < bd[c]) {
+                            bd[c] = d;
+                            bi[c] = (int32_t)(j0 + u * kOneBlock);
+                            open &= ~((d == 0.0 ? 1u : 0u) << c);
                         }
                     }
                 }
             }
-        } else if (low[c] <= thr) {
+#pragma unroll
+            for (int c = 0; c < Q; ++c) {
+                if (!((crowd >> c) & 1u)) continue;  // uniform
+                double wd = bd[c];
+                int32_t wi = bi[c];
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) {
+                    const double d = __shfl_xor(wd, o);
+                    const int32_t i = __shfl_xor(wi, o);
+                    if (one_better(d, i, wd, wi)) {
+                        wd = d;
+                        wi = i;
+                    }
+                }
+                if (lane == 0) {
+                    best_d[wid][c] = wd;
+                    best_i[wid][c] = wi;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < Q; ++c) {
+        if ((crowd >> c) & 1u) continue;
+        const float thr = thr_s[c];
+        const double* qc = q + (q0 + c < live ? q0 + c : live - 1) * D;
+        double bd = inf;
+        int32_t bi = INT_MAX;
+        if (low[c] <= thr) {  // (a threshold of +inf comes with a crowd)
             const double d = exact_dist<D, METRIC>(qc, x64 + (int64_t)at[c] * D);
             if (d <= radius) {
                 bd = d;
@@ -327,12 +359,14 @@ constexpr int one_queries() {
 // The byte prefilter of L1 in 8 dimensions (q8: the scan would use it) tests a
 // pair in 2 instructions, not 20, behind two more launches: 8192 queries
 // over 16 000 nodes 49 us, here 63; 1024 over 65 000 47 and 61; 16 384 over 500
-// 21 and 26; but 4096 over 8000 27 and 20, 256 over 65 000 78 and 34.
+// 21 and 26; but 2000 over 20 000 32 and 24, 256 over 65 000 78 and 34.  (Its
+// bytes tell nothing apart in a tree that fills a thousandth of its box: 8192
+// over 65 000 such nodes 1.4 ms, here 0.2.)
 bool knn_one_applies(const mptg_ctx* ctx, int64_t nq, int64_t n, bool q8) {
     const bool l2 = ctx->metric == MPTG_METRIC_L2;
     if (ctx->dim < 1 || ctx->dim > 8 || (ctx->metric != MPTG_METRIC_L1 && !l2)) return false;
     if (nq <= 0 || nq >= ((int64_t)1 << 31)) return false;
-    if (n <= (int64_t)1 << 16) return !(q8 && (nq >= (int64_t)ctx->cus * 64 || nq * n >= (int64_t)1 << 25));
+    if (n <= (int64_t)1 << 16) return !(q8 && (nq >= (int64_t)ctx->cus * 64 || nq * n >= (int64_t)3 << 24));
     if (q8 || nq < (int64_t)ctx->cus * 32) return false;
     if (ctx->dim == 1) return n <= 100000;
     if (ctx->dim == 5 || ctx->dim == 6) return n <= (l2 ? (int64_t)1 << 18 : 100000);

@@ -236,6 +236,30 @@ def test_knn_nearest_routes_agree(ctx_factory, metric, dim, n, nq, spread):
     assert np.array_equal(got[0][0][:300], few[0]) and np.array_equal(got[0][1][:300], few[1])
 
 
+@pytest.mark.parametrize("metric,dim", [(scenes.METRIC_L2, 1), (scenes.METRIC_L2, 2), (scenes.METRIC_L1, 3),
+                                        (scenes.METRIC_L2, 7), (scenes.METRIC_L1, 8)])
+@pytest.mark.parametrize("nq", [3, 1025, 4099])
+@pytest.mark.parametrize("places", [1, 9, 4000])
+def test_knn_nearest_of_many_at_one_place(ctx_factory, metric, dim, nq, places):
+    """Thousands of nodes at a few points, more pairs under the threshold than
+    a block lists: the lowest id of the nearest point, the oracle's, for
+    queries at the points, beside them and out of the radius."""
+    _say("knn crowded", metric, dim, nq, places)
+    ctx = ctx_factory()
+    rng = np.random.default_rng(dim + places)
+    n = 5003
+    pts = rng.uniform(-2, 2, (places, dim))[rng.integers(0, places, n)]
+    q = rng.uniform(-2.5, 2.5, (nq, dim))
+    q[::5] = pts[rng.integers(0, n, len(q[::5]))]
+    ctx.space(metric, dim)
+    ctx.tree_insert(pts)
+    o = oracle.Oracle(_plain(metric, dim))
+    for radius in (math.inf, 0.3, 0.0):
+        gi, gd = ctx.knn(q, 1, radius=radius)
+        oi, od = o.knn(pts, q, 1, radius=radius, threads=8)
+        assert np.array_equal(gi, oi) and np.array_equal(gd, od), radius
+
+
 # wave lists (knn_wave.hip): rows shorter than a wave, one row either side of
 # a wave's 64 nodes, the tree sizes where a query gets 4 and 16 waves, and
 # enough queries (an odd count) for four per wave
