@@ -181,24 +181,25 @@ static_assert(sizeof(MeshNode16) == 512, "sixteen-wide node is 512 bytes");
 int collapse16(const std::vector<MeshNode>& n2, int id, std::vector<MeshNode16>& out) {
     const int me = (int)out.size();
     out.push_back(MeshNode16{});
-    std::vector<int> slot{id};
+    int slot[kWide] = {id}, above[kWide], n = 1;
     for (int level = 0; level <= kWideLevels; ++level) {  // the last one as far as there is room
-        const std::vector<int> above = slot;
-        slot.clear();
-        for (size_t i = 0; i < above.size(); ++i) {
-            const MeshNode& g = n2[above[i]];
-            if (g.b > 0 && slot.size() + (above.size() - i) < (size_t)kWide) {
-                slot.push_back(g.a);
-                slot.push_back(g.b);
+        const int m = n;
+        std::copy(slot, slot + m, above);
+        n = 0;
+        for (int i = 0; i < m; ++i) {
+            const MeshNode& g = n2[(size_t)above[i]];
+            if (g.b > 0 && n + (m - i) < kWide) {
+                slot[n++] = g.a;
+                slot[n++] = g.b;
             } else {
-                slot.push_back(above[i]);
+                slot[n++] = above[i];
             }
         }
     }
     MeshNode16 node;
     for (MeshSlot& o : node.slot) o = {{INFINITY, INFINITY, INFINITY}, 0, {-INFINITY, -INFINITY, -INFINITY}, 0};
-    for (size_t k = 0; k < slot.size(); ++k) {
-        const MeshNode& g = n2[slot[k]];
+    for (int k = 0; k < n; ++k) {
+        const MeshNode& g = n2[(size_t)slot[k]];
         MeshSlot& o = node.slot[k];
         for (int i = 0; i < 3; ++i) {
             o.lo[i] = g.lo[i];
@@ -881,10 +882,13 @@ extern "C" int mptg_scene_mesh(mptg_ctx* ctx, const float* h_robot, int nrobot, 
         return fail(ctx, MPTG_E_ARG, "bad mesh arrays");
     if (nenv > (1 << 20)) return fail(ctx, MPTG_E_RANGE, "at most 2^20 environment triangles");
     if (nrobot > (1 << 16)) return fail(ctx, MPTG_E_RANGE, "at most 2^16 robot triangles");
-    for (int64_t i = 0; i < (int64_t)nrobot * 9; ++i)
-        if (!std::isfinite(h_robot[i])) return fail(ctx, MPTG_E_ARG, "non-finite robot vertex");
-    for (int64_t i = 0; i < (int64_t)nenv * 9; ++i)
-        if (!std::isfinite(h_env[i])) return fail(ctx, MPTG_E_ARG, "non-finite environment vertex");
+    auto finite = [](const float* v, int64_t n) {  // without a branch per value
+        int bad = 0;
+        for (int64_t i = 0; i < n; ++i) bad |= !(std::fabs(v[i]) < INFINITY);
+        return !bad;
+    };
+    if (!finite(h_robot, (int64_t)nrobot * 9)) return fail(ctx, MPTG_E_ARG, "non-finite robot vertex");
+    if (!finite(h_env, (int64_t)nenv * 9)) return fail(ctx, MPTG_E_ARG, "non-finite environment vertex");
     // environment BVH
     BvhBuilder bb;
     bb.refs.resize((size_t)nenv);
@@ -894,6 +898,7 @@ extern "C" int mptg_scene_mesh(mptg_ctx* ctx, const float* h_robot, int nrobot, 
         for (int i = 0; i < 3; ++i) r.c[i] = 0.5f * (r.lo[i] + r.hi[i]);
         r.id = t;
     }
+    bb.nodes.reserve((size_t)nenv + 1);
     if (nenv > 0) bb.build(0, nenv, 0);
     if (nenv > 0 && bvh_depth(bb.nodes, 0, 0) > kBuildDepth)
         return fail(ctx, MPTG_E_STATE, "environment BVH deeper than the traversal stack");
@@ -942,22 +947,19 @@ extern "C" int mptg_scene_mesh(mptg_ctx* ctx, const float* h_robot, int nrobot, 
     for (int g = 0; g < ngroup; ++g) {
         const int t1 = std::min(nrobot, (g + 1) << sh);
         float* o = &robot[group_offset(nrobot) + 8 * (size_t)g];
+        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        for (int v = 3 * (g << sh); v < 3 * t1; ++v) BvhBuilder::grow(lo, hi, &robot[3 * (size_t)v], &robot[3 * (size_t)v]);
         for (int i = 0; i < 3; ++i) {
-            float lo = INFINITY, hi = -INFINITY;
-            for (int v = 3 * (g << sh); v < 3 * t1; ++v) {
-                const float x = robot[(size_t)v * 3 + i];
-                lo = std::min(lo, x);
-                hi = std::max(hi, x);
-                reach = std::max(reach, std::fabs(x));
-            }
-            const float c = 0.5f * lo + 0.5f * hi;
+            reach = std::max({reach, std::fabs(lo[i]), std::fabs(hi[i])});
+            const float c = 0.5f * lo[i] + 0.5f * hi[i];
             o[i] = c;
-            o[4 + i] = std::nextafter(std::max(hi - c, c - lo), INFINITY);
+            o[4 + i] = std::nextafter(std::max(hi[i] - c, c - lo[i]), INFINITY);
         }
     }
     SceneDev& s = ctx->scene;
     MPTG_HIP(ctx, hipStreamSynchronize(ctx->stream));
     std::vector<MeshNode16> wide;
+    wide.reserve(bb.nodes.size() / 8 + 1);
     if (!bb.nodes.empty()) collapse16(bb.nodes, 0, wide);
     if ((rc = ensure(ctx, s.mesh_nodes, sizeof(MeshNode16) * std::max<size_t>(1, wide.size())))) return rc;
     if ((rc = ensure(ctx, s.mesh_tris, sizeof(float) * std::max<size_t>(16, tris.size())))) return rc;
@@ -973,7 +975,9 @@ extern "C" int mptg_scene_mesh(mptg_ctx* ctx, const float* h_robot, int nrobot, 
     s.mesh_nrobot = nrobot;
     s.mesh_reach = reach;
     s.mesh_env_reach = 0;
-    for (int64_t i = 0; i < (int64_t)nenv * 9; ++i) s.mesh_env_reach = std::max(s.mesh_env_reach, std::fabs(h_env[i]));
+    if (!bb.nodes.empty())
+        for (int i = 0; i < 3; ++i)
+            s.mesh_env_reach = std::max({s.mesh_env_reach, std::fabs(bb.nodes[0].lo[i]), std::fabs(bb.nodes[0].hi[i])});
     s.kind = MPTG_SCENE_MESH;
     ctx->valid_upto = 0;  // valid() changed: every node is checked again
     ctx->some_invalid = false;
