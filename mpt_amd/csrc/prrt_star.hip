@@ -596,6 +596,13 @@ struct WalkTree {
     uint16_t *parent, *child, *next, *prev, *queue;
 };
 
+// What a lane of the wave has stored to LDS before it, every lane reads after it.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 struct WalkPair {  // a lane's pair of the list
     int32_t e, nb, j;
     double d;
@@ -780,6 +787,7 @@ __global__ __launch_bounds__(1024) void star_rewire_lds(int D, int k, int total,
                         }
                         tail += __popcll(b);
                     }
+                    wave_lds_sync();  // queue, costs and low of this level, to every lane
                     if (bad || head == tail) break;
                     const int take = min(64, tail - head);
                     c = lane < take ? (int)T.child[T.queue[head + lane]] : kNoNode;
