@@ -7,8 +7,10 @@ equal the oracle's whatever the number of iterations per launch, also when
 the stop falls inside a captured span.  Each run call captures afresh and
 replays its graph several times, with host synchronisations and counter
 reads between the launches.  Every link path is covered: boxes (per-edge
-bisection), the grid (DMV short and long lists), the arm (wave kernels with
-their zero-filled continuation counters) and the triangle meshes."""
+bisection), the grid (DMV short and long lists), the arm (its lists and their
+counters) and the triangle meshes.  Also link() recorded by the stream's
+owner."""
+import ctypes as C
 import dataclasses
 import sys
 
@@ -169,3 +171,79 @@ def test_graph_reused_across_runs(ctx_factory):
             assert np.array_equal(gn, on) and np.array_equal(gp, op)
             for key in STAT_KEYS:
                 assert st[key] == ost[key], key
+
+
+class _StreamCapture:
+    """Graph capture of a context's stream by its owner, through the HIP
+    runtime that the library itself has loaded."""
+
+    def __init__(self, ctx):
+        with open("/proc/self/maps") as f:
+            path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+        self.hip, self.stream = C.CDLL(path), C.c_void_p(ctx.stream)
+
+    def _ok(self, rc):
+        assert rc == 0, rc
+
+    def record(self, fn):
+        graph, self.exe = C.c_void_p(), C.c_void_p()
+        self._ok(self.hip.hipStreamBeginCapture(self.stream, 2))  # relaxed: allocations are allowed
+        try:
+            fn()
+        finally:
+            self._ok(self.hip.hipStreamEndCapture(self.stream, C.byref(graph)))
+        self._ok(self.hip.hipGraphInstantiate(C.byref(self.exe), graph, None, None, C.c_size_t(0)))
+        self._ok(self.hip.hipGraphDestroy(graph))
+
+    def replay(self):
+        self._ok(self.hip.hipGraphLaunch(self.exe, self.stream))
+
+    def free(self):
+        self._ok(self.hip.hipGraphExecDestroy(self.exe))
+
+
+@pytest.mark.parametrize("kind,fresh", [("arm", True), ("arm", False), ("mesh", False), ("grid", False)])
+def test_link_captured_by_the_streams_owner(ctx_factory, kind, fresh):
+    """A link() call recorded into the owner's graph -- as the context's first
+    one (the lists it needs are allocated and cleared in the recording alone)
+    or after others -- then eager calls and replays in turn: every one gives
+    the oracle's verdicts and counts."""
+    _say("captured link", kind, fresh)
+    sc = {"arm": lambda: scenes.arm_scene(links=20, ndisks=200), "mesh": lambda: scenes.se3_scene(6000, 120),
+          "grid": lambda: scenes.grid_scene(size=512)}[kind]()
+    rng = np.random.default_rng(61)
+    n = 2200
+    a = rng.uniform(sc.lo, sc.hi, (n, sc.dim))
+    if kind == "mesh":
+        a[:, :4] = rng.normal(size=(n, 4))
+        a[:, :4] /= np.linalg.norm(a[:, :4], axis=1, keepdims=True)
+    b = a + rng.uniform(-0.05, 0.05, a.shape) * (sc.hi - sc.lo) * (np.arange(sc.dim) >= (4 if kind == "mesh" else 0))
+    b[::50] = a[::50] + (a[::50] - sc.lo) * 0.5 * (np.arange(sc.dim) >= (4 if kind == "mesh" else 0))
+    ov, oc = oracle.Oracle(sc).link(a, b, threads=16)
+    ctx = ctx_factory()
+    ctx.scene(sc)
+    da, db = ctx.to_device(a), ctx.to_device(b)
+    v, c = ctx.array(n, np.uint8), ctx.array(n, np.uint32)
+
+    def check(call, m):
+        v.zero()
+        c.zero()
+        call()
+        ctx.sync()
+        assert np.array_equal(v.numpy()[:m].astype(bool), ov[:m]) and np.array_equal(c.numpy()[:m], oc[:m])
+
+    def eager(m):
+        return lambda: ctx.link_dev(da.ptr, db.ptr, m, 0, False, v.ptr, c.ptr)
+
+    if not fresh:
+        check(eager(n), n)
+    cap = _StreamCapture(ctx)
+    cap.record(eager(n))
+    try:
+        for m in (n, 100, n):
+            check(eager(m), m)
+            check(cap.replay, n)
+            check(cap.replay, n)
+    finally:
+        ctx.sync()
+        cap.free()
