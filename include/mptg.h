@@ -343,7 +343,8 @@ int mptg_diag_math(mptg_ctx* ctx, int op, const double* h_x, int64_t n, double* 
    Launch shapes the device kernels take from the context.  None of them
    changes a result: they only split the same work differently. */
 typedef struct mptg_tune_params {
-    int32_t knn_blocks_per_cu;      /* kNN scan blocks per CU the tree split aims at (1..256) */
+    int32_t knn_blocks_per_cu;      /* kNN scan blocks per CU the tree split aims at (1..256):
+                                       k = 1 and the select path; others split by their own rule */
     int32_t dmv_long_waves_per_cu;  /* grid of the persistent DMV long-edge kernel (1..256) */
     int32_t mesh_waves_per_cu;      /* grid of the persistent mesh kernels (1..256) */
     int32_t arm_tail_waves;         /* kept for callers that set it (1..8); the arm link kernels
@@ -351,12 +352,13 @@ typedef struct mptg_tune_params {
     int32_t arm_cull;               /* likewise (0 or 1) */
     int32_t mesh_edge_waves;        /* kept likewise (1..32): a mesh edge's waypoints go to any wave */
     int32_t knn_select;             /* k > 1 on trees of 2^16 nodes or more: 1 bound, collect and
-                                       select (registers of k = 1 in the scan), 0 the k-list scan */
+                                       select (registers of k = 1 in the scan), 0 the wave lists */
     int32_t knn_grid;               /* L1/L2 in 2..8 dimensions on trees of 2^16 nodes or more: 1 a
                                        uniform grid built per call, searched cell by cell; 0 the scans */
     int32_t dmv_edge_lanes;         /* DMV link: lanes sharing one edge's checks (1, 2, 4, .., 64) */
     int32_t knn_q8;                 /* k = 1 under L1 in 8 or more dimensions: 1 a byte prefilter
-                                       (four coordinates per sum-of-absolute-differences), 0 FP32 */
+                                       (four coordinates per sum-of-absolute-differences; in 8
+                                       dimensions where the batch is large enough), 0 FP32 */
 } mptg_tune_params;
 
 enum {
@@ -388,20 +390,24 @@ int mptg_tune_set(mptg_ctx* ctx, const mptg_tune_params* p);
    traversal, src/mpt/impl/prrt/prrt.hpp:406-409, which has nothing to tune).
    The split shapes the scans; a tree the uniform grid serves (knn_grid on)
    sends every candidate through the grid, so switch knn_grid off first to
-   tune the scans themselves. */
+   tune the scans themselves.  Searches that do not split the tree this way
+   (k = 1 by a block per query, wave lists, SE(3)) report the present setting
+   alone. */
 int mptg_autotune_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, mptg_tune_report* rep);
 /* Times link() of n device edges (reference order) for each candidate of the
-   scene's link launch shape -- for DMV scenes the lanes per edge and then
-   the grid of the persistent long-edge kernel, for meshes the grid and then the waves per edge, for the arm
-   arm_tail_waves (rep: the last knob swept) -- and keeps the fastest;
-   the per-edge bisection kernels have none (MPTG_E_STATE). */
+   scene's link launch shape -- for DMV scenes the lanes per edge and then the
+   grid of the persistent long-edge kernel (rep: the last knob swept), for
+   meshes the grid -- and keeps the fastest.  The arm's kernels choose their
+   shape: the report holds the present setting's time alone.  The per-edge
+   bisection kernels have none (MPTG_E_STATE). */
 int mptg_autotune_link(mptg_ctx* ctx, const double* d_from, const double* d_to, int64_t n,
                        mptg_tune_report* rep);
 /* Grows the tree (these iterations count, as in mptg_prrt_run) with each
    candidate of the planner's launch knob and keeps the fastest per
    iteration; stops early at target_size.  Plain PRRT: iterations per graph
-   launch (0 = step by step).  PRRT*: waves per mesh edge, or per continued
-   arm edge (other scenes: MPTG_E_STATE). */
+   launch (0 = step by step).  PRRT*: the grid of the mesh kernels; on arm
+   scenes nothing is left to choose (an empty report, no iterations); other
+   scenes MPTG_E_STATE. */
 int mptg_autotune_prrt(mptg_ctx* ctx, int64_t target_size, mptg_tune_report* rep);
 
 /* one arm-scene link() call (as mptg_link_dev) timed phase by phase with HIP

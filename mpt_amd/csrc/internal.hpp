@@ -233,6 +233,9 @@ double planner_coord_bound(const mptg_ctx* ctx);
 // n_dev, skip and nq_dev as for launch_knn.  Whether nq queries over n nodes take
 // it rather than the scan (q8: with its byte prefilter).
 bool knn_one_applies(const mptg_ctx* ctx, int64_t nq, int64_t n, bool q8);
+// Whether launch_knn of nq queries over n nodes splits the tree over blocks as
+// knn_blocks_per_cu says.
+bool knn_reads_splits(const mptg_ctx* ctx, int64_t nq, int k, int64_t n);
 int knn_one_path(mptg_ctx* ctx, const double* d_q, int64_t nq, double radius, int32_t* d_idx, double* d_dist,
                  int64_t n, const int64_t* n_dev, const int32_t* skip, const uint32_t* nq_dev);
 

@@ -695,7 +695,7 @@ __global__ __launch_bounds__(kBlock) void knn_collect(const float* __restrict__ 
 
 // k best (exact distance, index) of each query's candidates over the chunks,
 // among those within the radius; a query with an overflowed region goes to
-// `over` for the k-list scan instead.  Candidates beyond the bound cannot
+// `over` for the wave lists instead.  Candidates beyond the bound cannot
 // displace the k best: at least k tree nodes lie within it.
 template <int D, int METRIC, int K>
 __global__ __launch_bounds__(kBlock) void knn_select(const double* __restrict__ x64, const double* __restrict__ q,
@@ -1062,7 +1062,7 @@ void dispatch_collect(mptg_ctx* ctx, dim3 grid, int64_t n, int64_t chunk, const 
 
 // One refinement level over the tree prefix [0, n): collect within the
 // bounds tau, select the k best; queries whose candidates overflowed take
-// the k-list scan over the prefix (gathered, scanned, scattered back).
+// the wave lists over the prefix (gathered, searched, scattered back).
 static int knn_refine(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radius, const double* tau,
                       int64_t n, double* out_d, int32_t* out_i) {
     const int K = k <= 20 ? 20 : 32;
@@ -1117,12 +1117,12 @@ static int knn_refine(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, doubl
 }
 
 // k > 1 over a large tree, refined over growing tree prefixes: the exact k
-// best over the first 1/256 of the tree (k-list scan) bound every query;
+// best over the first 1/256 of the tree (wave lists) bound every query;
 // collect within the bound over the first 1/16 and select its exact k best,
 // which bound the whole tree's; collect and select over the whole tree.  A
 // prefix's k-th distance is no smaller than the whole tree's, the collect
 // keeps every node within the bound and the select orders candidates by
-// exact (distance, index), so the result equals the k-list scan's.
+// exact (distance, index), so the result equals the wave lists'.
 static int knn_select_path(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radius, int32_t* d_idx,
                            double* d_dist, int64_t n) {
     int rc;
@@ -1140,7 +1140,20 @@ static int knn_select_path(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, 
     return knn_refine(ctx, d_q, nq, k, radius, tau, n, d_dist, d_idx);
 }
 
-constexpr int64_t kSelectMinTree = 1 << 16;  // smaller trees: the k-list scan
+// Smaller trees, dimensions without a collect kernel and lists past 32 take
+// the wave lists.
+constexpr int64_t kSelectMinTree = 1 << 16;
+static bool select_applies(const mptg_ctx* ctx, int k, int64_t n) {
+    return k > 1 && k <= 32 && n >= kSelectMinTree && ctx->tune.knn_select && ctx->metric != MPTG_METRIC_SE3 &&
+           ctx->dim >= 2 && (ctx->dim <= 8 || ctx->dim == 10 || ctx->dim == 20);
+}
+
+bool knn_reads_splits(const mptg_ctx* ctx, int64_t nq, int k, int64_t n) {
+    if (ctx->metric == MPTG_METRIC_SE3) return false;
+    if (knn_grid_applies(ctx, n)) return true;  // (the queries that the grid leaves)
+    if (k > 1) return select_applies(ctx, k, n);
+    return !knn_one_applies(ctx, nq, n, true) || !knn_one_applies(ctx, nq, n, false);
+}
 
 int launch_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radius, int32_t* d_idx,
                double* d_dist, int64_t tree_n, const int64_t* n_dev, const int32_t* skip, const uint32_t* nq_dev) {
@@ -1153,11 +1166,8 @@ int launch_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radiu
         return knn_scan_path(ctx, d_q, nq, radius, d_idx, d_dist, tree_n, n_dev, skip, nq_dev);
     }
     if (ctx->metric == MPTG_METRIC_SE3) return knn_wave_se3_path(ctx, d_q, nq, k, radius, d_idx, d_dist, tree_n, n_dev, skip);
-    const bool sel_dim = ctx->dim <= 8 || ctx->dim == 10 || ctx->dim == 20;
     const bool eager = nq > 0 && !n_dev && !skip && !ctx->capturing;
-    // (the select path keeps lists of up to 32; larger k takes the k-list scan)
-    const bool select = eager && k > 1 && k <= 32 && tree_n >= kSelectMinTree && ctx->tune.knn_select &&
-                        ctx->metric != MPTG_METRIC_SE3 && ctx->dim >= 2 && sel_dim;
+    const bool select = eager && select_applies(ctx, k, tree_n);
     if (eager && knn_grid_applies(ctx, tree_n)) {
         // the grid answers most queries; the rest take the scans, gathered
         // into a compact batch and scattered back
@@ -1175,7 +1185,7 @@ int launch_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double radiu
         hipLaunchKernelGGL(knn_gather, dim3((unsigned)(((int64_t)m * D + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                            ctx->stream, d_q, D, (const int64_t*)over, (int64_t)m, gq);
         // the select path streams the tree three times whatever the batch:
-        // few queries take the k-list scan
+        // few queries take the wave lists
         rc = select && m >= 2048 ? knn_select_path(ctx, gq, m, k, radius, gi, gd, tree_n)
                                  : knn_brute(ctx, gq, m, k, radius, gi, gd, tree_n);
         if (rc) return rc;

@@ -114,8 +114,10 @@ int mptg_autotune_knn(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, mptg_
     if ((rc = ensure(ctx, out, (sizeof(double) + sizeof(int32_t)) * (size_t)k * nq))) return rc;
     double* dist = (double*)out.p;
     int32_t* idx = (int32_t*)(dist + (size_t)k * nq);
+    std::vector<int> cand{1, 2, 4, 8, 16, 32, 64};
+    if (!knn_reads_splits(ctx, nq, k, ctx->size)) cand = {ctx->tune.knn_blocks_per_cu};
     return sweep(
-        ctx, MPTG_TUNE_KNN, {1, 2, 4, 8, 16, 32, 64}, [&](int v) { ctx->tune.knn_blocks_per_cu = v; },
+        ctx, MPTG_TUNE_KNN, cand, [&](int v) { ctx->tune.knn_blocks_per_cu = v; },
         [&] { return launch_knn(ctx, d_q, nq, k, __builtin_inf(), idx, dist, ctx->size); }, rep);
 }
 
@@ -134,13 +136,9 @@ int mptg_autotune_link(mptg_ctx* ctx, const double* d_from, const double* d_to, 
     auto call = [&] {
         return launch_link_masked(ctx, d_from, d_to, n, MPTG_ORDER_REFERENCE, 0, nullptr, verdict, checks);
     };
-    if (arm_wave) {
-        return sweep(ctx, MPTG_TUNE_ARM_TAIL, {1, 2, 4, 8}, [&](int v) { ctx->tune.arm_tail_waves = v; }, call, rep);
-    }
+    if (arm_wave)  // the kernels choose their shape: one time, and nothing to choose
+        return sweep(ctx, MPTG_TUNE_ARM_TAIL, {ctx->tune.arm_tail_waves}, [](int) {}, call, rep);
     if (ctx->scene.kind == MPTG_SCENE_MESH) {
-        if ((rc = sweep(ctx, MPTG_TUNE_MESH_EDGE, {1, 2, 4, 8, 16, 32},
-                        [&](int v) { ctx->tune.mesh_edge_waves = v; }, call, nullptr)))
-            return rc;
         return sweep(ctx, MPTG_TUNE_MESH, {8, 16, 32, 64, 128}, [&](int v) { ctx->tune.mesh_waves_per_cu = v; },
                      call, rep);
     }
@@ -159,9 +157,9 @@ int mptg_autotune_prrt(mptg_ctx* ctx, int64_t target_size, mptg_tune_report* rep
     if (ctx->size == 0) return fail(ctx, MPTG_E_EMPTY, "there are no valid initial states");
     if (ctx->scene.kind == MPTG_SCENE_HOST)
         return fail(ctx, MPTG_E_STATE, "host scenes run step by step: no launch shape to tune");
-    // the knob: plain PRRT, iterations per graph launch; PRRT* (step by step),
-    // the scene's per-edge link split (waves per mesh edge or per continued
-    // arm edge), whose best value depends on the planner's own edge mix
+    // the knob: plain PRRT, iterations per graph launch; PRRT* (step by step)
+    // on meshes, the grid of the mesh kernels, whose best value depends on the
+    // planner's own batches; the arm's kernels choose their shape
     int knob;
     std::vector<int> cand;
     int32_t* field;
@@ -172,15 +170,16 @@ int mptg_autotune_prrt(mptg_ctx* ctx, int64_t target_size, mptg_tune_report* rep
         field = &s.graph_iters;
         timed = 16;
     } else if (ctx->scene.kind == MPTG_SCENE_MESH) {
-        knob = MPTG_TUNE_MESH_EDGE;
-        cand = {1, 2, 4, 8, 16};
-        field = &ctx->tune.mesh_edge_waves;
+        knob = MPTG_TUNE_MESH;
+        cand = {16, 32, 64, 128};
+        field = &ctx->tune.mesh_waves_per_cu;
         timed = 4;
     } else if (ctx->scene.kind == MPTG_SCENE_ARM && ctx->link_mode == MPTG_LINK_BISECT) {
-        knob = MPTG_TUNE_ARM_TAIL;
-        cand = {1, 2, 4, 8};
-        field = &ctx->tune.arm_tail_waves;
-        timed = 4;
+        mptg_tune_report r{};
+        r.knob = MPTG_TUNE_ARM_TAIL;
+        r.chosen = ctx->tune.arm_tail_waves;
+        if (rep) *rep = r;
+        return MPTG_OK;
     } else {
         return fail(ctx, MPTG_E_STATE, "this PRRT* scene has no launch shape to tune");
     }

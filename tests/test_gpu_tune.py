@@ -35,9 +35,10 @@ def test_knn_every_split_is_exact_and_tuner_picks_fastest(ctx_factory):
     _say("tune knn")
     ctx = ctx_factory()
     rng = np.random.default_rng(71)
-    n, dim, k = 60000, 7, 20
+    n, dim, k = 66000, 7, 20  # the select path, which splits the tree by the knob
     pts = rng.uniform(-math.pi, math.pi, (n, dim))
     q = rng.uniform(-math.pi, math.pi, (4096, dim))
+    ctx.tune_set(knn_grid=0)
     ctx.space(scenes.METRIC_L2, dim)
     ctx.tree_insert(pts)
     oi, od = oracle.Oracle(_plain(scenes.METRIC_L2, dim)).knn(pts, q[:600], k)
@@ -52,6 +53,9 @@ def test_knn_every_split_is_exact_and_tuner_picks_fastest(ctx_factory):
     assert ctx.tune_get()["knn_blocks_per_cu"] == rep["chosen"]
     gi, gd = ctx.knn(q[:600], k)
     assert np.array_equal(gi, oi) and np.array_equal(gd, od)
+    # a search that does not read the knob has one candidate, the present one
+    rep = ctx.autotune_knn(dq.ptr, q.shape[0], 40)
+    assert list(rep["candidates"]) == [rep["chosen"]] == [ctx.tune_get()["knn_blocks_per_cu"]]
 
 
 @pytest.mark.parametrize("metric,dim,k", [(scenes.METRIC_L2, 7, 20), (scenes.METRIC_L1, 20, 5),
@@ -209,60 +213,62 @@ def test_mesh_grid_every_shape_is_exact(ctx_factory):
     a = np.concatenate([qa, rng.uniform(0, 100, (800, 3))], axis=1)
     b = a.copy()
     b[:, 4:] += rng.normal(0, 3, (800, 3))
-    # the ring replay of edges beyond 255 waypoints (wave 0 only) is covered
-    # by test_gpu_mesh.py at the default waves per edge
+    # the ring replay of edges beyond 255 waypoints is covered by test_gpu_mesh.py
     o = oracle.Oracle(sc)
     want = {kv: o.link(a, b, known_valid=kv, threads=16) for kv in (False, True)}
     ok = o.valid(a)
     for w in (1, 7, 128):
-        for ew in (1, 3, 32):
-            ctx.tune_set(mesh_waves_per_cu=w, mesh_edge_waves=ew)
+        ctx.tune_set(mesh_waves_per_cu=w)
+        for n in (1, 3, 800):  # few edges: waves by the edges, not by the knob
             for kv in (False, True):
-                gv, gc = ctx.link(a, b, endpoints_known_valid=kv)
-                assert np.array_equal(gv, want[kv][0]) and np.array_equal(gc, want[kv][1]), (w, ew, kv)
+                gv, gc = ctx.link(a[:n], b[:n], endpoints_known_valid=kv)
+                assert np.array_equal(gv, want[kv][0][:n]) and np.array_equal(gc, want[kv][1][:n]), (w, n, kv)
         assert np.array_equal(ctx.valid(a), ok), w
     da, db = ctx.to_device(a), ctx.to_device(b)
     rep = ctx.autotune_link(da.ptr, db.ptr, a.shape[0])
     _say(" ", rep, ctx.tune_get())
-    _check_report(rep, [8, 16, 32, 64, 128])  # the grid, swept after the waves per edge
+    _check_report(rep, [8, 16, 32, 64, 128])
     assert ctx.tune_get()["mesh_waves_per_cu"] == rep["chosen"]
 
 
-def test_arm_continuation_every_wave_count_is_exact(ctx_factory):
-    """Waves per edge of the arm continuation (1 = one wave walks all the
-    edge's rounds): verdicts and first-failure check counts equal the
-    oracle's for every count, from endpoints checked or vouched for, and
-    the surrogate order's verdicts equal the reference order's."""
-    _say("tune arm tail")
+@pytest.mark.parametrize("links", [5, 10, 20])
+def test_arm_link_every_batch_shape_is_exact(ctx_factory, links):
+    """The arm link's launch shapes, chosen by the batch: a block of eight
+    waves per edge below 8 edges per CU, an edge per wave from there on, with
+    whole and short last blocks.  Verdicts and first-failure check counts
+    equal the oracle's, from endpoints checked or vouched for; the surrogate
+    order's verdicts equal the reference order's."""
+    _say("arm batch shapes", links)
     import mpt_amd
     ctx = ctx_factory()
-    sc = scenes.arm_scene()
+    sc = scenes.arm_scene(links=links, ndisks=30)
     ctx.scene(sc)
+    ctx.surrogate_init(5)
     rng = np.random.default_rng(74)
-    a = rng.uniform(-math.pi, math.pi, (3000, 20))
-    b = np.clip(a + rng.normal(0, 0.5, (3000, 20)), -math.pi, math.pi)
-    b[-800:] = rng.uniform(-math.pi, math.pi, (800, 20))  # long edges: 8 rounds past the packed one
+    a = rng.uniform(-math.pi, math.pi, (3000, links))
+    b = np.clip(a + rng.normal(0, 0.5, a.shape), -math.pi, math.pi)
+    b[1::4] = rng.uniform(-math.pi, math.pi, b[1::4].shape)  # long edges: many rounds
     o = oracle.Oracle(sc)
-    want = {kv: o.link(a, b, known_valid=kv, threads=16) for kv in (False, True)}
-    for cull in (0, 1):
-        for waves in (1, 2, 3, 5, 8):
-            ctx.tune_set(arm_tail_waves=waves, arm_cull=cull)
-            for kv in (False, True):
-                gv, gc = ctx.link(a, b, endpoints_known_valid=kv)
-                assert np.array_equal(gv, want[kv][0]) and np.array_equal(gc, want[kv][1]), (cull, waves, kv)
+    for kv in (False, True):
+        wv, wc = o.link(a, b, known_valid=kv, threads=16)
+        for n in (1, 7, 256, 2047, 2048, 2049, 2999, 3000):
+            gv, gc = ctx.link(a[:n], b[:n], endpoints_known_valid=kv)
+            assert np.array_equal(gv, wv[:n]) and np.array_equal(gc, wc[:n]), (n, kv)
+            sv, _ = ctx.link(a[:n], b[:n], mpt_amd.ORDER_SURROGATE, endpoints_known_valid=kv)
+            assert np.array_equal(sv, wv[:n]), (n, kv)
+    # nothing is left to tune: the report holds the present setting's time
     da, db = ctx.to_device(a), ctx.to_device(b)
+    before = ctx.tune_get()
     rep = ctx.autotune_link(da.ptr, db.ptr, a.shape[0])
-    _say(" ", rep, ctx.tune_get())
-    _check_report(rep, [1, 2, 4, 8])
-    assert ctx.tune_get()["arm_tail_waves"] == rep["chosen"]
-    assert ctx.tune_get()["arm_cull"] in (0, 1)
+    _check_report(rep, [before["arm_tail_waves"]])
+    assert ctx.tune_get() == before
 
 
 @pytest.mark.parametrize("ndisks", [0, 1, 7, 2000])
-def test_arm_disk_grid_every_size_and_culling_is_exact(ctx_factory, ndisks):
-    """The disk grid (1 x 1 up to 32 x 32 cells) and both link cullings
-    (wave box, per-lane cells) and the split-lane validity: verdicts and
-    check counts equal the oracle's brute force over every disk."""
+def test_arm_disk_lists_of_every_size_are_exact(ctx_factory, ndisks):
+    """Disks from none to thousands, in and out of reach, for valid() and for
+    link() of few edges and many: verdicts and check counts equal the oracle's
+    brute force over every disk."""
     _say("arm grid", ndisks)
     import dataclasses
     base = scenes.arm_scene(links=10, ndisks=3)
@@ -280,14 +286,13 @@ def test_arm_disk_grid_every_size_and_culling_is_exact(ctx_factory, ndisks):
     o = oracle.Oracle(sc)
     q = rng.uniform(-math.pi, math.pi, (3000, 10))
     ov = o.valid(q)
-    a = q[:1500]
+    a = q[:2500]
     b = np.clip(a + rng.normal(0, 0.7, a.shape), -math.pi, math.pi)
     lv, lc = o.link(a, b, known_valid=False, threads=16)
-    for cull in (0, 1):
-        ctx.tune_set(arm_cull=cull)
-        assert np.array_equal(ctx.valid(q), ov), cull
-        gv, gc = ctx.link(a, b, endpoints_known_valid=False)
-        assert np.array_equal(gv, lv) and np.array_equal(gc, lc), cull
+    assert np.array_equal(ctx.valid(q), ov)
+    for n in (100, 2500):
+        gv, gc = ctx.link(a[:n], b[:n], endpoints_known_valid=False)
+        assert np.array_equal(gv, lv[:n]) and np.array_equal(gc, lc[:n]), n
     if ndisks == 2000:
         assert 0.01 < ov.mean() < 0.99
 
@@ -314,9 +319,9 @@ def test_planner_tuned_while_growing_equals_oracle(ctx_factory):
 
 
 def test_prrt_star_tuned_while_growing_equals_oracle(ctx_factory):
-    """PRRT* on the mesh scene: the tuner times planner iterations for each
-    count of waves per mesh edge on the live tree; the tree it leaves, grown
-    on to the target, is the oracle's."""
+    """PRRT* on the mesh scene: the tuner times planner iterations for each grid
+    of the mesh kernels on the live tree; the tree it leaves, grown on to the
+    target, is the oracle's.  On the arm nothing is left to tune."""
     _say("tune prrt* mesh")
     sc = scenes.se3_scene()
     ctx = ctx_factory()
@@ -326,8 +331,8 @@ def test_prrt_star_tuned_while_growing_equals_oracle(ctx_factory):
     ctx.prrt_add_start(sc.start)
     rep = ctx.autotune_prrt(2500)
     _say(" ", rep)
-    assert rep["knob"] == 6 and sorted(rep["candidates"]) == [1, 2, 4, 8, 16]
-    assert ctx.tune_get()["mesh_edge_waves"] == rep["chosen"]
+    assert rep["knob"] == 2 and sorted(rep["candidates"]) == [16, 32, 64, 128]
+    assert ctx.tune_get()["mesh_waves_per_cu"] == rep["chosen"]
     st = ctx.prrt_run(2500, GPU_ITER_CAP)
     gn, gp = ctx.tree_read()
     gc = ctx.prrt_costs()
@@ -335,7 +340,16 @@ def test_prrt_star_tuned_while_growing_equals_oracle(ctx_factory):
     assert np.array_equal(gn, on) and np.array_equal(gp, op) and np.array_equal(gc, oc)
     for key in ("rewire_tests", "rewires", "parent_changes", "deferred"):
         assert st[key] == oss[key], key
-    # PRRT* on a scene with no per-edge split to tune is refused
+    arm = scenes.arm_scene(links=10, ndisks=20)
+    ctx.scene(arm)
+    ctx.tree_clear()
+    ctx.prrt_star_init(arm, 1, 64, k=20)
+    ctx.prrt_add_start(arm.start)
+    before = ctx.tune_get()
+    rep = ctx.autotune_prrt(1000)
+    assert rep["knob"] == 4 and rep["candidates"] == {} and rep["chosen"] == before["arm_tail_waves"]
+    assert ctx.tune_get() == before and ctx.tree_size() == 1
+    # PRRT* on a scene whose kernels have no such knob is refused
     boxes = scenes.boxes_scene()
     ctx.scene(boxes)
     ctx.tree_clear()
@@ -385,7 +399,7 @@ def test_knn_byte_prefilter_equals_fp32_scan_and_oracle(ctx_factory, dim):
     q[0] = pts[3]
     q[1] = pts[5]
     q[2, :] = math.pi
-    q[3, :] = 5.0 * math.pi                           # beyond the bound: every node exact
+    q[3, :] = 5.0 * math.pi                           # beyond the bound: clamped to it
     q[4] = (pts[100] + pts[101]) / 2
     ctx.space(scenes.METRIC_L1, dim)
     ctx.tree_insert(pts)
