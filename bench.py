@@ -148,7 +148,8 @@ def bench_arm(ctx, args, timer):
     tree = grow_tree(ctx, sc, args.seed, B, args.tree_size)
     nodes_p = tree[0]
     log("  link autotune ...")
-    # on planner edges from the timed steps' tree
+    # on planner edges from the timed steps' tree (the arm's kernels choose
+    # their shape: the report is the time at it)
     ta, tb = surrogate.planner_edges(ctx, sc, nodes_p, 8192, seed=98)
     dta, dtb = ctx.to_device(ta), ctx.to_device(tb)
     tune_link = ctx.autotune_link(dta.ptr, dtb.ptr, ta.shape[0])
@@ -178,7 +179,7 @@ def bench_arm(ctx, args, timer):
         t = timer.time(run, 5)
         out[name] = {"ms": t * 1e3, "edge_checks_per_s": ne / t, "verdicts": v.numpy().copy(),
                      "checks": c.numpy().astype(np.int64)}
-    # per-phase HIP-event times of the link call (score, rank, head, tail, list)
+    # per-phase HIP-event times of the link call (head: the link kernel, tail: the checks it leaves)
     phases = {}
     for name, order in (("plain", mpt_amd.ORDER_REFERENCE), ("surrogate", mpt_amd.ORDER_SURROGATE)):
         runs = [ctx.link_phases(da.ptr, db.ptr, ne, order, True, v.ptr, c.ptr) for _ in range(5)]
@@ -261,7 +262,7 @@ def bench_arm(ctx, args, timer):
             "executed_tflops": flops_p / t_kernel_p / 1e12, "executed_frac": flops_p / t_kernel_p / FP32_PEAK,
             "executed_unit": "the kernels' own FP32 bounds (angles in FP64) on the FP32 peak",
             "work": wk_p}
-    res = {"plain": plain, "surrogate": sur, "tail_autotune": tune_link,
+    res = {"plain": plain, "surrogate": sur, "link_autotune": tune_link,
            "launch_shapes": ctx.tune_get(),
            "trees_identical": same_tree, "training": train,
            "edge_batch": edge_batch,
@@ -385,7 +386,7 @@ def bench_se3(ctx, args):
     sc = scenes.se3_scene()
     ctx.scene(sc)
     ctx.tree_clear()
-    # waves per mesh edge, tuned by the autotuner on a PRRT* tree of its own
+    # the mesh kernels' grid, tuned by the autotuner on a PRRT* tree of its own
     # (the planner's own mix of extend, choose-parent and rewire links)
     ctx.prrt_star_init(sc, seed=args.seed + 1000, batch=4096, k=20)
     ctx.prrt_add_start(sc.start)
@@ -411,7 +412,7 @@ def bench_se3(ctx, args):
             "edge_checks_per_s": links / dt, "extend_links": d["link_calls"], "choose_parent_links": d["cp_links"],
             "rewire_links": d["rw_links"], "rewires": d["rewires"], "deferred": d["deferred"],
             "tree_size_start": s0["size"], "tree_size": s1["size"], "goals": s1["goals"],
-            "autotune_mesh_edge_waves": tune,
+            "autotune_mesh_waves": tune,
             "launch_shapes": ctx.tune_get()}
 
 
@@ -485,13 +486,13 @@ def kernels_only(ctx, args):
     src.zero()
     timer = Timer(ctx)
     reps = max(1, args.steps)
-    tune = ctx.autotune_link(da.ptr, db.ptr, ne)  # the continuation's waves per edge, as the headline run
+    tune = ctx.autotune_link(da.ptr, db.ptr, ne)
     res = {"copy_bytes": nbytes,
            "copy_ms": timer.time(lambda: ctx.diag_copy(dst.ptr, src.ptr, nbytes), reps) * 1e3}
     for name, order in (("plain", mpt_amd.ORDER_REFERENCE), ("surrogate", mpt_amd.ORDER_SURROGATE)):
         res[f"link_{name}_ms"] = timer.time(
             lambda order=order: ctx.link_dev(da.ptr, db.ptr, ne, order, True, v.ptr, c.ptr), reps) * 1e3
-    print(json.dumps({"mode": "kernels", "edges": ne, "reps": reps, "tail_autotune": tune,
+    print(json.dumps({"mode": "kernels", "edges": ne, "reps": reps, "link_autotune": tune,
                       "launch_shapes": ctx.tune_get(), **res}))
 
 

@@ -327,7 +327,9 @@ class Context:
                                              1 if known_valid else 0, C.c_void_p(v_ptr), C.c_void_p(c_ptr)))
 
     def link_phases(self, a: int, b: int, n: int, order: int, known_valid: bool, verdict: int, checks: int) -> dict:
-        """Per-phase milliseconds of one arm link() call on device buffers."""
+        """Per-phase milliseconds of one arm link() call on device buffers:
+        score (the surrogate's picks), head (the link kernel), gap, tail (the
+        checks and edges it leaves); list is no longer a phase (0)."""
         ms = (C.c_float * 5)()
         self._chk(_lib.mptg_link_phases(self._h, C.c_void_p(a), C.c_void_p(b), n, order, 1 if known_valid else 0,
                                         C.c_void_p(verdict), C.c_void_p(checks), ms))
@@ -346,8 +348,10 @@ class Context:
 
     def link_work(self, a_ptr: int, b_ptr: int, n: int, known_valid: bool = False,
                   order: int = ORDER_REFERENCE) -> dict:
-        """Executed work of the arm link kernel in the given order and the
-        reference algorithm's work on the same edges (device buffers)."""
+        """Executed work of the arm link kernels in the given order (calls:
+        waypoint checks, fk: links, group: cell lookups, far: FP32 link-disk
+        tests, exact: checks repeated exactly by edge walks) and the reference
+        algorithm's work on the same edges (device buffers)."""
         w = (C.c_uint64 * 9)()
         self._chk(_lib.mptg_link_work(self._h, C.c_void_p(a_ptr), C.c_void_p(b_ptr), n, order,
                                       1 if known_valid else 0, w))

@@ -78,8 +78,8 @@ __host__ __device__ __forceinline__ uint32_t skip_picks(uint32_t k, const uint32
 // One coordinate of the midpoint of the node at `path`: the reference's
 // recursion (a+b)/2 restricted to that coordinate.  (A form with one select
 // per level -- the child's interval is {m_k, the end the step keeps}, and
-// that end changes only when the path turns -- gives the same bits, but the
-// continuation kernel spilled with it at 5 waves per SIMD and ran 3% slower.)
+// that end changes only when the path turns -- gives the same bits and more
+// registers.)
 __host__ __device__ __forceinline__ double coord_mid(double lo, double hi, uint32_t path, int depth) {
     for (int k = 0; k < depth; ++k) {
         double m = (lo + hi) / 2;

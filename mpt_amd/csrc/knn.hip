@@ -6,16 +6,18 @@
 // computed with the same left-to-right FP64 expression as the CPU oracle, so
 // indices and distances are bit-exact.
 //
-// Kernel shape (gfx950, wave64):
+// k = 1 in up to 8 dimensions takes knn_one.hip by its rule, k > 1 the wave
+// lists (knn_wave.hip), the grid (knn_grid.hip) or, on large trees, bound /
+// collect / select below.  The scan here, for k = 1 (gfx950, wave64):
 //   * one lane owns one query; a 256-thread block holds 4 waves = 256 queries;
 //   * blockIdx.y splits the tree into chunks so that a launch has enough
 //     waves to fill 256 CUs even for a few thousand queries;
 //   * every lane of a wave visits the same tree node at the same time, so the
 //     node's FP32 row is a wave-uniform (scalar) load broadcast to all lanes;
-//   * FP32 prefilter: d32 is compared against the lane's current k-th FP64
-//     distance plus a proven rounding margin; only lanes that pass evaluate
-//     the FP64 distance and insert into a register-resident sorted list;
-//   * partial lists of the chunks are merged by a second kernel;
+//   * FP32 prefilter: d32 is compared against the lane's best FP64 distance
+//     plus a proven rounding margin; only lanes that pass evaluate the FP64
+//     distance; under L1 in 8 or more dimensions a byte prefilter instead;
+//   * the chunks' results are merged by a second kernel;
 //   * SE(3) queries reverse the roles: a query gets a workgroup, its lanes take
 //     consecutive nodes (knn_wave_se3).
 //

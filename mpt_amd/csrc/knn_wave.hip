@@ -12,7 +12,7 @@
 // the end, and a wave's expected inserts are k (1 + ln(n / (W k))).
 //
 // Reading the tree: the FP32 shadow rows (contiguous 16-byte loads of
-// consecutive lanes) with the proven FP32 bound of knn.hip in front of the
+// consecutive lanes) with the proven FP32 bound of knn_bound.hpp in front of the
 // exact distance; in up to 2 dimensions an FP64 row is one 16-byte load and
 // the distance cheaper than a bound, so the exact distance is taken at once.
 // The next rows are loaded before the present ones are used.  A row is
@@ -203,7 +203,10 @@ int knn_wave_path(mptg_ctx* ctx, const double* d_q, int64_t nq, int k, double ra
     // waves per query: about 8 waves per SIMD in all, and at least 4 rounds
     // of 64 nodes per wave (below that the merge of the lists costs more than
     // the split saves); queries per wave: 4 once the queries alone fill the
-    // chip four times over
+    // chip four times over.  Sixteen waves is the most: one query over 10^6
+    // nodes keeps one CU busy for 0.57 ms (R^12, k = 20) to 1.3 (R^20, L1, k =
+    // 48), where the k-list scan spread over the chip took 2.4 and 7.4 for its
+    // lists' merge; at 256 queries it is 0.58 against 6.4 and 1.4 against 40.
     const int64_t fill = (int64_t)ctx->cus * 32, rounds = (n + 63) / 64;
     const int Q = ctx->dim <= 8 && nq >= 4 * fill ? 4 : 1;
     int W = 1;

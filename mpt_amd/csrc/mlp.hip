@@ -84,11 +84,11 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Rows [0, M) of X; logits to z (if not null).  TRAIN: labels y; the mean
-// loss's gradients (scaled by inv_n) to out.
 // Round to nearest even in hardware (finite values as float_to_bf16).
 __device__ __forceinline__ uint16_t to_bf16(float v) { return __builtin_bit_cast(uint16_t, (__bf16)v); }
 
+// Rows [0, M) of X; logits to z (if not null).  TRAIN: labels y; the mean
+// loss's gradients (scaled by inv_n) to out.
 template <bool TRAIN>
 __global__ __launch_bounds__(64 * kPassWaves) void mlp_pass(const uint16_t* __restrict__ X,
                                                             const float* __restrict__ y, int64_t M, float inv_n,

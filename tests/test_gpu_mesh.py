@@ -106,10 +106,9 @@ def test_mesh_link_parity(ctx_factory, se3):
 @pytest.mark.parametrize("waves", [1, 128])
 def test_mesh_link_mixed_lengths_in_one_batch(ctx_factory, se3, n, waves):
     """Zero-length, short, table-long and ring-long edges side by side in the
-    64-position batches of the link waves, for grids of few and many waves;
-    the largest batch has more table-long waypoints (some 150 an edge) than
-    the link call stores poses for.  Verdicts and first-failure check counts
-    equal the oracle's."""
+    64-position batches of the link waves; at one wave per CU a wave takes
+    many batches, and in the largest the items are hundreds of thousands.
+    Verdicts and first-failure check counts equal the oracle's."""
     import dataclasses
     _say("mesh link mixed", n, waves)
     sparse = scenes.se3_scene(n_env_tris=1200, seed_env=7)

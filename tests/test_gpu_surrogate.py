@@ -222,7 +222,7 @@ def test_surrogate_order_parity_and_savings(trained):
     sc_np = scores.numpy()
     o = oracle.Oracle(sc)
     # the surrogate order: the 4 best-scored waypoints of the top 4
-    # bisection levels (the packed round), then every other waypoint in
+    # bisection levels (the picks), then every other waypoint in
     # reference order
     for e in range(0, m, 2):
         W = len(o.waypoints(a[e], b[e]))

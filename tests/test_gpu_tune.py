@@ -62,10 +62,10 @@ def test_knn_every_split_is_exact_and_tuner_picks_fastest(ctx_factory):
                                           (scenes.METRIC_L2, 3, 32)])
 def test_knn_select_path_equals_klist_scan_and_oracle(ctx_factory, metric, dim, k):
     """k > 1 on trees of 2^16 nodes or more: bound from the first 1/16 of the
-    tree, collect, select.  Equals the k-list scan on every query and the
+    tree, collect, select.  Equals the wave lists on every query and the
     oracle on a sample, with duplicates and ties, a finite radius, and a tree
     whose first 1/16 lies far from the queries (loose bounds: candidate lists
-    overflow and those queries take the k-list scan)."""
+    overflow and those queries take the wave lists)."""
     _say("knn select", metric, dim, k)
     ctx = ctx_factory()
     rng = np.random.default_rng(80 + dim)
