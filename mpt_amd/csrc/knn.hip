@@ -333,6 +333,7 @@ __device__ __forceinline__ bool q8_query(const double* __restrict__ q, double bo
                                          uint32_t* qw) {
     constexpr int NW = (D + 3) / 4;
     bool inside = true;
+    bound *= 0x1.0p20;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
         uint32_t v = 0;
@@ -341,7 +342,7 @@ __device__ __forceinline__ bool q8_query(const double* __restrict__ q, double bo
             const int i = 4 * w + b;
             if (i < D) {
                 const double x = q[i];
-                inside = inside && __builtin_fabs(x) <= bound * 0x1.0p20;
+                inside = inside && __builtin_fabs(x) <= bound;
                 v |= q8_byte((float)x, Bf, inv_sf) << (8 * b);
             }
         }
