@@ -373,7 +373,7 @@ enum {
 };
 
 /* What one tuning call tried and chose: the knob, each candidate value and
-   its median time (ms per call; per planner iteration for MPTG_TUNE_GRAPH). */
+   its time (median ms per call; mean ms per planner iteration in mptg_autotune_prrt). */
 typedef struct mptg_tune_report {
     int32_t knob;
     int32_t ncand;

@@ -184,11 +184,14 @@ int mptg_autotune_prrt(mptg_ctx* ctx, int64_t target_size, mptg_tune_report* rep
         return fail(ctx, MPTG_E_STATE, "this PRRT* scene has no launch shape to tune");
     }
     // each candidate per round: one untimed call (a graph capture, or the
-    // first launches of the new shape), then `timed` timed iterations;
-    // rounds alternate the candidate order so that tree growth favours none;
-    // median over rounds.  Every iteration counts, as in mptg_prrt_run.
-    constexpr int kRounds = 3;
-    std::vector<std::vector<double>> per(cand.size());
+    // first launches of the new shape), then `timed` timed iterations; an even
+    // number of rounds alternates the candidate order, so that over all of a
+    // candidate's iterations a steady growth of the tree favours none (the
+    // median of three rounds was the place of one: later candidates came
+    // earlier).  Every iteration counts, as in mptg_prrt_run.
+    constexpr int kRounds = 4;
+    std::vector<double> spent(cand.size(), 0.0);
+    std::vector<int64_t> iters(cand.size(), 0);
     const int32_t keep = *field;
     bool stop = false;
     for (int round = 0; round < kRounds && !stop; ++round) {
@@ -204,7 +207,8 @@ int mptg_autotune_prrt(mptg_ctx* ctx, int64_t target_size, mptg_tune_report* rep
             if ((rc = mptg_prrt_run(ctx, target_size, timed, nullptr))) break;
             const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
             const int64_t ran = s.iteration - it0;
-            if (ran > 0) per[i].push_back(sec * 1e3 / (double)ran);
+            spent[i] += sec * 1e3;
+            iters[i] += ran;
             stop = ctx->size >= target_size;
         }
         if (rc) break;
@@ -217,11 +221,7 @@ int mptg_autotune_prrt(mptg_ctx* ctx, int64_t target_size, mptg_tune_report* rep
     r.knob = knob;
     int pick = -1;
     for (size_t i = 0; i < cand.size(); ++i) {
-        double best = -1.0;
-        if (!per[i].empty()) {
-            std::sort(per[i].begin(), per[i].end());
-            best = per[i][per[i].size() / 2];
-        }
+        const double best = iters[i] > 0 ? spent[i] / (double)iters[i] : -1.0;
         r.value[r.ncand] = cand[i];
         r.ms[r.ncand] = (float)best;
         ++r.ncand;
