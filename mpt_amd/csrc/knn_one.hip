@@ -250,9 +250,10 @@ __global__ __launch_bounds__(kOneBlock) void knn_one(const double* __restrict__ 
                     for (int c = 0; c < Q; ++c) {
                         if (!((in[u] & open) >> c & 1u)) continue;
                         const double d = exact_dist<D, METRIC>(q + (q0 + c < live ? q0 + c : live - 1) * D, x[u]);
-                        if (d <= radius && d < bd[c]) {
+                        const int32_t j = (int32_t)(j0 + u * kOneBlock);
+                        if (d <= radius && one_better(d, j, bd[c], bi[c])) {  // (a distance may be infinite)
                             bd[c] = d;
-                            bi[c] = (int32_t)(j0 + u * kOneBlock);
+                            bi[c] = j;
                             open &= ~((d == 0.0 ? 1u : 0u) << c);
                         }
                     }

@@ -243,7 +243,7 @@ def test_knn_nearest_routes_agree(ctx_factory, metric, dim, n, nq, spread):
 def test_knn_nearest_of_many_at_one_place(ctx_factory, metric, dim, nq, places):
     """Thousands of nodes at a few points, more pairs under the threshold than
     a block lists: the lowest id of the nearest point, the oracle's, for
-    queries at the points, beside them and out of the radius."""
+    queries at the points, beside them, out of the radius and at infinity."""
     _say("knn crowded", metric, dim, nq, places)
     ctx = ctx_factory()
     rng = np.random.default_rng(dim + places)
@@ -251,6 +251,7 @@ def test_knn_nearest_of_many_at_one_place(ctx_factory, metric, dim, nq, places):
     pts = rng.uniform(-2, 2, (places, dim))[rng.integers(0, places, n)]
     q = rng.uniform(-2.5, 2.5, (nq, dim))
     q[::5] = pts[rng.integers(0, n, len(q[::5]))]
+    q[2, 0] = math.inf  # every node at the one distance
     ctx.space(metric, dim)
     ctx.tree_insert(pts)
     o = oracle.Oracle(_plain(metric, dim))
