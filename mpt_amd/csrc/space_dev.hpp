@@ -59,11 +59,11 @@ struct SceneArgs {
 constexpr int kArmGridMax = 32;  // cells per axis at most
 constexpr int kDiskBatch = 4;    // disks loaded together in the culled loop
 
-// Cell of a coordinate along one axis; the host build and the device query
-// use this same expression, so it is monotone in v on both.
+// Cell of a coordinate along one axis (0 for no number); the host build and the
+// device query use this same expression, so it is monotone in v on both.
 MPTG_HD int arm_cell(double v, double v0, double inv, int n) {
     const double t = (v - v0) * inv;
-    return t < 0.0 ? 0 : (t >= (double)n ? n - 1 : (int)t);
+    return !(t >= 0.0) ? 0 : (t >= (double)n ? n - 1 : (int)t);
 }
 
 // FP32 clearance bounds of the arm (arm_near.hpp): cells per axis at most,
@@ -339,6 +339,7 @@ constexpr int kArmGroup = 5;
 
 // A joint past an angle that sincos does not take (from 2^20 pi/2 on) is no
 // number: no distance to it exceeds any radius, so the state hits every disk.
+// Every later joint is lost too, so the last one tells.
 __device__ __forceinline__ bool joint_lost(double x, double y) { return x != x || y != y; }
 
 template <int D, typename Coord>
@@ -373,7 +374,6 @@ __device__ __forceinline__ bool arm_ok_lane(const SceneArgs& sc, Coord&& coord) 
                 last_y = jy[k];
             }
         const double mx = (jx[0] + last_x) / 2, my = (jy[0] + last_y) / 2;
-        if (joint_lost(mx, my)) return sc.ndisks == 0;
         const double rho = sc.arm_lim[D + g];
         const double Rmax = (rho + ag.rtmax) * (1.0 + 0x1.0p-40) + 1e-12;
         const int gx0 = arm_cell(mx - Rmax, ag.x0, ag.ix, ag.nx), gx1 = arm_cell(mx + Rmax, ag.x0, ag.ix, ag.nx);
@@ -398,7 +398,7 @@ __device__ __forceinline__ bool arm_ok_lane(const SceneArgs& sc, Coord&& coord) 
         px = last_x;
         py = last_y;
     }
-    return true;
+    return !joint_lost(px, py) || sc.ndisks == 0;
 }
 
 // arm_ok_lane with L lanes per state: the L lanes of an aligned group of the
@@ -445,15 +445,13 @@ __device__ __forceinline__ bool arm_ok_split(const SceneArgs& sc, Coord&& coord,
         const double rho = sc.arm_lim[D + g];
         const double Rmax = (rho + ag.rtmax) * (1.0 + 0x1.0p-40) + 1e-12;
         int gx0 = 0, gx1 = -1, gy0 = 0, gy1 = -1;
-        bool hit = false;
-        if (active && ok && joint_lost(mx, my)) {
-            hit = sc.ndisks > 0;
-        } else if (active && ok) {
+        if (active && ok) {
             gx0 = arm_cell(mx - Rmax, ag.x0, ag.ix, ag.nx);
             gx1 = arm_cell(mx + Rmax, ag.x0, ag.ix, ag.nx);
             gy0 = arm_cell(my - Rmax, ag.y0, ag.iy, ag.ny);
             gy1 = arm_cell(my + Rmax, ag.y0, ag.iy, ag.ny);
         }
+        bool hit = false;
         // the group's disk runs, row after row, dealt to its L lanes in turn
         for (int gy = gy0; gy <= gy1 && !hit; ++gy) {
         const int j0 = ag.starts[gy * ag.nx + gx0], j1 = ag.starts[gy * ag.nx + gx1 + 1];
@@ -477,7 +475,7 @@ __device__ __forceinline__ bool arm_ok_split(const SceneArgs& sc, Coord&& coord,
         px = last_x;
         py = last_y;
     }
-    return ok;
+    return ok && (!active || !joint_lost(px, py) || sc.ndisks == 0);
 }
 
 template <int D>
