@@ -329,11 +329,10 @@ __device__ __forceinline__ uint32_t q8_byte(float x, float B, float inv_s) {
 
 // The query's byte row (NW words); false when a coordinate lies too far beyond B.
 template <int D>
-__device__ __forceinline__ bool q8_query(const double* __restrict__ q, double bound, float Bf, float inv_sf,
-                                         uint32_t* qw) {
+__device__ __forceinline__ bool q8_query(const double* __restrict__ q, float Bf, float inv_sf, uint32_t* qw) {
     constexpr int NW = (D + 3) / 4;
     bool inside = true;
-    bound *= 0x1.0p20;
+    const float far = Bf * 0x1.0p20f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
         uint32_t v = 0;
@@ -342,7 +341,7 @@ __device__ __forceinline__ bool q8_query(const double* __restrict__ q, double bo
             const int i = 4 * w + b;
             if (i < D) {
                 const double x = q[i];
-                inside = inside && __builtin_fabs(x) <= bound;
+                inside = inside && __builtin_fabsf((float)x) <= far;
                 v |= q8_byte((float)x, Bf, inv_sf) << (8 * b);
             }
         }
@@ -474,7 +473,7 @@ __global__ __launch_bounds__(kBlock) void knn_scan_q8(const float* __restrict__ 
     const double inv_s = 255.0 / (2.0 * bound);
 
     uint32_t qw[NW];
-    const bool inside = q8_query<D>(q + qc * D, bound, Bf, inv_sf, qw);
+    const bool inside = q8_query<D>(q + qc * D, Bf, inv_sf, qw);
     constexpr uint32_t C2 = (uint32_t)(2.0 * kQ8Slack * D) + 2;
     // a lane whose query lies too far outside the grid checks every node exactly;
     // inactive lanes take no node
